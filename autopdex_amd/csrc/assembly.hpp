@@ -44,12 +44,31 @@ struct KState {
 void ensure_krylov_scratch(Plan& P, hipStream_t st);
 // reduction partials of the Krylov kernels: 4 rows of kMaxBlocks = 8192 doubles
 constexpr int64_t kKrylovPartials = 4 * 8192;
+// A resident run's slots and its ResidentOut lie behind the rows of partials that the kernels before
+// it use; the kernels that finish those partials clear them.
+constexpr int kResidentMaxGroups = 256;
+constexpr int64_t kResidentSlotsAt = 2 * 8192;
+constexpr int kResidentSlotWords = 6 * kResidentMaxGroups;
+struct ResidentOut {
+  KState state;      // the scalars at the end of the run
+  long long aborted;  // a workgroup gave up waiting for the others
+};
+constexpr int kResidentClearWords = kResidentSlotWords + (int)(sizeof(ResidentOut) / 8);
 void spmv(Plan& P, const void* vals, const void* x, void* y, int precision, hipStream_t st);
 void sell_to_csr(Plan& P, const void* sell, void* csr, int precision, hipStream_t st);
 void csr_to_sell(Plan& P, const void* csr, void* sell, int precision, hipStream_t st);
 void jacobi_inverse(Plan& P, const void* vals, void* inv_diag, int precision, hipStream_t st);
 // FP64 inverse diagonal of an FP32 SELL matrix
 void jacobi_inverse_f32_to_f64(Plan& P, const float* vals, double* inv_diag, hipStream_t st);
+
+// The iterations of a PCG run from x = 0, r, z = D^-1 r, p_old and the scalars S to a stop flag in one
+// launch, waited for (resident.hip).  x and p_new receive the solution and the last direction,
+// host_state (pinned, sizeof(ResidentOut)) the scalars; S follows when the run asks for a reliable
+// update.  zt: 2 n_free words of scratch of the vectors' type.  false: the system does not fit, or
+// the run was given up; x is 0, r, z, p_old and S are as they were.
+template <class M, class V>
+bool pcg_resident(Plan& P, const M* vals, const V* inv, V* x, const V* r, const V* z, const V* p_old, V* p_new,
+                  unsigned long long* zt, KState* S, double* part, KState* host_state, hipStream_t st);
 
 // One preconditioned-CG solve on the plan's SELL matrix with values of type M
 // and Krylov vectors and scalars of type T (M = float, T = double: an FP32
@@ -71,12 +90,14 @@ struct PcgRun {
   // creates no events, records no timing and polls the stop flag synchronously (allocates
   // nothing)
   bool external = false;
+  bool streaming = false;  // a resident run was given up: not tried again
+  int start_k = 0;         // iterations before the present resident run
   int maxiter = 0, iterations = 0;
   int64_t launched = 0;
   size_t counted = 0;
   int64_t spmv_bytes = 0, upd_bytes = 0;
   hipEvent_t evs[2] = {nullptr, nullptr};
-  std::vector<EventPair> ev_spmv, ev_upd;
+  std::vector<EventPair> ev_spmv, ev_upd, ev_res;
 
   PcgRun(Plan& P, const M* vals, const T* inv, hipStream_t st);
   // caller-provided workspace: work = 6 n_free vectors, partials = kKrylovPartials doubles,

@@ -262,6 +262,14 @@ int apx_newton(apx_plan* plan, double* u_dev, const double* dirichlet_values_dev
   });
 }
 
+int apx_plan_set_resident_wait(apx_plan* plan, double seconds) {
+  return guarded([&] {
+    APX_REQUIRE(plan, APX_ERR_ARG, "null plan");
+    APX_REQUIRE(seconds <= 60.0, APX_ERR_ARG, "resident wait must be at most 60 seconds");
+    plan->resident_wait = seconds;
+  });
+}
+
 int apx_set_timing(apx_plan* plan, int enabled) {
   return guarded([&] {
     APX_REQUIRE(plan, APX_ERR_ARG, "null plan");

@@ -266,10 +266,17 @@ __global__ __launch_bounds__(kBS) void k_pcg_init(int64_t n, const T* __restrict
   block_partials<kBS, 2>(v, partials);
 }
 
-__global__ __launch_bounds__(kFinBS) void k_pcg_init_fin(KState* S, const double* partials, int nb, double tol,
+// the slots of a resident run start at zero (its meetings count from 1)
+__device__ __forceinline__ void clear_resident_slots(double* partials) {
+  static_assert(kResidentSlotsAt == 2 * kMaxBlocks && kResidentClearWords <= 2 * kMaxBlocks, "slots behind two rows");
+  for (int i = threadIdx.x; i < kResidentClearWords; i += kFinBS) partials[kResidentSlotsAt + i] = 0.0;
+}
+
+__global__ __launch_bounds__(kFinBS) void k_pcg_init_fin(KState* S, double* partials, int nb, double tol,
                                                          double atol, int maxiter, double delta) {
   double s[2];
   finalize_sums<2>(partials, nb, s);
+  clear_resident_slots(partials);
   if (threadIdx.x == 0) {
     S->gamma = s[0];
     S->gamma_prev = s[0];
@@ -389,9 +396,10 @@ __global__ __launch_bounds__(kBS) void k_pcg_reanchor(int64_t n, const int32_t* 
   block_partials<kBS, 2>(v, partials);
 }
 
-__global__ __launch_bounds__(kFinBS) void k_pcg_reanchor_fin(KState* S, const double* partials, int nb) {
+__global__ __launch_bounds__(kFinBS) void k_pcg_reanchor_fin(KState* S, double* partials, int nb) {
   double s[2];
   finalize_sums<2>(partials, nb, s);
+  clear_resident_slots(partials);
   if (threadIdx.x == 0) {
     S->beta = s[0] / S->gamma_prev;
     S->gamma = s[0];
@@ -409,18 +417,17 @@ PcgRun<M, T>::PcgRun(Plan& P_, const M* vals_, const T* inv_, hipStream_t st_)
   n = P.n_free;
   T* w;
   if constexpr (sizeof(T) == 8) {
-    if (P.w64.n < (size_t)(6 * n)) P.w64.alloc(6 * n);
+    if (P.w64.n < (size_t)(7 * n)) P.w64.alloc(7 * n);
     w = (T*)P.w64.p;
   } else {
-    if (P.w32.n < (size_t)(6 * n)) P.w32.alloc(6 * n);
+    if (P.w32.n < (size_t)(7 * n)) P.w32.alloc(7 * n);
     w = (T*)P.w32.p;
   }
-  r = w; z = w + n; pa = w + 2 * n; pb = w + 3 * n; q = w + 4 * n; xw = w + 5 * n;
+  // (w + 4 n: q, or the resident run's 2 n words)
+  r = w; z = w + n; pa = w + 2 * n; pb = w + 3 * n; q = w + 4 * n; xw = w + 6 * n;
   ensure_krylov_scratch(P, st);
   S = (KState*)P.kstate.p;
   part = P.partials.p;
-  APX_HIP(hipEventCreateWithFlags(&evs[0], hipEventDisableTiming));
-  APX_HIP(hipEventCreateWithFlags(&evs[1], hipEventDisableTiming));
   // SELL values + columns (int16 offsets or int32), chunk offsets, z and p_old read, p_new and q written
   spmv_bytes = P.sell_total * (int64_t)(sizeof(M) + (P.sell_dcol.p ? 2 : 4)) + (P.n_chunks + 1) * 4 +
                n * 4 * (int64_t)sizeof(T);
@@ -431,7 +438,7 @@ template <class M, class T>
 PcgRun<M, T>::PcgRun(Plan& P_, const M* vals_, const T* inv_, hipStream_t st_, T* w, double* partials, KState* state)
     : P(P_), vals(vals_), inv(inv_), st(st_), S(state), part(partials), external(true) {
   n = P.n_free;
-  r = w; z = w + n; pa = w + 2 * n; pb = w + 3 * n; q = w + 4 * n; xw = w + 5 * n;
+  r = w; z = w + n; pa = w + 2 * n; pb = w + 3 * n; q = w + 4 * n;  // and a further n: the caller gives x
 }
 
 template <class M, class T>
@@ -443,6 +450,7 @@ PcgRun<M, T>::~PcgRun() {
 template <class M, class T>
 void PcgRun<M, T>::init(const T* b, T* x_, double tol, double atol, int maxiter_, double delta) {
   x = x_ ? x_ : xw;
+  start_k = 0;
   maxiter = maxiter_ <= 0 ? (int)std::min<int64_t>(10 * n, INT32_MAX / 2) : maxiter_;
   const int g = grid_for(n);
   hipLaunchKernelGGL(k_pcg_init<T>, dim3(g), dim3(kBS), 0, st, n, b, inv, x, r, z, pa, S, part, tol, atol,
@@ -483,6 +491,34 @@ void PcgRun<M, T>::launch_iteration() {
 
 template <class M, class T>
 KState PcgRun<M, T>::run() {
+  {
+    // in one launch where the system fits on the compute units (resident.hip)
+    static_assert(sizeof(ResidentOut) <= 256, "ResidentOut must fit its pinned slot");
+    KState* pinned_state = (KState*)((char*)P.pinned + 768);  // pinned bytes 768..1023
+    const bool odd = start_k & 1;
+    const bool timed = P.timing && !external;
+    const EventPair e = timed ? timing_pair(P) : EventPair{};
+    t_launch_events = timed ? &e : nullptr;
+    const bool ran = !streaming && pcg_resident<M, T>(P, vals, inv, x, r, z, odd ? pb : pa, odd ? pa : pb,
+                                                      (unsigned long long*)q, S, part, pinned_state, st);
+    if (timed && !t_launch_events)
+      ev_res.push_back(e);
+    else if (timed)
+      P.evpool.insert(P.evpool.end(), {e.a, e.b});
+    t_launch_events = nullptr;
+    if (ran) {
+      iterations = pinned_state->k;
+      // the last direction was written beside p_old; iteration k reads it from pb (k odd) or pa
+      if (((iterations ^ start_k) & 1) == 0) std::swap(pa, pb);
+      start_k = iterations;
+      return *pinned_state;
+    }
+    streaming = true;
+  }
+  if (!external && !evs[0]) {
+    APX_HIP(hipEventCreateWithFlags(&evs[0], hipEventDisableTiming));
+    APX_HIP(hipEventCreateWithFlags(&evs[1], hipEventDisableTiming));
+  }
   constexpr int kBatch = 16;
   volatile int* flag = (volatile int*)P.pinned;  // [slot*4 + {k, maxiter, done, reliable}]
   auto enqueue_batch = [&](int slot) {
@@ -521,7 +557,6 @@ KState PcgRun<M, T>::run() {
   KState hs;
   if (external) {
     // through the plan's pinned block (bytes 768..1023), so no pageable staging is involved
-    static_assert(sizeof(KState) <= 256, "KState must fit the pinned slot");
     char* slot = (char*)P.pinned + 768;
     APX_HIP(hipMemcpyAsync(slot, S, sizeof(KState), hipMemcpyDeviceToHost, st));
     APX_HIP(hipStreamSynchronize(st));
@@ -551,6 +586,7 @@ void PcgRun<M, T>::collect_timing() {
   timing_collect(P, sizeof(M) == sizeof(T) ? (f64 ? "pcg_spmv_f64" : "pcg_spmv_f32") : "pcg_spmv_f32m_f64v", ev_spmv,
                  spmv_bytes, k);
   timing_collect(P, f64 ? "pcg_update_f64" : "pcg_update_f32", ev_upd, upd_bytes, k);
+  timing_collect(P, f64 ? "pcg_resident_f64" : "pcg_resident_f32", ev_res, 0, ev_res.size());
   counted = iterations;
 }
 

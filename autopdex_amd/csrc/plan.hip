@@ -157,10 +157,16 @@ void plan_build_host(Plan& P, std::vector<std::vector<int32_t>>& conn_perm,
   // 4. SELL-64 layout of the reduced matrix
   P.n_chunks = (P.n_free + kSellC - 1) / kSellC;
   P.sell_ptr_h.assign(P.n_chunks + 1, 0);
+  P.bandwidth = 0;
+  P.max_row = 0;
   for (int64_t c = 0; c < P.n_chunks; ++c) {
     int32_t w = 0;
-    for (int64_t r = c * kSellC; r < std::min<int64_t>(P.n_free, (c + 1) * kSellC); ++r)
+    for (int64_t r = c * kSellC; r < std::min<int64_t>(P.n_free, (c + 1) * kSellC); ++r) {
       w = std::max(w, P.indptr_h[r + 1] - P.indptr_h[r]);
+      if (P.indptr_h[r + 1] > P.indptr_h[r])  // columns are sorted
+        P.bandwidth = std::max<int64_t>({P.bandwidth, r - P.indices_h[P.indptr_h[r]], P.indices_h[P.indptr_h[r + 1] - 1] - r});
+    }
+    P.max_row = std::max(P.max_row, (int)w);
     APX_REQUIRE((int64_t)P.sell_ptr_h[c] + (int64_t)w * kSellC < (int64_t)INT32_MAX, APX_ERR_UNSUPPORTED,
                 "SELL layout exceeds int32 indexing");
     P.sell_ptr_h[c + 1] = P.sell_ptr_h[c] + w * kSellC;

@@ -80,6 +80,8 @@ struct Plan {
   // instead of 4 in the SpMV's stream.  Matrices of bandwidth under 2^15 (every structured grid
   // here, 3-DOF grids up to about 100^3 nodes) qualify.
   DevBuf<int16_t> sell_dcol;
+  int64_t bandwidth = 0;  // largest |column - row|
+  int max_row = 0;        // most entries in a row
   DevBuf<int32_t> csr2sell;    // nnz
   DevBuf<int32_t> diag_slot;   // n_free, position of the diagonal in SELL
 
@@ -91,6 +93,11 @@ struct Plan {
   DevBuf<double> tw, tpart;    // network training workspace (4 n_free) and its reduction partials
   DevBuf<double> kstate;       // device Krylov scalars
   double* pinned = nullptr;    // host pinned scalars
+  // Resident Krylov runs (resident.hip): the device's compute units and wall clock (read on first
+  // use), and the seconds a workgroup waits for the others before the run is given up (negative:
+  // no resident runs).
+  int cus = 0, clock_khz = 0;
+  double resident_wait = 2.0;
   struct UNet* net = nullptr;  // attached learned preconditioner (not owned)
   const double* net_g = nullptr;  // nodal coefficient channel of the network input (device, optional)
   // Jacobi scaling of the network (1 / sqrt|A_ii| per free DOF): the network maps

@@ -156,6 +156,12 @@ typedef struct apx_krylov_stats {
 int apx_pcg(apx_plan* plan, const void* vals_dev, const void* b_dev, void* x_dev, int precision,
             int precond, double tol, double atol, int maxiter, apx_krylov_stats* stats, void* stream);
 
+/* A Jacobi-PCG solve whose vectors fit on the compute units runs all its iterations in one launch,
+ * in which workgroups wait for each other.  A wait longer than `seconds` (default 2; at most 60)
+ * gives that launch up, and the solve goes on with one launch per kernel, as larger systems do;
+ * negative: always one launch per kernel.  The two agree to rounding.       */
+int apx_plan_set_resident_wait(apx_plan* plan, double seconds);
+
 /* Allocation-free apx_pcg.  No counterpart in the reference: it is for callers that
  * cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  Same arguments, kernels, iterates and
