@@ -1,5 +1,5 @@
-// Element-loop assembly kernels: residual, reduced-CSR tangent values and
-// tangent diagonal for the 'user potential' mode.
+// Element-loop assembly kernels: residual and tangent diagonal by colours, the tangent's element
+// matrices, and the dispatch between these, the owner tiles and the row-owner kernels.
 //
 // Replaces jacrev / jacfwd(jacrev) of the element potential under lax.map and
 // the .at[].add scatter (assembler.py:1064-1149, :219-436).
@@ -13,7 +13,7 @@
 
 namespace apx {
 
-enum { MODE_RES = 0, MODE_TAN = 1, MODE_DIAG = 2, MODE_COO = 3 };
+enum { MODE_RES = 0, MODE_DIAG = 2, MODE_COO = 3 };
 
 struct AsmArgs {
   const double* coords;  // SoA, dim x n_nodes
@@ -22,9 +22,8 @@ struct AsmArgs {
   int64_t e0, e1;        // element range of one colour
   const double* u;       // n_dofs
   ModelParams mp;
-  const int32_t* slots;  // colour-major, n_elems x (npe d)^2
   double* r;             // residual or diagonal output (n_dofs)
-  void* vals;            // reduced CSR values
+  void* vals;            // element matrices (BCOO)
 };
 
 template <class M, class T, int MODE, int BS>
@@ -75,16 +74,6 @@ __global__ __launch_bounds__(BS) void k_team(AsmArgs A) {
       for (int i = 0; i < D; ++i)
 #pragma unroll
         for (int B = 0; B < ND; ++B) data[i * ND + B] = out[i][B];
-    } else {
-      T* vals = (T*)A.vals;
-      const int32_t* sl = A.slots + (e * ND + (int64_t)t * D) * ND;
-#pragma unroll
-      for (int i = 0; i < D; ++i)
-#pragma unroll
-        for (int B = 0; B < ND; ++B) {
-          const int32_t s = sl[i * ND + B];
-          if (s >= 0) vals[s] += out[i][B];
-        }
     }
   }
 }
@@ -129,7 +118,6 @@ static void run_set(Plan& P, ElemSet& S, const double* u, double* r, void* vals,
   A.conn = S.conn.p;
   A.u = u;
   A.mp = S.params;
-  A.slots = S.slots.p;
   A.r = r;
   A.vals = vals;
   if constexpr (M::NODAL) {
@@ -137,7 +125,7 @@ static void run_set(Plan& P, ElemSet& S, const double* u, double* r, void* vals,
                 "variable-coefficient Poisson set needs nodal fields g and f bound");
   }
   if constexpr (MODE == MODE_COO) {
-    // element blocks go to disjoint slots: one launch over the original element order
+    // element blocks go to disjoint places: one launch over the original element order
     if (S.conn_orig.n < (size_t)(S.n_elems * S.npe)) {
       std::vector<int32_t> c32(S.conn_host.begin(), S.conn_host.end());
       S.conn_orig.upload(c32.data(), c32.size());
@@ -251,7 +239,7 @@ void assemble_residual(Plan& P, const double* u, double* r, hipStream_t st) {
   for (auto& S : P.sets) {
     if (tile_supported(P, S, 0)) {
       tile_residual(P, S, u, r, !have, st);
-    } else {
+    } else if (!gather_residual(P, S, u, r, !have, st)) {
       if (!have) fill<double>(r, P.n_dofs, 0.0, st);
       dispatch<double, MODE_RES>(P, S, u, r, nullptr, st);
     }
@@ -267,15 +255,7 @@ void assemble_tangent(Plan& P, const double* u, void* vals, int precision, hipSt
       if (S.model != APX_MODEL_LINE_TRACTION) tile_tangent(P, S, u, vals, precision, st);
     return;
   }
-  if (precision == APX_FP64) {
-    fill<double>((double*)vals, P.sell_total, 0.0, st);
-    for (auto& S : P.sets)
-      if (S.model != APX_MODEL_LINE_TRACTION) dispatch<double, MODE_TAN>(P, S, u, nullptr, vals, st);
-  } else {
-    fill<float>((float*)vals, P.sell_total, 0.0f, st);
-    for (auto& S : P.sets)
-      if (S.model != APX_MODEL_LINE_TRACTION) dispatch<float, MODE_TAN>(P, S, u, nullptr, vals, st);
-  }
+  rows_tangent(P, u, vals, precision, false, st);
 }
 
 void assemble_tangent_rounded(Plan& P, const double* u, float* vals, hipStream_t st) {
@@ -284,9 +264,7 @@ void assemble_tangent_rounded(Plan& P, const double* u, float* vals, hipStream_t
       if (S.model != APX_MODEL_LINE_TRACTION) tile_tangent(P, S, u, vals, kFP64RoundedToFP32, st);
     return;
   }
-  if (P.vals64.n < (size_t)P.sell_total) P.vals64.alloc(P.sell_total);
-  assemble_tangent(P, u, P.vals64.p, APX_FP64, st);
-  round_to_f32(P.vals64.p, vals, P.sell_total, st);
+  rows_tangent(P, u, vals, kFP64RoundedToFP32, false, st);
 }
 
 int64_t tangent_coo_entries(const Plan& P) {

@@ -33,6 +33,12 @@ void tile_residual(Plan& P, ElemSet& S, const double* u, double* r, bool overwri
 void tile_tangent(Plan& P, ElemSet& S, const double* u, void* vals, int precision, hipStream_t st);
 void tile_diagonal(Plan& P, ElemSet& S, const double* u, double* diag, bool overwrite, hipStream_t st);
 
+// rows.hip: row-owner kernels for all other meshes
+// the whole tangent, every stored entry written, in SELL or canonical CSR order
+void rows_tangent(Plan& P, const double* u, void* vals, int precision, bool csr, hipStream_t st);
+// r (+)= the set's residual; false: no kernel for this set (nothing done)
+bool gather_residual(Plan& P, ElemSet& S, const double* u, double* r, bool overwrite, hipStream_t st);
+
 // krylov.hip
 struct KState {
   double gamma, gamma_prev, pAp, alpha, beta, rr, atol2, bb, rr0, rmax2, delta2;

@@ -9,8 +9,7 @@ static thread_local std::string g_last_error;
 void set_last_error(const std::string& msg) { g_last_error = msg; }
 void newton(Plan& P, double* u, const double* dvals, const apx_newton_options& o, apx_newton_stats& s,
             hipStream_t st);
-void plan_build_host(Plan& P, std::vector<std::vector<int32_t>>& conn_perm,
-                     std::vector<std::vector<int32_t>>& slots_perm);
+void plan_build_host(Plan& P, std::vector<std::vector<int32_t>>& conn_perm);
 }  // namespace apx
 
 using namespace apx;
@@ -102,8 +101,8 @@ int apx_plan_bind_nodal_field(apx_plan* plan, int set, int which, const double* 
 int apx_plan_build_pattern(apx_plan* plan) {
   return guarded([&] {
     APX_REQUIRE(plan, APX_ERR_ARG, "null plan");
-    std::vector<std::vector<int32_t>> cp, sl;
-    plan_build_host(*plan, cp, sl);
+    std::vector<std::vector<int32_t>> cp;
+    plan_build_host(*plan, cp);
   });
 }
 
@@ -177,6 +176,7 @@ int apx_assemble_tangent(apx_plan* plan, const double* u_dev, void* vals_dev, in
     ScopedTimer t(P, precision == APX_FP64 ? "tangent_call_f64" : precision == APX_FP32 ? "tangent_call_f32"
                                                                                         : "tangent_call_f64_to_f32",
                   S(stream), tangent_bytes(P, out));
+    if (!tangent_by_tiles(P)) return rows_tangent(P, u_dev, vals_dev, precision, true, S(stream));
     void* sell = sell_buffer(P, out);
     if (precision == APX_FP64_ROUNDED)
       assemble_tangent_rounded(P, u_dev, (float*)sell, S(stream));

@@ -1,5 +1,5 @@
-// Host-side plan construction: reduced CSR pattern, element colouring and
-// element -> CSR slot maps.  Replaces, once per mesh and Dirichlet mask, the
+// Host-side plan construction: reduced CSR pattern, element colouring and the
+// lists of the row-owner kernels.  Replaces, once per mesh and Dirichlet mask, the
 // per-call index construction of _get_indices (assembler.py:47-141) and the
 // scipy COO -> CSR -> [:, free][free] reduction of scipy_assembling
 // (solver.py:1180-1222).  The reduced pattern equals scipy's canonical CSR:
@@ -9,7 +9,7 @@
 #include <chrono>
 #include <cstring>
 
-#include "plan.hpp"
+#include "assembly.hpp"
 
 namespace apx {
 
@@ -77,14 +77,71 @@ int64_t Plan::device_bytes() const {
   int64_t b = coords.bytes() + dmask.bytes() + full2red.bytes() + red2full.bytes() + indptr.bytes() +
               indices.bytes() + diag_slot.bytes() + sell_ptr.bytes() + sell_cols.bytes() + sell_dcol.bytes() +
               csr2sell.bytes() + vals64.bytes() + vals32.bytes() + w64.bytes() + w32.bytes() + r_full.bytes() +
-              diag_full.bytes() + partials.bytes();
-  for (auto& s : sets) b += s.conn.bytes() + s.slots.bytes();
+              diag_full.bytes() + partials.bytes() + element_vectors.bytes() + element_matrices.bytes();
+  for (auto& s : sets)
+    b += s.conn.bytes() + s.conn_orig.bytes() + s.inc_ptr.bytes() + s.inc.bytes() + s.touched.bytes() + s.rn_ptr.bytes() +
+         s.rn.bytes() + s.code.bytes();
   return b;
 }
 
-// Build the host-side reduced pattern and colour/slot data (no device calls).
-void plan_build_host(Plan& P, std::vector<std::vector<int32_t>>& conn_perm,
-                     std::vector<std::vector<int32_t>>& slots_perm) {
+// Node -> (element, local index) pairs of a set, in element order.
+static void build_incidence(const Plan& P, ElemSet& s) {
+  const int64_t m = s.n_elems * s.npe;
+  APX_REQUIRE(m < INT32_MAX, APX_ERR_UNSUPPORTED, "element set exceeds int32 indexing");
+  s.inc_ptr_h.assign(P.n_nodes + 1, 0);
+  for (int64_t k = 0; k < m; ++k) s.inc_ptr_h[s.conn_host[k] + 1]++;
+  for (int64_t n = 0; n < P.n_nodes; ++n) s.inc_ptr_h[n + 1] += s.inc_ptr_h[n];
+  std::vector<int32_t> at(s.inc_ptr_h.begin(), s.inc_ptr_h.end() - 1);
+  s.inc_h.resize(m);
+  for (int64_t k = 0; k < m; ++k) s.inc_h[at[s.conn_host[k]]++] = (int32_t)k;
+}
+
+// The lists of a set's row-owner tangent (ElemSet::rn, code).  adj: sorted neighbours of a node.
+static void build_rows(const Plan& P, ElemSet& s, const std::vector<int64_t>& adj_ptr, const std::vector<int32_t>& adj) {
+  const int d = P.d, npe = s.npe;
+  s.rn_ptr_h.assign(1, 0);
+  s.rn_h.clear();
+  s.rn_max = 0;
+  for (int64_t c = 0; c < P.n_chunks; ++c) {
+    const int64_t end = std::min<int64_t>(P.n_free, (c + 1) * kSellC);
+    for (int64_t row = c * kSellC, last = -1; row < end; ++row) {
+      const int32_t n = P.red2full_h[row] / d;
+      if (n == last) continue;
+      last = n;
+      if (s.inc_ptr_h[n + 1] > s.inc_ptr_h[n])
+        s.rn_h.insert(s.rn_h.end(), {s.inc_ptr_h[n], s.inc_ptr_h[n + 1], n * d});
+    }
+    s.rn_ptr_h.push_back((int32_t)(s.rn_h.size() / 3));
+    s.rn_max = std::max(s.rn_max, s.rn_ptr_h[c + 1] - s.rn_ptr_h[c]);
+  }
+  s.code_h.assign((size_t)s.n_elems * npe * npe, 0);
+  std::vector<uint16_t> place;
+  for (int64_t n = 0; n < P.n_nodes; ++n) {
+    if (s.inc_ptr_h[n + 1] == s.inc_ptr_h[n]) continue;
+    const int32_t *b = adj.data() + adj_ptr[n], *e = adj.data() + adj_ptr[n + 1];
+    place.clear();
+    int at = 0;
+    for (const int32_t* p = b; p != e; ++p) {
+      int free = 0, count = 0;
+      for (int k = 0; k < d; ++k)
+        if (!P.dmask_host[(int64_t)*p * d + k]) {
+          free |= 1 << k;
+          ++count;
+        }
+      APX_REQUIRE(at < 0x2000, APX_ERR_UNSUPPORTED, "a row of the reduced matrix has more than 8191 entries");
+      place.push_back((uint16_t)((count ? at : 0) | free << 13));
+      at += count;
+    }
+    for (int32_t k = s.inc_ptr_h[n]; k < s.inc_ptr_h[n + 1]; ++k) {
+      const int64_t* c = &s.conn_host[(int64_t)(s.inc_h[k] / npe) * npe];
+      for (int a = 0; a < npe; ++a)
+        s.code_h[(size_t)k * npe + a] = place[std::lower_bound(b, e, (int32_t)c[a]) - b];
+    }
+  }
+}
+
+// Build the host-side reduced pattern, colours and row-owner lists (no device calls).
+void plan_build_host(Plan& P, std::vector<std::vector<int32_t>>& conn_perm) {
   const int d = P.d;
   const int64_t N = P.n_nodes, ndof = P.n_dofs;
   APX_REQUIRE(!P.sets.empty(), APX_ERR_STATE, "plan has no element sets");
@@ -229,10 +286,17 @@ void plan_build_host(Plan& P, std::vector<std::vector<int32_t>>& conn_perm,
     break;
   }
 
-  // 5. greedy element colouring per set (node-disjoint colours) and slot maps
-  //    (slots index the SELL layout)
+  // 4d. lists of the row-owner kernels, for sets whose residual or tangent has no owner tiles
+  const bool tiles = tangent_by_tiles(P);
+  for (auto& s : P.sets) {
+    const bool rows = !tiles && s.model != APX_MODEL_LINE_TRACTION;
+    if (!rows && tile_supported(P, s, 0)) continue;
+    build_incidence(P, s);
+    if (rows) build_rows(P, s, adj_ptr, adj);
+  }
+
+  // 5. greedy element colouring per set (node-disjoint colours)
   conn_perm.assign(P.sets.size(), {});
-  slots_perm.assign(P.sets.size(), {});
   std::vector<uint64_t> used(N);
   for (int si = 0; si < (int)P.sets.size(); ++si) {
     auto& s = P.sets[si];
@@ -256,37 +320,43 @@ void plan_build_host(Plan& P, std::vector<std::vector<int32_t>>& conn_perm,
     std::vector<int64_t> perm(s.n_elems);
     for (int64_t e = 0; e < s.n_elems; ++e) perm[pos[colour[e]]++] = e;  // stable within a colour
 
-    const int nd = s.npe * d;
     auto& cp = conn_perm[si];
-    auto& sl = slots_perm[si];
     cp.resize(s.n_elems * s.npe);
-    sl.resize((size_t)s.n_elems * nd * nd);
     for (int64_t i = 0; i < s.n_elems; ++i) {
       const int64_t* c = &s.conn_host[perm[i] * s.npe];
       for (int a = 0; a < s.npe; ++a) cp[i * s.npe + a] = (int32_t)c[a];
-      for (int A = 0; A < nd; ++A) {
-        int32_t row = P.full2red_h[c[A / d] * d + A % d];
-        for (int B = 0; B < nd; ++B) {
-          int32_t col = P.full2red_h[c[B / d] * d + B % d];
-          int32_t slot = -1;
-          if (row >= 0 && col >= 0) {
-            const int32_t* b = P.indices_h.data() + P.indptr_h[row];
-            const int32_t* e = P.indices_h.data() + P.indptr_h[row + 1];
-            const int32_t* f = std::lower_bound(b, e, col);
-            APX_REQUIRE(f != e && *f == col, APX_ERR_INTERNAL, "slot lookup failed");
-            slot = P.csr2sell_h[f - P.indices_h.data()];
-          }
-          sl[((size_t)i * nd + A) * nd + B] = slot;
-        }
-      }
     }
   }
 }
 
+// The row-owner lists of a set (build_incidence, build_rows) to the device.
+static void upload_rows(Plan& P, ElemSet& S) {
+  if (S.inc_ptr_h.empty()) return;
+  std::vector<int32_t> c32(S.conn_host.begin(), S.conn_host.end()), nodes;
+  S.conn_orig.upload(c32.data(), c32.size());
+  for (int64_t n = 0; n < P.n_nodes; ++n)
+    if (S.inc_ptr_h[n + 1] > S.inc_ptr_h[n]) nodes.push_back((int32_t)n);
+  S.n_touched = (int64_t)nodes.size();
+  S.touched_all = S.n_touched == P.n_nodes;
+  if (!S.touched_all) S.touched.upload(nodes.data(), nodes.size());
+  S.inc_ptr.upload(S.inc_ptr_h.data(), S.inc_ptr_h.size());
+  S.inc.upload(S.inc_h.data(), S.inc_h.size());
+  if (!S.rn_ptr_h.empty()) {
+    S.rn_ptr.upload(S.rn_ptr_h.data(), S.rn_ptr_h.size());
+    S.rn.upload(S.rn_h.data(), S.rn_h.size());
+    S.code.upload(S.code_h.data(), S.code_h.size());
+  }
+  std::vector<int32_t>().swap(S.inc_ptr_h);
+  std::vector<int32_t>().swap(S.inc_h);
+  std::vector<int32_t>().swap(S.rn_ptr_h);
+  std::vector<int32_t>().swap(S.rn_h);
+  std::vector<uint16_t>().swap(S.code_h);
+}
+
 void plan_finalize(Plan& P) {
   auto t0 = std::chrono::steady_clock::now();
-  std::vector<std::vector<int32_t>> conn_perm, slots_perm;
-  plan_build_host(P, conn_perm, slots_perm);
+  std::vector<std::vector<int32_t>> conn_perm;
+  plan_build_host(P, conn_perm);
 
   // SoA coordinates
   std::vector<double> soa(P.n_nodes * P.dim);
@@ -336,8 +406,9 @@ void plan_finalize(Plan& P) {
   std::vector<int32_t>().swap(P.sell_cols_h);
   std::vector<int32_t>().swap(P.csr2sell_h);
   for (size_t si = 0; si < P.sets.size(); ++si) {
-    P.sets[si].conn.upload(conn_perm[si].data(), conn_perm[si].size());
-    P.sets[si].slots.upload(slots_perm[si].data(), slots_perm[si].size());
+    ElemSet& S = P.sets[si];
+    S.conn.upload(conn_perm[si].data(), conn_perm[si].size());
+    upload_rows(P, S);
   }
   // pinned host scalars: [0, 512) B PCG flags and norms, [512, 768) B FCG state copies,
   // [768, 1024) B the final Krylov state of an allocation-free PCG run

@@ -25,8 +25,20 @@ struct ElemSet {
   std::vector<int64_t> conn_host;  // original order, n_elems * npe
   // colour-permuted device data
   DevBuf<int32_t> conn;            // n_elems * npe, colour-major order
-  DevBuf<int32_t> slots;           // n_elems * (npe*d)^2 reduced CSR slots, -1 = Dirichlet
-  DevBuf<int32_t> conn_orig;       // original element order (made on first BCOO export)
+  DevBuf<int32_t> conn_orig;       // original element order
+  // Row-owner kernels (rows.hip; sets without owner tiles): node -> (element * npe + local index) in
+  // element order, and the nodes that have elements.
+  DevBuf<int32_t> inc_ptr, inc, touched;
+  int64_t n_touched = 0;
+  bool touched_all = false;        // every node, in order: no list
+  // Their tangent: per 64-row chunk of the reduced matrix the nodes of the set with rows in it (as
+  // begin and end in inc and first DOF), and per pair of inc and node of its element where that
+  // node's columns lie in the row: first position | free DOFs << 13.
+  DevBuf<int32_t> rn_ptr, rn;
+  int rn_max = 0;                  // most such nodes in a chunk
+  DevBuf<uint16_t> code;
+  std::vector<int32_t> inc_ptr_h, inc_h, rn_ptr_h, rn_h;  // until uploaded
+  std::vector<uint16_t> code_h;
   std::vector<int64_t> colour_offsets;  // n_colours + 1
   // Structured Q1 grid (the connectivity of mesher.structured_mesh): element
   // e = i * gny + j has nodes b, b + 1, b + gny + 2, b + gny + 1 with
@@ -50,6 +62,8 @@ struct Plan {
   int dim = 0, d = 0;
   int64_t n_nodes = 0, n_dofs = 0, n_free = 0, nnz = 0;
   bool finalized = false;
+  // scratch of the row-owner kernels
+  DevBuf<double> element_vectors, element_matrices;
   double build_seconds = 0.0;
 
   std::vector<double> coords_host;   // n_nodes * dim row-major
@@ -68,7 +82,7 @@ struct Plan {
   DevBuf<int32_t> indices;     // nnz
   // Internal matrix layout: SELL-64 (chunks of 64 rows = one wavefront; within
   // a chunk entries are stored column-major, lane = row, padded to the chunk's
-  // longest row).  Element slot maps point into this layout; the C ABI
+  // longest row).  The C ABI
   // exchanges values in canonical CSR order through csr2sell.
   int64_t sell_total = 0, n_chunks = 0;
   bool stencil_pattern = false;  // reduced rows = free nodes of the 3 x 3 stencil of a structured grid
@@ -155,7 +169,6 @@ constexpr int kSellC = 64;
 
 // plan.hip
 void plan_finalize(Plan& P);
-void plan_build_host(Plan& P, std::vector<std::vector<int32_t>>& conn_perm,
-                     std::vector<std::vector<int32_t>>& slots_perm);
+void plan_build_host(Plan& P, std::vector<std::vector<int32_t>>& conn_perm);
 
 }  // namespace apx

@@ -1,0 +1,202 @@
+"""Row-owner assembly (meshes without owner tiles) against the BCOO export (the element kernels,
+reduced on the host) and the oracle's residual: every element type, node numberings and element
+orders that no mesher makes, Dirichlet DOFs anywhere, sizes around one 64-row chunk, rows wider
+than the kernel forms at a time, several sets."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from tests import problems as P
+
+pytestmark = pytest.mark.gpu
+
+
+def _q2_grid(nx, ny):
+    from autopdex_amd import mesher
+    coords, _ = mesher.structured_mesh((2 * nx, 2 * ny), P.TAPERED, "quad")
+    m = 2 * ny + 1
+    i, j = (a.ravel() for a in np.meshgrid(np.arange(nx), np.arange(ny), indexing="ij"))
+    off = ((0, 0), (2, 0), (2, 2), (0, 2), (1, 0), (2, 1), (1, 2), (0, 1), (1, 1))
+    return coords, np.stack([(2 * i + a) * m + 2 * j + b for a, b in off], axis=1).astype(np.int64)
+
+
+def _fan(n):
+    """n quads around one node."""
+    t = np.linspace(0, 2 * np.pi, 2 * n, endpoint=False)
+    ring = np.stack([np.cos(t), np.sin(t)], axis=1) * np.where(np.arange(2 * n) % 2, 1.4, 1.0)[:, None]
+    k = np.arange(n)
+    quads = np.stack([np.zeros(n, int), 1 + 2 * k, 1 + 2 * k + 1, 1 + (2 * k + 2) % (2 * n)], axis=1)
+    return np.concatenate([[[0.0, 0.0]], ring]), quads.astype(np.int64)
+
+
+def _book(n, layers):
+    """n x layers bricks around an axis: rows of over 500 entries at its nodes for n = 30."""
+    flat, quads = _fan(n)
+    m = flat.shape[0]
+    coords = np.concatenate([np.column_stack([flat, np.full(m, 0.3 * z)]) for z in range(layers + 1)])
+    return coords, np.concatenate([np.concatenate([quads + z * m, quads + (z + 1) * m], axis=1) for z in range(layers)])
+
+
+def _problem(kind, size, shuffle, seed):
+    """(dofs, settings, static, oracle sets, d) with a random numbering and random Dirichlet DOFs."""
+    from autopdex_amd import mesher, models, seeder, spaces
+    from oracle import elements as OE
+    rng = np.random.default_rng(seed)
+    if kind == "q2":
+        coords, elems = _q2_grid(*size)
+    elif kind == "fan":
+        coords, elems = _fan(size[0])
+    elif kind == "book":
+        coords, elems = _book(*size)
+    elif kind in ("hex", "hexpoisson", "hexvark"):
+        coords, elems = mesher.structured_mesh(size, P.UNIT_CUBE, "brick")
+    else:
+        coords, elems = mesher.structured_mesh(size, P.TAPERED if kind == "panel" else P.UNIT_SQUARE, "quad")
+    n = coords.shape[0]
+    h = np.ptp(coords, axis=0).max() / max(size)
+    if kind == "book":  # displacements of the 0.1-wide wedges
+        h *= 0.2
+    if kind == "q2":  # nodes at half the element's edge, and a short right edge: no folded elements
+        h *= 0.2
+    coords = coords + 0.05 * h * rng.standard_normal(coords.shape) * (kind not in ("fan", "book"))
+    if shuffle:
+        perm = rng.permutation(n)
+        new = np.empty_like(coords)
+        new[perm] = coords
+        coords, elems = new, np.ascontiguousarray(perm[elems][rng.permutation(elems.shape[0])])
+    d = {"panel": 2, "q2": 2, "fan": 2, "hex": 3, "book": 3}.get(kind, 1)
+    shape = (n, d) if d > 1 else (n,)
+    mask = rng.random(shape) < 0.15
+    settings = {"connectivity": (elems,), "dirichlet dofs": mask, "node coordinates": coords,
+                "dirichlet conditions": np.zeros(shape)}
+    quad = seeder.gauss_legendre_nd(coords.shape[1], 2)
+    lam, mu = 1.7, 0.6
+    mode = "user potential"
+    if kind == "q2":
+        weak = models.hyperelastic_steady_state_weak(models.neo_hooke, lambda x, s: s["E"], lambda x, s: s["nu"],
+                                                     "plain strain")
+        pot = models.isoparametric_domain_element_galerkin(weak, spaces.fem_iso_line_quad_brick,
+                                                           *seeder.gauss_legendre_nd(dimension=2, order=4))
+        settings.update({"E": mu * (3 * lam + 2 * mu) / (lam + mu), "nu": lam / (2 * (lam + mu))})
+        mode, elem = "user element", OE.NeoHooke(lam, mu)
+    elif d > 1:
+        pot = models.mixed_reference_domain_potential(models.hyperelastic_integrand(models.neo_hooke, lam, mu),
+                                                      {"u": spaces.fem_iso_line_quad_brick}, *quad, "u")
+        elem = OE.NeoHooke(lam, mu)
+    elif kind == "hexvark" or kind == "vark":
+        g, f = 0.5 * rng.standard_normal(n), rng.standard_normal(n)
+        settings.update({"g": g, "f": f})
+        pot = models.mixed_reference_domain_potential(models.poisson_variable_coefficient_integrand("g", "f"),
+                                                      {"u": spaces.fem_iso_line_quad_brick}, *quad, "u")
+        elem = OE.PoissonVarK()
+    else:
+        pot = models.mixed_reference_domain_potential(models.poisson_source_integrand(),
+                                                      {"u": spaces.fem_iso_line_quad_brick}, *quad, "u")
+        elem = OE.PoissonSource()
+        if coords.shape[1] == 3:  # the kernels take the centre's second coordinate for the third too
+            elem.center = np.array([1.0, 0.5, 0.5])
+    static = P.static([pot])
+    static["assembling mode"] = (mode,)
+    u = 0.02 * h * rng.standard_normal(shape)
+    nodal = (settings["g"], settings["f"]) if "g" in settings else None
+    return u, settings, static, [(elem, elems, nodal)], d
+
+
+CASES = [("hex", (1, 1, 1), 0), ("hex", (3, 4, 5), 0), ("hex", (6, 5, 22), 0), ("hex", (4, 3, 5), 1),
+         ("hexpoisson", (4, 5, 70), 0), ("hexvark", (5, 4, 6), 1), ("panel", (1, 2), 0), ("panel", (7, 5), 1),
+         ("panel", (20, 33), 0), ("panel", (16, 31), 0), ("q2", (1, 1), 0), ("q2", (9, 17), 0), ("q2", (5, 4), 1),
+         ("poisson", (9, 11), 1), ("vark", (12, 30), 1), ("fan", (7,), 0),
+         ("book", (30, 2), 0), ("book", (5, 3), 1)]
+
+
+@pytest.mark.parametrize("kind,size,shuffle", CASES)
+def test_row_owner_assembly(torch_gpu, kind, size, shuffle):
+    torch = torch_gpu
+    from autopdex_amd import _native as N
+    from autopdex_amd import assembler, backend
+    from oracle import assembly as OA
+    u, settings, static, sets, d = _problem(kind, size, shuffle, seed=len(kind) + sum(size))
+    print(f"[case] rows {kind} {size} shuffle {shuffle}", flush=True)
+    prob = backend.get_problem(u, settings, static)
+    coo = assembler.assemble_tangent(u, settings, static, form="bcoo")
+    free = ~settings["dirichlet dofs"].ravel()
+    want = coo.tocsr()[:, free][free]
+    want.sort_indices()
+    got = assembler.assemble_tangent(u, settings, static)
+    assert np.array_equal(got.indptr, want.indptr) and np.array_equal(got.indices, want.indices)
+    scale = np.abs(want.data).max()
+    assert np.abs(got.data - want.data).max() <= 1e-13 * scale  # a few hundred FP64 roundings
+    f32 = assembler.assemble_tangent(u, settings, static, precision="fp32")
+    assert np.abs(f32.data - want.data).max() <= 1e-5 * scale   # the same in FP32
+    ud = prob.to_device(u.ravel())
+    rounded = torch.empty(prob.nnz, dtype=torch.float32, device="cuda")
+    N.call("apx_assemble_tangent", prob.plan, C.c_void_p(ud.data_ptr()), C.c_void_p(rounded.data_ptr()),
+           N.APX_FP64_ROUNDED, None)
+    torch.cuda.synchronize()
+    assert np.array_equal(rounded.cpu().numpy(), got.data.astype(np.float32))
+    # the layout that the solvers read: two solves must agree with the CSR values
+    x = np.random.default_rng(0).standard_normal(prob.n_free)
+    vals = torch.from_numpy(got.data).cuda()
+    y = torch.empty(prob.n_free, dtype=torch.float64, device="cuda")
+    xd = torch.from_numpy(x).cuda()
+    N.call("apx_spmv", prob.plan, C.c_void_p(vals.data_ptr()), C.c_void_p(xd.data_ptr()), C.c_void_p(y.data_ptr()),
+           N.APX_FP64, None)
+    torch.cuda.synchronize()
+    assert np.abs(y.cpu().numpy() - want @ x).max() <= 1e-12 * scale * np.abs(x).max()
+    r = assembler.assemble_residual(u, settings, static)
+    ro = OA.residual(sets, settings["node coordinates"], u.ravel(), d)
+    assert np.abs(r.ravel() - ro).max() <= 1e-12 * np.abs(ro).max()
+
+
+@pytest.mark.parametrize("kind,size", [("hex", (3, 4, 6)), ("panel", (11, 14)), ("q2", (5, 6))])
+def test_tangent_of_two_sets(torch_gpu, kind, size):
+    """A plan whose elements come as two sets (one with its own material): sums over the sets."""
+    torch = torch_gpu
+    from autopdex_amd import _native as N
+    from autopdex_amd import assembler, backend
+    from oracle import assembly as OA
+    from oracle import elements as OE
+    u, settings, static, sets, d = _problem(kind, size, 1, seed=11)
+    (elem, elems, _), pot = sets[0], static["model"][0]
+    k = elems.shape[0] // 3
+    print(f"[case] two sets {kind} {size}", flush=True)
+    settings["connectivity"] = (np.ascontiguousarray(elems[:k]), np.ascontiguousarray(elems[k:]))
+    static["model"], static["assembling mode"] = (pot, pot), static["assembling mode"] * 2
+    prob = backend.get_problem(u, settings, static)
+    prob.set_params(1, [0.9, 1.3])
+    ud = prob.to_device(u.ravel())
+    both = [(elem, settings["connectivity"][0], None), (OE.NeoHooke(0.9, 1.3), settings["connectivity"][1], None)]
+    free = ~settings["dirichlet dofs"].ravel()
+    want = OA.reduced_tangent(both, settings["node coordinates"], u.ravel(), d, free)
+    scale = np.abs(want.data).max()
+    out = {}
+    for prec, dt in ((N.APX_FP64, torch.float64), (N.APX_FP32, torch.float32), (N.APX_FP64_ROUNDED, torch.float32)):
+        vals = torch.empty(prob.nnz, dtype=dt, device="cuda")
+        N.call("apx_assemble_tangent", prob.plan, C.c_void_p(ud.data_ptr()), C.c_void_p(vals.data_ptr()), prec, None)
+        torch.cuda.synchronize()
+        out[prec] = vals.cpu().numpy()
+    assert np.abs(out[N.APX_FP64] - want.data).max() <= 1e-12 * scale
+    assert np.abs(out[N.APX_FP32] - want.data).max() <= 1e-5 * scale
+    assert np.array_equal(out[N.APX_FP64_ROUNDED], out[N.APX_FP64].astype(np.float32))
+    r = torch.empty(prob.n_dofs, dtype=torch.float64, device="cuda")
+    N.call("apx_assemble_residual", prob.plan, C.c_void_p(ud.data_ptr()), C.c_void_p(r.data_ptr()), None)
+    torch.cuda.synchronize()
+    ro = OA.residual(both, settings["node coordinates"], u.ravel(), d)
+    assert np.abs(r.cpu().numpy() - ro).max() <= 1e-12 * np.abs(ro).max()
+
+
+@pytest.mark.parametrize("kind,size", [("hex", (3, 3, 4)), ("panel", (9, 7)), ("q2", (4, 5))])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_newton_on_row_owner_tangent(torch_gpu, kind, size, precision):
+    """The SELL order of the row-owner tangent, through a Newton solve from a perturbed state."""
+    from autopdex_amd import solver
+    from oracle import assembly as OA
+    u, settings, static, sets, d = _problem(kind, size, 0, seed=5)
+    u[settings["dirichlet dofs"]] = 0.0
+    print(f"[case] newton rows {kind} {size} {precision}", flush=True)
+    static = dict(static, **{"hip precision": precision, "linear tolerance": 1e-10 if precision == "fp64" else 1e-6})
+    sol, infos = solver.solver(u, settings, static, newton_tol=1e-10)
+    assert not infos[2]
+    r = OA.residual(sets, settings["node coordinates"], sol.ravel(), d)
+    assert np.linalg.norm(r[~settings["dirichlet dofs"].ravel()]) <= 1.1e-10
