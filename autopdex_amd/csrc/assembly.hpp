@@ -97,6 +97,10 @@ struct PcgRun {
   // nothing)
   bool external = false;
   bool streaming = false;  // a resident run was given up: not tried again
+  // the matrix as its upper diagonals (streaming runs; null: read as SELL), known from the first
+  // streaming run on it
+  const M* upper = nullptr;
+  bool upper_known = false;
   int start_k = 0;         // iterations before the present resident run
   int maxiter = 0, iterations = 0;
   int64_t launched = 0;
@@ -111,12 +115,15 @@ struct PcgRun {
   PcgRun(Plan& P, const M* vals, const T* inv, hipStream_t st, T* work, double* partials, KState* state);
   ~PcgRun();
   void init(const T* b, T* x, double tol, double atol, int maxiter, double delta);
+  bool extract_lines();
   void launch_iteration();
   KState run();
   void reanchor(const double* r_full);
   void collect_timing();
 };
 
+// Does apx_pcg_noalloc take a solve with values of this size on the plan?
+bool noalloc_accepts(const Plan& P, size_t value_bytes);
 // Jacobi-PCG; workspace taken from the plan.
 apx_krylov_stats pcg(Plan& P, const void* vals, const void* inv_diag, const void* b, void* x, int precision,
                      double tol, double atol, int maxiter, hipStream_t st);

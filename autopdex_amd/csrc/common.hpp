@@ -82,6 +82,17 @@ struct DevBuf {
     APX_HIP(hipMalloc(&p, count * sizeof(T)));
     n = count;
   }
+  // alloc, or false where the device has no room
+  bool try_alloc(size_t count) {
+    release();
+    if (hipMalloc(&p, count * sizeof(T)) == hipSuccess) {
+      n = count;
+      return true;
+    }
+    (void)hipGetLastError();
+    p = nullptr;
+    return false;
+  }
   void upload(const T* host, size_t count) {
     alloc(count);
     if (count) APX_HIP(hipMemcpy(p, host, count * sizeof(T), hipMemcpyHostToDevice));

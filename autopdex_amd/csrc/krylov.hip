@@ -80,13 +80,17 @@ void ensure_krylov_scratch(Plan& P, hipStream_t st) {
 // in-kernel last-block scheme would need an agent-scope release per block,
 // which writes back the whole L2 each time.
 template <int BS, int NV>
-__device__ inline void block_partials(double (&v)[NV], double* partials) {
+__device__ inline void block_partials_at(double (&v)[NV], double* partials, int64_t block) {
   __shared__ double lds[BS / 64];
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
     const double s = block_sum<BS>(v[j], lds);
-    if (threadIdx.x == 0) partials[j * kMaxBlocks + blockIdx.x] = s;
+    if (threadIdx.x == 0) partials[j * kMaxBlocks + block] = s;
   }
+}
+template <int BS, int NV>
+__device__ inline void block_partials(double (&v)[NV], double* partials) {
+  block_partials_at<BS, NV>(v, partials, blockIdx.x);
 }
 
 constexpr int kFinBS = 1024;
@@ -322,6 +326,208 @@ __global__ __launch_bounds__(kSpmvBS) void k_pcg_spmv(int64_t n, int64_t n_chunk
   block_partials<kSpmvBS, 1>(v, partials);
 }
 
+// ---- PCG on a symmetric 9-point matrix ---------------------------------------------------
+// Where the pattern is that of a 9-point stencil on lines of m rows (Plan::line) and A_ij and A_ji
+// have the same bits, the streaming iterations read the matrix as its upper diagonals
+// A[d][i] = A(i, i + o_d), o = 0, 1, m - 1, m, m + 1: five values a row and no columns.
+//
+// A wavefront owns up to 62 neighbouring rows on each of `lines` consecutive lines (lanes 0 and
+// W + 1 hold the rows beside them) and walks down the lines: p of the line below is formed once
+// and stays in registers for three lines, the values that couple a line to the one above are kept
+// from that line, and neighbours within a line come from the lane beside (DPP).  Seven loads of
+// 64 consecutive values a line, all issued a line ahead.  The matrix is read past the caches
+// (non-temporal), which leaves them to the vectors: the update kernel after it 43.9 -> 41.4 us.
+//
+// Bound by HBM: at 2047^2 rows, FP64, 302 MB in 56.5 us (5.3 TB/s) against 512 MB in 109 us for
+// k_pcg_spmv; the iteration 157 -> 114 us.  The same diagonals read without the walk (27 loads a
+// row, neighbours' lines from L2) took 89 us.  Which rows form a line is arithmetic
+// only: entries that a grid's end takes out of the pattern are stored zeros.  Rows of the chunks
+// with entries elsewhere (Plan::irregular) are summed from the SELL values.
+constexpr int kLineLanes = 62;
+constexpr int kLineBS = 256;
+
+struct LineGrid {
+  int m;        // rows per line
+  int width;    // rows per wavefront and line
+  int segments; // wavefronts side by side on a line
+  int lines;    // lines per wavefront
+  int64_t tasks;
+};
+
+template <class T>
+__device__ __forceinline__ T from_lane_below(T v) {  // lane i: lane i - 1's
+  if constexpr (sizeof(T) == 4) {
+    return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x138, 0xf, 0xf, false));
+  } else {
+    const int2 w = __builtin_bit_cast(int2, v);
+    return __builtin_bit_cast(T, int2{__builtin_amdgcn_update_dpp(0, w.x, 0x138, 0xf, 0xf, false),
+                                      __builtin_amdgcn_update_dpp(0, w.y, 0x138, 0xf, 0xf, false)});
+  }
+}
+template <class T>
+__device__ __forceinline__ T from_lane_above(T v) {  // lane i: lane i + 1's
+  if constexpr (sizeof(T) == 4) {
+    return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x130, 0xf, 0xf, false));
+  } else {
+    const int2 w = __builtin_bit_cast(int2, v);
+    return __builtin_bit_cast(T, int2{__builtin_amdgcn_update_dpp(0, w.x, 0x130, 0xf, 0xf, false),
+                                      __builtin_amdgcn_update_dpp(0, w.y, 0x130, 0xf, 0xf, false)});
+  }
+}
+
+// The upper diagonals of a SELL matrix, zero where the pattern has no entry; clears the flag that
+// k_lines_check sets.
+template <class M, class C>
+__global__ __launch_bounds__(kBS) void k_lines_from_sell(int64_t n, int m, const int32_t* __restrict__ indptr,
+                                                         const int32_t* __restrict__ sptr, const C* __restrict__ cols,
+                                                         const M* __restrict__ vals, M* __restrict__ A,
+                                                         int* asymmetric) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *asymmetric = 0;
+  const int o[5] = {0, 1, m - 1, m, m + 1};
+  for (int64_t i = blockIdx.x * (int64_t)kBS + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBS) {
+    const int64_t at = sptr[i >> 6] + (i & 63);
+    const int w = indptr[i + 1] - indptr[i];
+    M a[5] = {};
+    for (int k = 0; k < w; ++k) {
+      const int off = sell_col(cols[at + k * 64], (int32_t)i) - (int32_t)i;
+      const M v = vals[at + k * 64];
+#pragma unroll
+      for (int d = 0; d < 5; ++d)
+        if (off == o[d]) a[d] = v;
+    }
+#pragma unroll
+    for (int d = 0; d < 5; ++d) A[d * n + i] = a[d];
+  }
+}
+
+// Sets the flag where an entry below the diagonal differs from its mirror image in any bit.
+template <class M, class C>
+__global__ __launch_bounds__(kBS) void k_lines_check(int64_t n, int m, const int32_t* __restrict__ indptr,
+                                                     const int32_t* __restrict__ sptr, const C* __restrict__ cols,
+                                                     const M* __restrict__ vals, const M* __restrict__ A,
+                                                     int* asymmetric) {
+  using B = std::conditional_t<sizeof(M) == 8, unsigned long long, unsigned>;
+  const int o[5] = {0, 1, m - 1, m, m + 1};
+  bool differs = false;
+  for (int64_t i = blockIdx.x * (int64_t)kBS + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBS) {
+    const int64_t at = sptr[i >> 6] + (i & 63);
+    const int w = indptr[i + 1] - indptr[i];
+    for (int k = 0; k < w; ++k) {
+      const int col = sell_col(cols[at + k * 64], (int32_t)i);
+      const M v = vals[at + k * 64];
+      if (col >= i) break;  // columns ascend
+#pragma unroll
+      for (int d = 1; d < 5; ++d)
+        if (i - col == o[d]) differs |= __builtin_bit_cast(B, A[d * n + col]) != __builtin_bit_cast(B, v);
+    }
+  }
+  if (differs) *asymmetric = 1;
+}
+
+template <class M, class T, class C>
+__global__ __launch_bounds__(kLineBS) void k_pcg_lines(int64_t n, LineGrid L, const M* __restrict__ A,
+                                                       const uint32_t* __restrict__ irregular,
+                                                       const int32_t* __restrict__ sptr, const C* __restrict__ cols,
+                                                       const M* __restrict__ vals, const T* __restrict__ z,
+                                                       T* __restrict__ pa, T* __restrict__ pb, T* __restrict__ q,
+                                                       KState* S, double* partials) {
+  if (halted(S)) return;
+  const T beta = (T)S->beta;
+  const bool odd = S->k & 1;
+  const T* __restrict__ po = odd ? pb : pa;
+  T* __restrict__ pn = odd ? pa : pb;
+  const int lane = threadIdx.x & 63, N = (int)n;
+  const int64_t block = xcd_block(blockIdx.x, gridDim.x);
+  const int64_t task = block * (kLineBS / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  double v[1] = {0.0};
+  if (task < L.tasks) {
+    const int seg = (int)(task % L.segments), l0 = (int)(task / L.segments) * L.lines;
+    const int j0 = seg * L.width, width = min(L.width, L.m - j0);
+    const bool mine = lane >= 1 && lane <= width;
+    // the wave's rows on line l0; later lines may run past the last row
+    int64_t first = (int64_t)l0 * L.m + j0;  // row of lane 1
+    const int last = min(l0 + L.lines, (N + L.m - 1) / L.m);
+    struct Line {
+      T z, po;
+      M d[5];
+    } next;
+    // row of this lane `lines` lines further on, or out of range
+    auto at = [&](int lines) { return first + (int64_t)lines * L.m + lane - 1; };
+    auto inside = [&](int64_t r) { return r >= 0 && r < n && lane <= width + 1; };
+    auto load_p = [&](int lines) {
+      const int64_t r = at(lines);
+      next.z = next.po = T(0);
+      if (inside(r)) {
+        next.z = z[r];
+        next.po = po[r];
+      }
+    };
+    auto load_d = [&](int lines) {
+      const int64_t r = at(lines);
+#pragma unroll
+      for (int d = 0; d < 5; ++d) next.d[d] = M(0);
+      if (inside(r)) {
+#pragma unroll
+        for (int d = 0; d < 5; ++d) next.d[d] = __builtin_nontemporal_load(A + d * n + r);
+      }
+    };
+    load_p(-1);
+    T pm = next.z + beta * next.po;
+    load_p(0);
+    T pc = next.z + beta * next.po;
+    load_d(-1);
+    T u2 = from_lane_above((T)next.d[2]), u3 = (T)next.d[3], u4 = from_lane_below((T)next.d[4]);
+    load_p(1);
+    load_d(0);
+    T pmL = from_lane_below(pm), pmR = from_lane_above(pm), pcL = from_lane_below(pc), pcR = from_lane_above(pc);
+    for (int l = l0; l < last; ++l, first += L.m) {
+      const Line now = next;
+      if (l + 1 < last) {
+        load_p(2);
+        load_d(1);
+      }
+      const T pd = now.z + beta * now.po;
+      const T pdL = from_lane_below(pd), pdR = from_lane_above(pd);
+      const T d1 = (T)now.d[1];
+      T s = u4 * pmL;
+      s += u3 * pm;
+      s += u2 * pmR;
+      s += from_lane_below(d1) * pcL;
+      s += (T)now.d[0] * pc;
+      s += d1 * pcR;
+      s += (T)now.d[2] * pdL;
+      s += (T)now.d[3] * pd;
+      s += (T)now.d[4] * pdR;
+      const int64_t row = first + lane - 1;
+      if (first < n) {
+        const int64_t c0 = first >> 6, c1 = min(first + width - 1, n - 1) >> 6;
+        if (((irregular[c0 >> 5] >> (c0 & 31)) | (irregular[c1 >> 5] >> (c1 & 31))) & 1) {
+          const int64_t c = row >> 6;
+          if (mine && row < n && ((irregular[c >> 5] >> (c & 31)) & 1)) {
+            const int32_t e = sptr[c] + (int32_t)(row & 63), w = (sptr[c + 1] - sptr[c]) >> 6;
+            s = sell_row<M, T>(vals + e, cols + e, w, (int32_t)row, [&](int32_t col) { return z[col] + beta * po[col]; });
+          }
+        }
+      }
+      if (mine && row < n) {
+        pn[row] = pc;
+        q[row] = s;
+        v[0] += (double)pc * (double)s;
+      }
+      u2 = from_lane_above((T)now.d[2]);
+      u3 = (T)now.d[3];
+      u4 = from_lane_below((T)now.d[4]);
+      pm = pc;
+      pmL = pcL;
+      pmR = pcR;
+      pc = pd;
+      pcL = pdL;
+      pcR = pdR;
+    }
+  }
+  block_partials_at<kLineBS, 1>(v, partials, block);
+}
+
 __global__ __launch_bounds__(kFinBS) void k_pcg_alpha_fin(KState* S, const double* partials, int nb) {
   if (halted(S)) return;
   double tot[1];
@@ -451,6 +657,8 @@ template <class M, class T>
 void PcgRun<M, T>::init(const T* b, T* x_, double tol, double atol, int maxiter_, double delta) {
   x = x_ ? x_ : xw;
   start_k = 0;
+  upper = nullptr;  // the matrix may be another one
+  upper_known = false;
   maxiter = maxiter_ <= 0 ? (int)std::min<int64_t>(10 * n, INT32_MAX / 2) : maxiter_;
   const int g = grid_for(n);
   hipLaunchKernelGGL(k_pcg_init<T>, dim3(g), dim3(kBS), 0, st, n, b, inv, x, r, z, pa, S, part, tol, atol,
@@ -459,9 +667,71 @@ void PcgRun<M, T>::init(const T* b, T* x_, double tol, double atol, int maxiter_
   APX_LAUNCH_CHECK();
 }
 
+// Lines per wavefront: 32 wavefronts a compute unit where there are that many, at least 8 lines (the
+// lines above and below a wavefront's are read twice).  2047^2 rows, FP64: 17 lines (16 wavefronts)
+// 62.3 us, 12 lines 59.0, 8 lines 56.9, 6 lines 55.9, 4 lines 55.2.
+static LineGrid line_grid(const Plan& P) {
+  LineGrid L;
+  L.m = P.line;
+  L.segments = (P.line + kLineLanes - 1) / kLineLanes;
+  L.width = (P.line + L.segments - 1) / L.segments;
+  const int64_t lines = (P.n_free + P.line - 1) / P.line, waves = 256 * 32;
+  L.lines = (int)std::max<int64_t>(8, (lines * L.segments + waves - 1) / waves);
+  L.tasks = (lines + L.lines - 1) / L.lines * L.segments;
+  return L;
+}
+static int line_blocks(const Plan& P) {
+  constexpr int wpb = kLineBS / 64;
+  return (int)round_xcd((line_grid(P).tasks + wpb - 1) / wpb);
+}
+
+// Lines of fewer than 32 rows would leave more than half of a wavefront's lanes idle.  Systems that
+// apx_pcg_noalloc takes keep the SELL kernel, whose sums it shares bit by bit (and where the launches'
+// latency, not the bytes, sets the pace).
+static bool lines_pay(const Plan& P, size_t value_bytes) {
+  return P.line >= 32 && !noalloc_accepts(P, value_bytes);
+}
+
+// The upper diagonals of the run's matrix into the plan's buffer for them, and the flag that tells
+// whether they are not the whole of it (copied to the host with the stop flags); false: another
+// pattern, or no memory (the run then reads the SELL matrix).
+template <class M, class T>
+bool PcgRun<M, T>::extract_lines() {
+  if (external || !lines_pay(P, sizeof(T))) return false;
+  const size_t want = (size_t)(5 * n);
+  M* A;
+  auto room = [&](auto& buf) {
+    if (buf.n < want && !buf.try_alloc(want)) return false;
+    A = (M*)buf.p;
+    return true;
+  };
+  bool have;
+  if constexpr (sizeof(M) == 8)
+    have = room(P.lines64);
+  else
+    have = room(P.lines32);
+  if (!have) return false;
+  if (!P.asymmetric.p) P.asymmetric.alloc(1);
+  const int g = (int)std::min<int64_t>((n + kBS - 1) / kBS, 65536);
+  auto run = [&](auto cols) {
+    using C = std::remove_const_t<std::remove_pointer_t<decltype(cols)>>;
+    hipLaunchKernelGGL((k_lines_from_sell<M, C>), dim3(g), dim3(kBS), 0, st, n, P.line, P.indptr.p, P.sell_ptr.p, cols,
+                       vals, A, P.asymmetric.p);
+    hipLaunchKernelGGL((k_lines_check<M, C>), dim3(g), dim3(kBS), 0, st, n, P.line, P.indptr.p, P.sell_ptr.p, cols,
+                       vals, (const M*)A, P.asymmetric.p);
+  };
+  if (P.sell_dcol.p)
+    run((const int16_t*)P.sell_dcol.p);
+  else
+    run((const int32_t*)P.sell_cols.p);
+  APX_LAUNCH_CHECK();
+  upper = A;
+  return true;
+}
+
 template <class M, class T>
 void PcgRun<M, T>::launch_iteration() {
-  const int gs = grid_chunks(P.n_chunks), gu = grid_for(n);
+  const int gs = upper ? line_blocks(P) : grid_chunks(P.n_chunks), gu = grid_for(n);
   const bool timed = P.timing && !external;
   // timed: the pairs take the SpMV's and the update's own start and end timestamps
   const EventPair e1 = timed ? timing_pair(P) : EventPair{}, e2 = timed ? timing_pair(P) : EventPair{};
@@ -475,7 +745,16 @@ void PcgRun<M, T>::launch_iteration() {
       launch_kernel((k_pcg_spmv<M, T, 4, C>), dim3(gs), dim3(kSpmvBS), 0, st, n, P.n_chunks, P.sell_ptr.p, cols, vals,
                     z, pa, pb, q, S, part);
   };
-  if (P.sell_dcol.p)
+  auto by_lines = [&](auto cols) {
+    using C = std::remove_const_t<std::remove_pointer_t<decltype(cols)>>;
+    launch_kernel(k_pcg_lines<M, T, C>, dim3(gs), dim3(kLineBS), 0, st, n, line_grid(P), upper, P.irregular.p,
+                  P.sell_ptr.p, cols, vals, (const T*)z, pa, pb, q, S, part);
+  };
+  if (upper && P.sell_dcol.p)
+    by_lines((const int16_t*)P.sell_dcol.p);
+  else if (upper)
+    by_lines((const int32_t*)P.sell_cols.p);
+  else if (P.sell_dcol.p)
     spmv((const int16_t*)P.sell_dcol.p);
   else
     spmv((const int32_t*)P.sell_cols.p);
@@ -530,8 +809,12 @@ KState PcgRun<M, T>::run() {
   };
   auto halted_host = [&](int slot) { return flag[4 * slot + 2] != 0 || flag[4 * slot + 3] != 0; };
   // flags after init / reanchor
+  const bool extracted = !upper_known && extract_lines();
+  if (extracted) APX_HIP(hipMemcpyAsync((void*)(flag + 12), P.asymmetric.p, sizeof(int), hipMemcpyDeviceToHost, st));
   APX_HIP(hipMemcpyAsync((void*)(flag + 8), &S->k, 4 * sizeof(int), hipMemcpyDeviceToHost, st));
   APX_HIP(hipStreamSynchronize(st));
+  if (extracted && flag[12]) upper = nullptr;
+  upper_known = true;
   if (external && !halted_host(2)) {
     // no events: enqueue a batch, copy the flags, wait for the stream, test
     const int64_t limit = (int64_t)launched + maxiter + kBatch;
@@ -583,8 +866,10 @@ void PcgRun<M, T>::collect_timing() {
   const bool f64 = sizeof(T) == 8;
   // only launches that executed an iteration are counted; the rest exited at entry
   const size_t k = (size_t)iterations - counted;
+  // by lines: the upper values; z and p_old read, p_new and q written
+  const int64_t line_bytes = n * (5 * (int64_t)sizeof(M) + 4 * (int64_t)sizeof(T));
   timing_collect(P, sizeof(M) == sizeof(T) ? (f64 ? "pcg_spmv_f64" : "pcg_spmv_f32") : "pcg_spmv_f32m_f64v", ev_spmv,
-                 spmv_bytes, k);
+                 upper ? line_bytes : spmv_bytes, k);
   timing_collect(P, f64 ? "pcg_update_f64" : "pcg_update_f32", ev_upd, upd_bytes, k);
   timing_collect(P, f64 ? "pcg_resident_f64" : "pcg_resident_f32", ev_res, 0, ev_res.size());
   counted = iterations;

@@ -52,14 +52,21 @@ __global__ void k_zero_bytes(unsigned char* p, size_t n) {
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = 0;
 }
 
+struct Need {
+  size_t state, part, vals, inv, work;
+  size_t total() const { return state + part + vals + inv + work; }
+};
+Need scratch_need(const Plan& P, size_t ts) {
+  return {256, blocks256(kKrylovPartials * sizeof(double)), blocks256((size_t)P.sell_total * ts),
+          blocks256((size_t)P.n_free * ts), blocks256((size_t)6 * P.n_free * ts)};
+}
+
 template <class T>
 apx_krylov_stats pcg_noalloc(Plan& P, const T* vals_csr, const T* b, T* x, int precond, double tol, double atol,
                              int maxiter, hipStream_t st) {
-  const size_t ts = sizeof(T);
-  const size_t need_state = 256, need_part = blocks256(kKrylovPartials * sizeof(double));
-  const size_t need_vals = blocks256((size_t)P.sell_total * ts), need_inv = blocks256((size_t)P.n_free * ts);
-  const size_t need_work = blocks256((size_t)6 * P.n_free * ts);
-  const size_t need = need_state + need_part + need_vals + need_inv + need_work;
+  const Need part_of = scratch_need(P, sizeof(T));
+  const size_t need_state = part_of.state, need_part = part_of.part, need_vals = part_of.vals, need_inv = part_of.inv;
+  const size_t need = part_of.total();
   if (need > kScratchBytes)
     throw Error(APX_ERR_ARG, "apx_pcg_noalloc: the solve needs " + std::to_string(need) + " bytes of scratch (" +
                                  std::to_string(P.n_free) + " rows, " + std::to_string(P.sell_total) +
@@ -92,6 +99,8 @@ apx_krylov_stats pcg_noalloc(Plan& P, const T* vals_csr, const T* b, T* x, int p
   return out;
 }
 }  // namespace
+
+bool noalloc_accepts(const Plan& P, size_t value_bytes) { return scratch_need(P, value_bytes).total() <= kScratchBytes; }
 
 }  // namespace apx
 

@@ -77,11 +77,43 @@ int64_t Plan::device_bytes() const {
   int64_t b = coords.bytes() + dmask.bytes() + full2red.bytes() + red2full.bytes() + indptr.bytes() +
               indices.bytes() + diag_slot.bytes() + sell_ptr.bytes() + sell_cols.bytes() + sell_dcol.bytes() +
               csr2sell.bytes() + vals64.bytes() + vals32.bytes() + w64.bytes() + w32.bytes() + r_full.bytes() +
-              diag_full.bytes() + partials.bytes() + element_vectors.bytes() + element_matrices.bytes();
+              diag_full.bytes() + partials.bytes() + lines64.bytes() + lines32.bytes() + element_vectors.bytes() + element_matrices.bytes();
   for (auto& s : sets)
     b += s.conn.bytes() + s.conn_orig.bytes() + s.inc_ptr.bytes() + s.inc.bytes() + s.touched.bytes() + s.rn_ptr.bytes() +
          s.rn.bytes() + s.code.bytes();
   return b;
+}
+
+// Is the reduced matrix that of a 9-point stencil on lines of m rows, but for a few chunks (the
+// corners of a grid whose Dirichlet mask leaves them free)?  m is read off a fullest row in the
+// middle.
+static void find_lines(Plan& P) {
+  P.line = 0;
+  if (P.max_row != 9 || P.n_free >= INT32_MAX / 2) return;
+  int64_t full = P.n_free / 2;
+  while (P.indptr_h[full + 1] - P.indptr_h[full] != 9) full = (full + 1) % P.n_free;
+  const int32_t* c = P.indices_h.data() + P.indptr_h[full];
+  const int32_t m = c[8] - (int32_t)full - 1;
+  const int32_t off[9] = {-m - 1, -m, -m + 1, -1, 0, 1, m - 1, m, m + 1};
+  std::vector<uint32_t> irregular((P.n_chunks + 31) / 32, 0);
+  // up to one chunk in sixteen may be read from the SELL values
+  int64_t left = P.n_chunks / 16;
+  for (int64_t ch = 0; ch < P.n_chunks; ++ch) {
+    bool regular = true;
+    for (int64_t r = ch * kSellC; r < std::min<int64_t>(P.n_free, (ch + 1) * kSellC) && regular; ++r) {
+      int at = 0;  // both ascend
+      for (int32_t k = P.indptr_h[r]; k < P.indptr_h[r + 1] && regular; ++k, ++at) {
+        const int32_t o = P.indices_h[k] - (int32_t)r;
+        while (at < 9 && off[at] < o) ++at;
+        regular = at < 9 && off[at] == o;
+      }
+    }
+    if (regular) continue;
+    if (--left < 0) return;
+    irregular[ch / 32] |= 1u << (ch % 32);
+  }
+  P.line = m;
+  P.irregular_h.swap(irregular);
 }
 
 // Node -> (element, local index) pairs of a set, in element order.
@@ -239,6 +271,8 @@ void plan_build_host(Plan& P, std::vector<std::vector<int32_t>>& conn_perm) {
       P.csr2sell_h[k] = (int32_t)s;
     }
   }
+
+  find_lines(P);
 
   // 4b. structured Q1 grids (owner-tile kernels)
   for (auto& s : P.sets) {
@@ -403,6 +437,7 @@ void plan_finalize(Plan& P) {
     }
   }
   P.csr2sell.upload(P.csr2sell_h.data(), P.csr2sell_h.size());
+  if (P.line) P.irregular.upload(P.irregular_h.data(), P.irregular_h.size());
   std::vector<int32_t>().swap(P.sell_cols_h);
   std::vector<int32_t>().swap(P.csr2sell_h);
   for (size_t si = 0; si < P.sets.size(); ++si) {

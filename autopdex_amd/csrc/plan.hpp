@@ -94,6 +94,16 @@ struct Plan {
   // instead of 4 in the SpMV's stream.  Matrices of bandwidth under 2^15 (every structured grid
   // here, 3-DOF grids up to about 100^3 nodes) qualify.
   DevBuf<int16_t> sell_dcol;
+  // Reduced pattern of a 9-point stencil on lines of `line` rows (one DOF per node on a structured
+  // quad grid): every entry lies 0, 1, line - 1, line or line + 1 rows from the diagonal, but for
+  // the chunks whose bit is set in irregular.  0: no such pattern.
+  int32_t line = 0;
+  std::vector<uint32_t> irregular_h;
+  DevBuf<uint32_t> irregular;
+  // a streaming PCG run's matrix as its five upper diagonals, and whether they are not all of it
+  DevBuf<double> lines64;
+  DevBuf<float> lines32;
+  DevBuf<int> asymmetric;
   int64_t bandwidth = 0;  // largest |column - row|
   int max_row = 0;        // most entries in a row
   DevBuf<int32_t> csr2sell;    // nnz
