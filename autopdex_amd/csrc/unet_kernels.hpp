@@ -993,17 +993,34 @@ __device__ __forceinline__ uint32_t relu_keep(uint32_t q, uint32_t m) {
   return q & keep;
 }
 
+//
+// Both operands want four consecutive pixels of one channel in a lane, and LDS holds a pixel's
+// channels together: ds_read_b64_tr_b16 reads four pixels x 16 channels per 16 lanes and hands
+// lane i channel i's four pixels (the layout that the 16 x 16 x 16 MFMA takes).  A wavefront
+// owns KPW blocks of 16 k for all co tiles, so that a block of 16 pixels takes KPW + NT reads for
+// KPW x NT MFMAs (13 and 36 at 64 -> 64 channels).  Formed from 16-bit reads, four per operand and
+// fragment, the same MFMAs waited for 9,600 LDS instructions a tile: over the 25 layers of 64 -> 64
+// channels of a batch of four 513^2 grids 48 us a launch (now 13.9), 16 -> 16 at 513^2 41.7 (27.7).
+constexpr int wgrad_stride(int c) {
+  // elements per pixel: rows start 8 dwords apart modulo the 64 banks, so that the 8 rows of a half
+  // wavefront's read meet in no bank
+  return c == 16 ? 16 : c + 16;
+}
+
+typedef short wgrad_s4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ bf16x4 read_transposed(const uint16_t* p) {
+  return (bf16x4)__builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) wgrad_s4*)p);
+}
+
 template <int CI, int CO, bool YM>
 __global__ __launch_bounds__(kConvThreads) void k_conv3x3_wgrad(WgradArgs a) {
-  constexpr int S = lds_stride(CI);
+  constexpr int S = CI >= 16 ? wgrad_stride(CI) : lds_stride(CI);
   constexpr int COP = round16(CO);
   constexpr int KB = CI >= 16 ? 9 * (CI / 16) : (9 * CI + 15) / 16;
   constexpr int WK = KB * 16;
   constexpr int NT = COP / 16;
-  constexpr int SD = COP + 4;  // LDS stride of the dY tile
-  // fragments (co tile n, k block kb) are distributed over the 4 wavefronts
-  constexpr int NF = NT * KB;
-  constexpr int FPW = (NF + kTileH - 1) / kTileH;
+  constexpr int SD = wgrad_stride(COP);  // LDS stride of the dY tile
+  constexpr int KPW = (KB + kTileH - 1) / kTileH;  // k blocks per wavefront
   static_assert(CI % 8 == 0 || CI <= 2, "X loads: 8 channels, or one pixel of at most 2");
   static_assert(CO % 16 == 0 || CO <= 2, "dY loads: 8 channels, or one pixel of at most 2");
   constexpr int XL = CI % 8 == 0 ? CI / 8 : 1, DL = CO % 8 == 0 ? CO / 8 : 1;  // loads per pixel
@@ -1024,9 +1041,20 @@ __global__ __launch_bounds__(kConvThreads) void k_conv3x3_wgrad(WgradArgs a) {
   if constexpr (CO < COP)
     for (int i = threadIdx.x; i < NPD * (COP - CO); i += kConvThreads)
       sd[(i / (COP - CO)) * SD + CO + i % (COP - CO)] = 0;
-  f32x4 acc[FPW];
+  f32x4 acc[KPW][NT];
 #pragma unroll
-  for (int f = 0; f < FPW; ++f) acc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int f = 0; f < KPW; ++f)
+#pragma unroll
+    for (int n = 0; n < NT; ++n) acc[f][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // this lane's place in a transposed read (pixel 4 lg + lr / 4, channels 4 (lr % 4)), and where the
+  // wave's k blocks start: tap t's pixel and first channel
+  const int px_lane = 4 * lg + (lr >> 2), ch_lane = 4 * (lr & 3);
+  int kstart[KPW];
+#pragma unroll
+  for (int f = 0; f < KPW; ++f) {
+    const int kb = min(wave * KPW + f, KB - 1), t = kb * 16 / CI;
+    kstart[f] = ((t / 3) * (kTileW + 2) + t % 3) * S + kb * 16 % CI;
+  }
   float bacc = 0.f;  // bias partial: thread -> (row = wave, co = lane) when lane < COP
   u32x4 qx[RX], qd[RD];
   for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
@@ -1115,58 +1143,46 @@ __global__ __launch_bounds__(kConvThreads) void k_conv3x3_wgrad(WgradArgs a) {
       for (int px = 0; px < kTileW; ++px) s += bf2f(sd[(wave * kTileW + px) * SD + lane]);
       bacc += s;
     }
-    // K = pixels of the tile: 4 rows x 64 px = 16 blocks of 16 px.  A wave's fragments cover at
-    // most two co tiles, n0 and n0 + 1 (FPW <= KB), so their A fragments are read once per pixel
-    // block and selected per fragment (the compiler cannot see that fid / KB is constant over f)
-    constexpr int kAN = 2;
-    static_assert(FPW <= KB, "a wave's fragments span at most two co tiles");
-    const int n0 = min(wave * FPW / KB, NT - 1);
+    // K = pixels of the tile: 4 rows x 64 px = 16 blocks of 16 px
+#pragma unroll 2
     for (int pb = 0; pb < kTileH * (kTileW / 16); ++pb) {
       const int row = pb / (kTileW / 16), px0 = (pb % (kTileW / 16)) * 16;
-      // A fragment: A[co = n*16 + lr][px = px0 + 4 lg + j] = dY[px][co]
-      bf16x4 an[kAN];
+      // A fragments: A[co = n*16 + lr][px = px0 + 4 lg + j] = dY[px][co]
+      bf16x4 an[NT], bn[KPW];
+      const uint16_t* d0 = sd + (row * kTileW + px0 + px_lane) * SD + ch_lane;
 #pragma unroll
-      for (int q = 0; q < kAN; ++q) {
-        const int nq = min(n0 + q, NT - 1);
+      for (int n = 0; n < NT; ++n) an[n] = read_transposed(d0 + n * 16);
+      // B fragments: B[px = px0 + 4 lg + j][k = kb*16 + lr] = X[px + o_t][ci]
+      if constexpr (CI >= 16) {
+        const uint16_t* x0 = sx + (row * (kTileW + 2) + px0 + px_lane) * S + ch_lane;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) an[q][j] = (short)sd[(row * kTileW + px0 + 4 * lg + j) * SD + nq * 16 + lr];
-      }
+        for (int f = 0; f < KPW; ++f) bn[f] = read_transposed(x0 + kstart[f]);
+      } else {
 #pragma unroll
-      for (int f = 0; f < FPW; ++f) {
-        const int fid = wave * FPW + f;
-        if (fid < NF) {
-        const int n = fid / KB, kb = fid % KB;
-        bf16x4 bf;
-        const bf16x4 af = n == n0 ? an[0] : an[kAN - 1];
-        // B fragment: B[px = px0 + 4 lg + j][k = kb*16 + lr] = X[px + o_t][ci]
+        for (int f = 0; f < KPW; ++f) {
+          const int k = (wave * KPW + f) * 16 + lr, t = k / CI, c = k % CI;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int k = kb * 16 + lr;
-          const int px = px0 + 4 * lg + j;
-          short v = 0;
-          if constexpr (CI >= 16) {
-            const int t = k / CI, c = k % CI;
-            v = (short)sx[((row + t / 3) * (kTileW + 2) + px + t % 3) * S + c];
-          } else if (k < 9 * CI) {
-            const int t = k / CI, c = k % CI;
-            v = (short)sx[((row + t / 3) * (kTileW + 2) + px + t % 3) * S + c];
-          }
-          bf[j] = v;
-        }
-        acc[f] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(af, bf, acc[f], 0, 0, 0);
+          for (int j = 0; j < 4; ++j)
+            bn[f][j] = k < 9 * CI ? (short)sx[((row + t / 3) * (kTileW + 2) + px0 + 4 * lg + j + t % 3) * S + c] : 0;
         }
       }
+#pragma unroll
+      for (int f = 0; f < KPW; ++f)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[f][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(an[n], bn[f], acc[f][n], 0, 0, 0);
     }
   }
-  // write this block's partial: D[co][k] (lane: k = kb*16 + lr, co = n*16 + 4 lg + j)
+  // write this block's partial: D[co][k] (lane: k = kb*16 + lr, co = n*16 + 4 lg + j); a last
+  // wavefront's k blocks past KB were computed for nothing
   float* out = a.partial + (int64_t)blockIdx.x * (COP * WK + COP);
 #pragma unroll
-  for (int f = 0; f < FPW; ++f) {
-    const int fid = wave * FPW + f;
-    if (fid < NF) {
-      const int n = fid / KB, kb = fid % KB;
+  for (int f = 0; f < KPW; ++f) {
+    const int kb = wave * KPW + f;
+    if (kb < KB) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) out[(n * 16 + 4 * lg + j) * WK + kb * 16 + lr] = acc[f][j];
+      for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) out[(n * 16 + 4 * lg + j) * WK + kb * 16 + lr] = acc[f][n][j];
     }
   }
   if (lane < COP) sbias[wave][lane] = bacc;
