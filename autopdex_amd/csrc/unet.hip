@@ -97,16 +97,20 @@ void launch_conv_ws(const ConvArgs& a, hipStream_t st) {
 // weight gradient: the blocks the device holds at once (at most kWgradBlocks, the partial
 // buffer's rows); returns the number launched, whose partials k_reduce_wgrad sums
 template <int CI, int CO, bool YM>
-int launch_wgrad_t(const WgradArgs& a, hipStream_t st) {
+int wgrad_blocks_t(const WgradArgs& a) {
   const int64_t tiles = (int64_t)a.B * ((a.W + kTileW - 1) / kTileW) * ((a.H + kTileH - 1) / kTileH);
   static const int64_t cap = std::min<int64_t>(resident_blocks(k_conv3x3_wgrad<CI, CO, YM>), kWgradBlocks);
-  const int g = (int)std::max<int64_t>(1, std::min<int64_t>(tiles, cap));
-  hipLaunchKernelGGL((k_conv3x3_wgrad<CI, CO, YM>), dim3(g), dim3(kConvThreads), 0, st, a);
-  return g;
+  return (int)std::max<int64_t>(1, std::min<int64_t>(tiles, cap));
 }
+// blocks = 0: the number of blocks (partials) of a launch; else the launch
 template <int CI, int CO>
-int launch_wgrad_t(const WgradArgs& a, hipStream_t st) {
-  return a.ymask ? launch_wgrad_t<CI, CO, true>(a, st) : launch_wgrad_t<CI, CO, false>(a, st);
+int wgrad_t(const WgradArgs& a, int blocks, hipStream_t st) {
+  if (!blocks) return a.ymask ? wgrad_blocks_t<CI, CO, true>(a) : wgrad_blocks_t<CI, CO, false>(a);
+  if (a.ymask)
+    hipLaunchKernelGGL((k_conv3x3_wgrad<CI, CO, true>), dim3(blocks), dim3(kConvThreads), 0, st, a);
+  else
+    hipLaunchKernelGGL((k_conv3x3_wgrad<CI, CO, false>), dim3(blocks), dim3(kConvThreads), 0, st, a);
+  return blocks;
 }
 
 #define APX_CONV_CASES(X) \
@@ -145,15 +149,15 @@ void launch_conv(int ci, int co, bool f32, const ConvArgs& a, hipStream_t st) {
                                        " channels");
 }
 
-int launch_wgrad(int ci, int co, const WgradArgs& a, hipStream_t st) {
+int wgrad(int ci, int co, const WgradArgs& a, int blocks, hipStream_t st) {
 #define APX_X(A, B) \
-  if (ci == A && co == B) return launch_wgrad_t<A, B>(a, st);
+  if (ci == A && co == B) return wgrad_t<A, B>(a, blocks, st);
   APX_CONV_CASES(APX_X)
 #undef APX_X
-  if (ci == 16 && co == 1) return launch_wgrad_t<16, 1>(a, st);
-  if (ci == 16 && co == 2) return launch_wgrad_t<16, 2>(a, st);
-  if (ci == 1 && co == 16) return launch_wgrad_t<1, 16>(a, st);
-  if (ci == 2 && co == 16) return launch_wgrad_t<2, 16>(a, st);
+  if (ci == 16 && co == 1) return wgrad_t<16, 1>(a, blocks, st);
+  if (ci == 16 && co == 2) return wgrad_t<16, 2>(a, blocks, st);
+  if (ci == 1 && co == 16) return wgrad_t<1, 16>(a, blocks, st);
+  if (ci == 2 && co == 16) return wgrad_t<2, 16>(a, blocks, st);
   throw Error(APX_ERR_UNSUPPORTED, "no weight-gradient kernel for " + std::to_string(ci) + " -> " +
                                        std::to_string(co) + " channels");
 }
@@ -558,53 +562,73 @@ __global__ __launch_bounds__(kTailThreads) void k_unet_tail(TailArgs args, const
 }
 
 // ---- parameters ---------------------------------------------------------------------------
-__global__ void k_cast_weights(const float* theta, uint16_t* wf, int64_t w_off, int64_t wf_off, int64_t n) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    wf[wf_off + i] = f2bf(theta[w_off + i]);
-}
-
-// dgrad weights: wd[ci][t'*CO + co] = W[co][(8 - t')*CI + ci]
-__global__ void k_flip_weights(const float* theta, uint16_t* wd, int64_t w_off, int64_t wd_off, int CI, int CO,
-                               int wk, int d_cop, int d_wk) {
-  const int64_t n = (int64_t)d_cop * d_wk;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    const int ci = (int)(i / d_wk), k = (int)(i % d_wk);
+// All layers' bf16 weights in one launch (two launches a layer took 4.8 us each of a 46-layer
+// network's training step, 220 us a step in all): blockIdx.y the layer, blockIdx.z 0 the forward
+// layout, 1 the backward-data layout wd[ci][t'*CO + co] = W[co][(8 - t')*CI + ci].
+constexpr int kMaxLayers = 4 * kMaxLevels;  // 2 + 4 (levels - 1) + 1
+struct PrepareArgs {
+  struct Layer {
+    int64_t w_off, wf_off, wd_off;
+    int n, ci, co, wk, d_n, d_wk;
+  } layer[kMaxLayers];
+};
+__global__ __launch_bounds__(256) void k_prepare_weights(PrepareArgs A, const float* __restrict__ theta,
+                                                         uint16_t* __restrict__ wf, uint16_t* __restrict__ wd) {
+  const PrepareArgs::Layer& y = A.layer[blockIdx.y];
+  const int first = blockIdx.x * 256 + threadIdx.x, step = gridDim.x * 256;
+  if (blockIdx.z == 0) {
+    for (int i = first; i < y.n; i += step) wf[y.wf_off + i] = f2bf(theta[y.w_off + i]);
+    return;
+  }
+  for (int i = first; i < y.d_n; i += step) {
+    const int ci = i / y.d_wk, k = i % y.d_wk;
     float v = 0.f;
-    if (ci < CI && k < 9 * CO) {
-      const int tp = k / CO, co = k % CO;
-      v = theta[w_off + (int64_t)co * wk + (8 - tp) * CI + ci];
+    if (ci < y.ci && k < 9 * y.co) {
+      const int tp = k / y.co, co = k % y.co;
+      v = theta[y.w_off + (int64_t)co * y.wk + (8 - tp) * y.ci + ci];
     }
-    wd[wd_off + i] = f2bf(v);
+    wd[y.wd_off + i] = f2bf(v);
   }
 }
 
-// the weight-gradient partials summed over the nblk blocks (row b at b * stride: COP*WK weight
-// entries, then the biases): 64 outputs per block, each of its 16 waves summing a contiguous
-// range of the rows in order, the 16 range sums added in order (deterministic)
+// The weight-gradient partials of several layers summed over their blocks (row b at b * stride:
+// COP*WK weight entries, then the biases): blockIdx.y the layer, 64 outputs per block, each of its
+// 16 waves summing a contiguous range of the rows in order, the 16 range sums added in order
+// (deterministic).  One launch for all layers whose partials fit the buffer together: a launch a
+// layer left the chip idle at both ends of each (35 launches of 8.7 us a step, 305 us, for four
+// 513^2 grids; now two of 63 us).
 constexpr int kReduceWaves = 16;
-__global__ __launch_bounds__(64 * kReduceWaves) void k_reduce_wgrad(const float* partial, int nblk, int64_t stride,
-                                                                    int cop, int wk, int co_real, float* grad,
-                                                                    int64_t w_off, int64_t b_off) {
+struct ReduceArgs {
+  struct Layer {
+    int64_t at, w_off, b_off;
+    int nblk, stride, n_w, n;  // n_w weight entries, n with the real biases
+  } layer[kMaxLayers];
+  int zero_bias;  // a linear network has none: the preconditioner stays linear (and odd)
+};
+__global__ __launch_bounds__(64 * kReduceWaves) void k_reduce_wgrad(ReduceArgs A, const float* __restrict__ partial,
+                                                                    float* __restrict__ grad) {
   __shared__ float red[kReduceWaves][64];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int64_t n = (int64_t)cop * wk + co_real;
-  const int64_t i = blockIdx.x * 64LL + lane;
-  const int per = (nblk + kReduceWaves - 1) / kReduceWaves, b0 = w * per, b1 = min(nblk, b0 + per);
+  const ReduceArgs::Layer& y = A.layer[blockIdx.y];
+  if ((int)blockIdx.x * 64 >= y.n) return;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i = blockIdx.x * 64 + lane;
+  const int per = (y.nblk + kReduceWaves - 1) / kReduceWaves, b0 = w * per, b1 = min(y.nblk, b0 + per);
   float s = 0.f;
-  if (i < n)
-    for (int b = b0; b < b1; ++b) s += partial[(int64_t)b * stride + i];
+  if (i < y.n) {
+    const float* p = partial + y.at + i;
+#pragma unroll 8
+    for (int b = b0; b < b1; ++b) s += p[(int64_t)b * y.stride];
+  }
   red[w][lane] = s;
   __syncthreads();
-  if (w == 0 && i < n) {
+  if (w == 0 && i < y.n) {
     float t = 0.f;
     for (int k = 0; k < kReduceWaves; ++k) t += red[k][lane];
-    if (i < (int64_t)cop * wk)
-      grad[w_off + i] = t;
+    if (i < y.n_w)
+      grad[y.w_off + i] = t;
     else
-      grad[b_off + (i - (int64_t)cop * wk)] = t;
+      grad[y.b_off + (i - y.n_w)] = A.zero_bias ? 0.f : t;
   }
 }
-
 __global__ void k_adam(float* theta, const float* g, float* m, float* v, int64_t n, float lr, float b1, float b2,
                        float eps, float c1, float c2) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
@@ -850,15 +874,15 @@ void UNet::build_tail() {
 }
 
 void UNet::prepare_weights(hipStream_t st) {
-  for (auto& ly : layers) {
-    int g;
-    grid1d((int64_t)ly.cop * ly.wk, g);
-    hipLaunchKernelGGL(k_cast_weights, dim3(g), dim3(256), 0, st, theta.p, wf.p, ly.w_off, ly.wf_off,
-                       (int64_t)ly.cop * ly.wk);
-    grid1d((int64_t)ly.d_cop * ly.d_wk, g);
-    hipLaunchKernelGGL(k_flip_weights, dim3(g), dim3(256), 0, st, theta.p, wd.p, ly.w_off, ly.wd_off, ly.ci, ly.co,
-                       ly.wk, ly.d_cop, ly.d_wk);
+  PrepareArgs A;
+  int most = 1;
+  for (size_t l = 0; l < layers.size(); ++l) {
+    const NetLayer& ly = layers[l];
+    A.layer[l] = {ly.w_off, ly.wf_off, ly.wd_off, ly.cop * ly.wk, ly.ci, ly.co, ly.wk, ly.d_cop * ly.d_wk, ly.d_wk};
+    most = std::max({most, ly.cop * ly.wk, ly.d_cop * ly.d_wk});
   }
+  hipLaunchKernelGGL(k_prepare_weights, dim3((most + 1023) / 1024, (unsigned)layers.size(), 2), dim3(256), 0, st, A,
+                     theta.p, wf.p, wd.p);
   APX_LAUNCH_CHECK();
   weights_ready = true;
 }
@@ -897,21 +921,41 @@ void conv_dgrad(UNet& N, int li, int level, const uint16_t* dy, const uint16_t* 
   launch_conv(ly.co, ly.ci, false, a, st);
 }
 
+// The layers of a backward pass whose partials are in the buffer and wait to be summed.  The buffer
+// holds any one layer's; a layer that does not fit behind the others has them summed first.
+struct PendingReduce {
+  ReduceArgs args;
+  int n = 0;
+  int64_t at = 0;
+  void flush(UNet& N, hipStream_t st) {
+    if (!n) return;
+    int most = 0;
+    for (int l = 0; l < n; ++l) most = std::max(most, args.layer[l].n);
+    args.zero_bias = !N.relu;
+    hipLaunchKernelGGL(k_reduce_wgrad, dim3((most + 63) / 64, n), dim3(64 * kReduceWaves), 0, st, args,
+                       (const float*)N.wpart.p, N.grad.p);
+    n = 0;
+    at = 0;
+  }
+};
+
 void conv_wgrad(UNet& N, int li, int level, const uint16_t* x, const uint16_t* dy, const uint16_t* ymask,
-                hipStream_t st) {
+                PendingReduce& R, hipStream_t st) {
   const NetLayer& ly = N.layers[li];
   WgradArgs a{};
   a.x = x;
   a.dy = dy;
   a.ymask = ly.relu ? ymask : nullptr;
-  a.partial = N.wpart.p;
   a.B = N.batch;
   a.H = N.H[level];
   a.W = N.W[level];
-  const int nblk = launch_wgrad(ly.ci, ly.co, a, st);
-  const int64_t n_out = (int64_t)ly.cop * ly.wk + ly.co;
-  hipLaunchKernelGGL(k_reduce_wgrad, dim3((unsigned)((n_out + 63) / 64)), dim3(64 * kReduceWaves), 0, st, N.wpart.p,
-                     nblk, (int64_t)ly.cop * ly.wk + ly.cop, ly.cop, ly.wk, ly.co, N.grad.p, ly.w_off, ly.b_off);
+  const int nblk = wgrad(ly.ci, ly.co, a, 0, st);
+  const int64_t stride = (int64_t)ly.cop * ly.wk + ly.cop;
+  if (R.at + nblk * stride > (int64_t)N.wpart.n || R.n == kMaxLayers) R.flush(N, st);
+  a.partial = N.wpart.p + R.at;
+  wgrad(ly.ci, ly.co, a, nblk, st);
+  R.args.layer[R.n++] = {R.at, ly.w_off, ly.b_off, nblk, (int)stride, ly.cop * ly.wk, ly.cop * ly.wk + ly.co};
+  R.at += nblk * stride;
 }
 
 // d_0 = conv_e[0](conv_in(x0)) without storing conv_in's output: the input layer is formed while
@@ -1191,30 +1235,28 @@ double UNet::loss_backward(const float* target, hipStream_t st) {
 
 void UNet::backward(hipStream_t st) {
   const int L = levels;
+  PendingReduce R;
   // backward through the decoder
-  conv_wgrad(*this, L_out, 0, u[0].p, gy.p, nullptr, st);
+  conv_wgrad(*this, L_out, 0, u[0].p, gy.p, nullptr, R, st);
   conv_dgrad(*this, L_out, 0, gy.p, nullptr, gU[0].p, st);
   for (int l = 0; l + 1 < L; ++l) {
-    conv_wgrad(*this, L_d[l], l, s[l].p, gU[l].p, u[l].p, st);
+    conv_wgrad(*this, L_d[l], l, s[l].p, gU[l].p, u[l].p, R, st);
     conv_dgrad(*this, L_d[l], l, gU[l].p, u[l].p, gS[l].p, st);
     restrict_(*this, l, ch[l], gS[l].p, gT[l].p, st);  // P^T = R
-    conv_wgrad(*this, L_up[l], l + 1, u[l + 1].p, gT[l].p, nullptr, st);
+    conv_wgrad(*this, L_up[l], l + 1, u[l + 1].p, gT[l].p, nullptr, R, st);
     conv_dgrad(*this, L_up[l], l + 1, gT[l].p, nullptr, gU[l + 1].p, st);
   }
-  conv_wgrad(*this, L_b, L - 1, a[L - 1].p, gU[L - 1].p, u[L - 1].p, st);
+  conv_wgrad(*this, L_b, L - 1, a[L - 1].p, gU[L - 1].p, u[L - 1].p, R, st);
   conv_dgrad(*this, L_b, L - 1, gU[L - 1].p, u[L - 1].p, gA[L - 1].p, st);
   for (int l = L - 2; l >= 0; --l) {
-    conv_wgrad(*this, L_down[l], l + 1, rd[l].p, gA[l + 1].p, a[l + 1].p, st);
+    conv_wgrad(*this, L_down[l], l + 1, rd[l].p, gA[l + 1].p, a[l + 1].p, R, st);
     conv_dgrad(*this, L_down[l], l + 1, gA[l + 1].p, a[l + 1].p, gR[l].p, st);
     prolong_add(*this, l, ch[l], gR[l].p, gS[l].p, gD[l].p, st);  // R^T = P, plus the skip
-    conv_wgrad(*this, L_e[l], l, a[l].p, gD[l].p, d[l].p, st);
+    conv_wgrad(*this, L_e[l], l, a[l].p, gD[l].p, d[l].p, R, st);
     conv_dgrad(*this, L_e[l], l, gD[l].p, d[l].p, gA[l].p, st);
   }
-  conv_wgrad(*this, L_in, 0, x0.p, gA[0].p, a[0].p, st);
-  if (!relu) {
-    // linear network: no biases, so the preconditioner is linear (and odd)
-    for (auto& ly : layers) APX_HIP(hipMemsetAsync(grad.p + ly.b_off, 0, ly.co * sizeof(float), st));
-  }
+  conv_wgrad(*this, L_in, 0, x0.p, gA[0].p, a[0].p, R, st);
+  R.flush(*this, st);
   APX_LAUNCH_CHECK();
 }
 
