@@ -94,22 +94,23 @@ void launch_conv_ws(const ConvArgs& a, hipStream_t st) {
   launch_conv_ws_t<CI, CO, 4>(a, st);
 }
 
-// weight gradient: the blocks the device holds at once (at most kWgradBlocks, the partial
-// buffer's rows); returns the number launched, whose partials k_reduce_wgrad sums
+// weight gradient: a layer's workgroups, as many as the device holds at once (at most kWgradBlocks,
+// the partial buffer's rows) and it has tiles
 template <int CI, int CO, bool YM>
 int wgrad_blocks_t(const WgradArgs& a) {
   const int64_t tiles = (int64_t)a.B * ((a.W + kTileW - 1) / kTileW) * ((a.H + kTileH - 1) / kTileH);
   static const int64_t cap = std::min<int64_t>(resident_blocks(k_conv3x3_wgrad<CI, CO, YM>), kWgradBlocks);
   return (int)std::max<int64_t>(1, std::min<int64_t>(tiles, cap));
 }
-// blocks = 0: the number of blocks (partials) of a launch; else the launch
+// blocks = 0: the workgroups of layer 0 of the batch; else the launch of all its layers
 template <int CI, int CO>
-int wgrad_t(const WgradArgs& a, int blocks, hipStream_t st) {
-  if (!blocks) return a.ymask ? wgrad_blocks_t<CI, CO, true>(a) : wgrad_blocks_t<CI, CO, false>(a);
-  if (a.ymask)
-    hipLaunchKernelGGL((k_conv3x3_wgrad<CI, CO, true>), dim3(blocks), dim3(kConvThreads), 0, st, a);
+int wgrad_t(const WgradBatch& b, int blocks, hipStream_t st) {
+  const bool ym = b.layer[0].ymask != nullptr;
+  if (!blocks) return ym ? wgrad_blocks_t<CI, CO, true>(b.layer[0]) : wgrad_blocks_t<CI, CO, false>(b.layer[0]);
+  if (ym)
+    hipLaunchKernelGGL((k_conv3x3_wgrad<CI, CO, true>), dim3(blocks), dim3(kConvThreads), 0, st, b);
   else
-    hipLaunchKernelGGL((k_conv3x3_wgrad<CI, CO, false>), dim3(blocks), dim3(kConvThreads), 0, st, a);
+    hipLaunchKernelGGL((k_conv3x3_wgrad<CI, CO, false>), dim3(blocks), dim3(kConvThreads), 0, st, b);
   return blocks;
 }
 
@@ -149,7 +150,7 @@ void launch_conv(int ci, int co, bool f32, const ConvArgs& a, hipStream_t st) {
                                        " channels");
 }
 
-int wgrad(int ci, int co, const WgradArgs& a, int blocks, hipStream_t st) {
+int wgrad(int ci, int co, const WgradBatch& a, int blocks, hipStream_t st) {
 #define APX_X(A, B) \
   if (ci == A && co == B) return wgrad_t<A, B>(a, blocks, st);
   APX_CONV_CASES(APX_X)
@@ -566,6 +567,7 @@ __global__ __launch_bounds__(kTailThreads) void k_unet_tail(TailArgs args, const
 // network's training step, 220 us a step in all): blockIdx.y the layer, blockIdx.z 0 the forward
 // layout, 1 the backward-data layout wd[ci][t'*CO + co] = W[co][(8 - t')*CI + ci].
 constexpr int kMaxLayers = 4 * kMaxLevels;  // 2 + 4 (levels - 1) + 1
+static_assert(kMaxLayers <= kWgradLayers, "a batch holds every layer");
 struct PrepareArgs {
   struct Layer {
     int64_t w_off, wf_off, wd_off;
@@ -596,7 +598,7 @@ __global__ __launch_bounds__(256) void k_prepare_weights(PrepareArgs A, const fl
 // 16 waves summing a contiguous range of the rows in order, the 16 range sums added in order
 // (deterministic).  One launch for all layers whose partials fit the buffer together: a launch a
 // layer left the chip idle at both ends of each (35 launches of 8.7 us a step, 305 us, for four
-// 513^2 grids; now two of 63 us).
+// 513^2 grids; now two of 52 us).
 constexpr int kReduceWaves = 16;
 struct ReduceArgs {
   struct Layer {
@@ -921,42 +923,80 @@ void conv_dgrad(UNet& N, int li, int level, const uint16_t* dy, const uint16_t* 
   launch_conv(ly.co, ly.ci, false, a, st);
 }
 
-// The layers of a backward pass whose partials are in the buffer and wait to be summed.  The buffer
-// holds any one layer's; a layer that does not fit behind the others has them summed first.
-struct PendingReduce {
-  ReduceArgs args;
+// The weight gradients of a backward pass: noted as their inputs are written (which nothing in the
+// pass overwrites), run at its end, the layers of one kind per launch.  The partial buffer holds any
+// one layer; where the next does not fit behind the others, those are launched and summed first.
+struct WeightGradients {
+  struct Job {
+    const NetLayer* ly;
+    WgradArgs a;
+    bool done;
+  } jobs[kMaxLayers];
   int n = 0;
-  int64_t at = 0;
-  void flush(UNet& N, hipStream_t st) {
-    if (!n) return;
-    int most = 0;
-    for (int l = 0; l < n; ++l) most = std::max(most, args.layer[l].n);
-    args.zero_bias = !N.relu;
-    hipLaunchKernelGGL(k_reduce_wgrad, dim3((most + 63) / 64, n), dim3(64 * kReduceWaves), 0, st, args,
-                       (const float*)N.wpart.p, N.grad.p);
-    n = 0;
-    at = 0;
+
+  void add(UNet& N, int li, int level, const uint16_t* x, const uint16_t* dy, const uint16_t* ymask) {
+    APX_REQUIRE(n < kMaxLayers, APX_ERR_INTERNAL, "more layers than a network has");
+    const NetLayer& ly = N.layers[li];
+    Job& j = jobs[n++];
+    j = {};
+    j.ly = &ly;
+    j.a.x = x;
+    j.a.dy = dy;
+    j.a.ymask = ly.relu ? ymask : nullptr;
+    j.a.B = N.batch;
+    j.a.H = N.H[level];
+    j.a.W = N.W[level];
+  }
+
+  void run(UNet& N, hipStream_t st) {
+    WgradBatch batch;
+    ReduceArgs sums;
+    int n_sums = 0, blocks = 0;
+    int64_t at = 0;
+    batch.n = 0;
+    auto launch = [&](const NetLayer& ly) {
+      if (batch.n) wgrad(ly.ci, ly.co, batch, blocks, st);
+      batch.n = blocks = 0;
+    };
+    auto reduce = [&] {
+      if (!n_sums) return;
+      int most = 0;
+      for (int l = 0; l < n_sums; ++l) most = std::max(most, sums.layer[l].n);
+      sums.zero_bias = !N.relu;
+      hipLaunchKernelGGL(k_reduce_wgrad, dim3((most + 63) / 64, n_sums), dim3(64 * kReduceWaves), 0, st, sums,
+                         (const float*)N.wpart.p, N.grad.p);
+      n_sums = 0;
+      at = 0;
+    };
+    for (int i = 0; i < n; ++i) {
+      if (jobs[i].done) continue;
+      const NetLayer& kind = *jobs[i].ly;
+      for (int k = i; k < n; ++k) {
+        Job& j = jobs[k];
+        const NetLayer& ly = *j.ly;
+        if (j.done || ly.ci != kind.ci || ly.co != kind.co || !j.a.ymask != !jobs[i].a.ymask) continue;
+        WgradBatch one;
+        one.n = 1;
+        one.layer[0] = j.a;
+        j.a.blocks = wgrad(ly.ci, ly.co, one, 0, st);
+        const int64_t stride = (int64_t)ly.cop * ly.wk + ly.cop;
+        if (at + j.a.blocks * stride > (int64_t)N.wpart.n) {
+          launch(kind);
+          reduce();
+        }
+        j.a.first = blocks;
+        j.a.partial = N.wpart.p + at;
+        batch.layer[batch.n++] = j.a;
+        blocks += j.a.blocks;
+        sums.layer[n_sums++] = {at, ly.w_off, ly.b_off, j.a.blocks, (int)stride, ly.cop * ly.wk, ly.cop * ly.wk + ly.co};
+        at += j.a.blocks * stride;
+        j.done = true;
+      }
+      launch(kind);
+    }
+    reduce();
   }
 };
-
-void conv_wgrad(UNet& N, int li, int level, const uint16_t* x, const uint16_t* dy, const uint16_t* ymask,
-                PendingReduce& R, hipStream_t st) {
-  const NetLayer& ly = N.layers[li];
-  WgradArgs a{};
-  a.x = x;
-  a.dy = dy;
-  a.ymask = ly.relu ? ymask : nullptr;
-  a.B = N.batch;
-  a.H = N.H[level];
-  a.W = N.W[level];
-  const int nblk = wgrad(ly.ci, ly.co, a, 0, st);
-  const int64_t stride = (int64_t)ly.cop * ly.wk + ly.cop;
-  if (R.at + nblk * stride > (int64_t)N.wpart.n || R.n == kMaxLayers) R.flush(N, st);
-  a.partial = N.wpart.p + R.at;
-  wgrad(ly.ci, ly.co, a, nblk, st);
-  R.args.layer[R.n++] = {R.at, ly.w_off, ly.b_off, nblk, (int)stride, ly.cop * ly.wk, ly.cop * ly.wk + ly.co};
-  R.at += nblk * stride;
-}
 
 // d_0 = conv_e[0](conv_in(x0)) without storing conv_in's output: the input layer is formed while
 // staging the level-0 tiles (bit-identical to the two launches)
@@ -1235,28 +1275,28 @@ double UNet::loss_backward(const float* target, hipStream_t st) {
 
 void UNet::backward(hipStream_t st) {
   const int L = levels;
-  PendingReduce R;
+  WeightGradients G;
   // backward through the decoder
-  conv_wgrad(*this, L_out, 0, u[0].p, gy.p, nullptr, R, st);
+  G.add(*this, L_out, 0, u[0].p, gy.p, nullptr);
   conv_dgrad(*this, L_out, 0, gy.p, nullptr, gU[0].p, st);
   for (int l = 0; l + 1 < L; ++l) {
-    conv_wgrad(*this, L_d[l], l, s[l].p, gU[l].p, u[l].p, R, st);
+    G.add(*this, L_d[l], l, s[l].p, gU[l].p, u[l].p);
     conv_dgrad(*this, L_d[l], l, gU[l].p, u[l].p, gS[l].p, st);
     restrict_(*this, l, ch[l], gS[l].p, gT[l].p, st);  // P^T = R
-    conv_wgrad(*this, L_up[l], l + 1, u[l + 1].p, gT[l].p, nullptr, R, st);
+    G.add(*this, L_up[l], l + 1, u[l + 1].p, gT[l].p, nullptr);
     conv_dgrad(*this, L_up[l], l + 1, gT[l].p, nullptr, gU[l + 1].p, st);
   }
-  conv_wgrad(*this, L_b, L - 1, a[L - 1].p, gU[L - 1].p, u[L - 1].p, R, st);
+  G.add(*this, L_b, L - 1, a[L - 1].p, gU[L - 1].p, u[L - 1].p);
   conv_dgrad(*this, L_b, L - 1, gU[L - 1].p, u[L - 1].p, gA[L - 1].p, st);
   for (int l = L - 2; l >= 0; --l) {
-    conv_wgrad(*this, L_down[l], l + 1, rd[l].p, gA[l + 1].p, a[l + 1].p, R, st);
+    G.add(*this, L_down[l], l + 1, rd[l].p, gA[l + 1].p, a[l + 1].p);
     conv_dgrad(*this, L_down[l], l + 1, gA[l + 1].p, a[l + 1].p, gR[l].p, st);
     prolong_add(*this, l, ch[l], gR[l].p, gS[l].p, gD[l].p, st);  // R^T = P, plus the skip
-    conv_wgrad(*this, L_e[l], l, a[l].p, gD[l].p, d[l].p, R, st);
+    G.add(*this, L_e[l], l, a[l].p, gD[l].p, d[l].p);
     conv_dgrad(*this, L_e[l], l, gD[l].p, d[l].p, gA[l].p, st);
   }
-  conv_wgrad(*this, L_in, 0, x0.p, gA[0].p, a[0].p, R, st);
-  R.flush(*this, st);
+  G.add(*this, L_in, 0, x0.p, gA[0].p, a[0].p);
+  G.run(*this, st);
   APX_LAUNCH_CHECK();
 }
 

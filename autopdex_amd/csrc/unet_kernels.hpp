@@ -981,8 +981,19 @@ struct WgradArgs {
   const uint16_t* x;      // B x H x W x CI
   const uint16_t* dy;     // B x H x W x CO
   const uint16_t* ymask;  // ReLU output of the layer (YM only)
-  float* partial;         // gridDim x (COP*WK + COP)
+  float* partial;         // blocks x (COP*WK + COP)
   int B, H, W;
+  int blocks, first;      // workgroups of this layer, and the launch's index of their first
+};
+// The layers of one launch.  A layer's workgroups hold one tile each on the coarse grids, far fewer
+// than compute units, and each layer's launch takes the 10 us that a tile's chain of load, LDS and
+// MFMAs takes: the layers of one kind, all of whose inputs stay in memory until the pass ends, share
+// a launch instead (25 launches of 13.3 us for 64 -> 64 channels of four 513^2 grids, 332 us; now
+// two of 46 us).
+constexpr int kWgradLayers = 48;
+struct WgradBatch {
+  WgradArgs layer[kWgradLayers];
+  int n;
 };
 
 // zero the 16-bit halves of q whose mask half is not > 0 (ReLU backward)
@@ -1000,7 +1011,7 @@ __device__ __forceinline__ uint32_t relu_keep(uint32_t q, uint32_t m) {
 // owns KPW blocks of 16 k for all co tiles, so that a block of 16 pixels takes KPW + NT reads for
 // KPW x NT MFMAs (13 and 36 at 64 -> 64 channels).  Formed from 16-bit reads, four per operand and
 // fragment, the same MFMAs waited for 9,600 LDS instructions a tile: over the 25 layers of 64 -> 64
-// channels of a batch of four 513^2 grids 48 us a launch (now 13.9), 16 -> 16 at 513^2 41.7 (27.7).
+// channels of a batch of four 513^2 grids 48 us a layer (now 13.9), 16 -> 16 at 513^2 41.7 (27.7).
 constexpr int wgrad_stride(int c) {
   // elements per pixel: rows start 8 dwords apart modulo the 64 banks, so that the 8 rows of a half
   // wavefront's read meet in no bank
@@ -1013,7 +1024,11 @@ __device__ __forceinline__ bf16x4 read_transposed(const uint16_t* p) {
 }
 
 template <int CI, int CO, bool YM>
-__global__ __launch_bounds__(kConvThreads) void k_conv3x3_wgrad(WgradArgs a) {
+__global__ __launch_bounds__(kConvThreads) void k_conv3x3_wgrad(WgradBatch batch) {
+  int layer = 0;
+  while (layer + 1 < batch.n && (int)blockIdx.x >= batch.layer[layer + 1].first) ++layer;
+  const WgradArgs& a = batch.layer[layer];
+  const int block = (int)blockIdx.x - a.first;
   constexpr int S = CI >= 16 ? wgrad_stride(CI) : lds_stride(CI);
   constexpr int COP = round16(CO);
   constexpr int KB = CI >= 16 ? 9 * (CI / 16) : (9 * CI + 15) / 16;
@@ -1057,7 +1072,7 @@ __global__ __launch_bounds__(kConvThreads) void k_conv3x3_wgrad(WgradArgs a) {
   }
   float bacc = 0.f;  // bias partial: thread -> (row = wave, co = lane) when lane < COP
   u32x4 qx[RX], qd[RD];
-  for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+  for (int64_t tile = block; tile < ntiles; tile += a.blocks) {
     const int img = (int)(tile / ((int64_t)tiles_x * tiles_y));
     const int trem = (int)(tile % ((int64_t)tiles_x * tiles_y));
     const int ty0 = (trem / tiles_x) * kTileH, tx0 = (trem % tiles_x) * kTileW;
@@ -1174,7 +1189,7 @@ __global__ __launch_bounds__(kConvThreads) void k_conv3x3_wgrad(WgradArgs a) {
   }
   // write this block's partial: D[co][k] (lane: k = kb*16 + lr, co = n*16 + 4 lg + j); a last
   // wavefront's k blocks past KB were computed for nothing
-  float* out = a.partial + (int64_t)blockIdx.x * (COP * WK + COP);
+  float* out = a.partial + (int64_t)block * (COP * WK + COP);
 #pragma unroll
   for (int f = 0; f < KPW; ++f) {
     const int kb = wave * KPW + f;
