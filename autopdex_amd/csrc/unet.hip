@@ -16,6 +16,7 @@
 // preconditioner).  There is no counterpart in the reference.
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 
 #include "assembly.hpp"
 #include "unet.hpp"
@@ -1488,52 +1489,99 @@ void net_output_to_reduced_img(Plan& P, UNet& N, const double* r, void* z, int z
 namespace {
 constexpr int kRedBlocks = 512;
 
-__global__ void k_res_terms(int64_t n, const double* r, const double* w, const double* z, const double* e,
-                            double* res, double* part) {
+// What the loss of one image is made of, as block partials part[j * kRedBlocks + block]:
+//   0 res.res  1 r.r  2 (z - e).(z - e)  3 e.e   res = r - w, w = A z
+//   4, 5, 6    mode 1: z.w, z.r;  mode 2: z.res, e.res, e.r
+constexpr int kLossSums = 7;
+template <int MODE>
+__global__ __launch_bounds__(256) void k_loss_sums(int64_t n, const double* __restrict__ r,
+                                                   const double* __restrict__ w, const double* __restrict__ z,
+                                                   const double* __restrict__ e, double* __restrict__ res,
+                                                   double* __restrict__ part) {
   __shared__ double lds[4];
-  double s[4] = {0.0, 0.0, 0.0, 0.0};
+  double s[kLossSums] = {};
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    const double ri = r[i], di = ri - w[i];
+    const double ri = r[i], wi = w[i], di = ri - wi, zi = z[i];
     res[i] = di;
     s[0] += di * di;
     s[1] += ri * ri;
     if (e) {
-      const double de = z[i] - e[i];
+      const double ei = e[i], de = zi - ei;
       s[2] += de * de;
-      s[3] += e[i] * e[i];
+      s[3] += ei * ei;
+      if constexpr (MODE == 2) {
+        s[5] += ei * di;
+        s[6] += ei * ri;
+      }
     }
+    if constexpr (MODE == 1) {
+      s[4] += zi * wi;
+      s[5] += zi * ri;
+    }
+    if constexpr (MODE == 2) s[4] += zi * di;
   }
-  for (int j = 0; j < 4; ++j) {
+#pragma unroll
+  for (int j = 0; j < (MODE == 0 ? 4 : kLossSums); ++j) {
     const double t = block_sum<256>(s[j], lds);
     if (threadIdx.x == 0) part[j * kRedBlocks + blockIdx.x] = t;
   }
 }
 
-// part[j * kRedBlocks + block] = sum a_j . b_j (j = 0..2; a null a_j gives 0)
-__global__ void k_dots3(int64_t n, const double* a0, const double* b0, const double* a1, const double* b1,
-                        const double* a2, const double* b2, double* part) {
-  __shared__ double lds[4];
-  double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    s0 += a0[i] * b0[i];
-    if (a1) s1 += a1[i] * b1[i];
-    if (a2) s2 += a2[i] * b2[i];
+// The image's loss and the factors of its gradient -cr g + ce (z - e), left on the device so that the
+// step needs the host only once, at its end (a copy and a wait per image, two for the functionals,
+// kept the stream idle 0.3 ms of a step with four images).
+struct LossArgs {
+  const double* part;
+  const double* vals;        // the matrix, whose first diagonal entry gives the sign sA of the (definite) matrix
+  const int32_t* diag_slot;
+  const float* scale;        // of this image
+  double n, w_e;
+  int blocks, have_e;
+  double *cr, *ce, *loss;    // of this image
+};
+template <int MODE>
+__global__ __launch_bounds__(64 * kLossSums) void k_loss_coefficients(LossArgs A) {
+  __shared__ double t[kLossSums];
+  const int j = threadIdx.x >> 6, lane = threadIdx.x & 63;  // one wavefront per sum
+  double v = 0.0;
+  if (MODE != 0 || j < 4) {
+#pragma unroll
+    for (int k = 0; k < kRedBlocks / 64; ++k)
+      if (k * 64 + lane < A.blocks) v += A.part[j * kRedBlocks + k * 64 + lane];
   }
-  s0 = block_sum<256>(s0, lds);
-  s1 = block_sum<256>(s1, lds);
-  s2 = block_sum<256>(s2, lds);
-  if (threadIdx.x == 0) {
-    part[blockIdx.x] = s0;
-    part[kRedBlocks + blockIdx.x] = s1;
-    part[2 * kRedBlocks + blockIdx.x] = s2;
+  v = wave_sum(v);
+  if (lane == 0) t[j] = v;
+  __syncthreads();
+  if (threadIdx.x) return;
+  const double sA = A.vals[A.diag_slot[0]] < 0.0 ? -1.0 : 1.0;
+  const double rr = fmax(t[1], 1e-300), ee = fmax(t[3], 1e-300), err = A.have_e ? A.w_e * t[2] / ee : 0.0;
+  double cr, loss;
+  if constexpr (MODE == 0) {
+    // d/dz: -2 A (r - A z) / ||r||^2 + 2 w_e (z - e) / ||e||^2 ; d/dy = s d/dz
+    loss = t[0] / rr + err;
+    cr = 2.0 / rr;
+  } else if constexpr (MODE == 1) {
+    // energy functional J(z) = sA (z.Az / 2 - z.r) / (s^2 n), gradient sA (A z - r) / (s^2 n)
+    const double sb = *A.scale, norm = sb * sb * A.n;
+    loss = sA * (0.5 * t[4] - t[5]) / norm + err;
+    cr = sA / norm;
+  } else {
+    // relative A-norm error (z - e).Ahat(z - e) / e.Ahat e, Ahat = sA A SPD, A e = r:
+    // Ahat (z - e) = -sA res, so the value is -sA (z - e).res / E and the gradient -2 sA res / E
+    const double E = fmax(sA * t[6], 1e-300);
+    loss = -sA * (t[4] - t[5]) / E + err;
+    cr = 2.0 * sA / E;
   }
+  *A.loss = loss;
+  *A.cr = cr;
+  *A.ce = 2.0 * A.w_e / ee;
 }
 
 // dL/dy at the network output: z = s * dsq * y, so dL/dy = s * dsq * dL/dz
 __global__ void k_grad_out(int64_t n, const int32_t* red2full, const double* Ares, const double* z, const double* e,
-                           double cr, double ce, const double* dsq, const float* scale, int img, float inv_batch,
-                           int64_t n_dofs, uint16_t* gy) {
-  const double s = scale[img];
+                           const double* coef_r, const double* coef_e, const double* dsq, const float* scale, int img,
+                           float inv_batch, int64_t n_dofs, uint16_t* gy) {
+  const double s = scale[img], cr = *coef_r, ce = *coef_e;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
     double g = -cr * Ares[i];
     if (e) g += ce * (z[i] - e[i]);
@@ -1546,78 +1594,49 @@ __global__ void k_grad_out(int64_t n, const int32_t* red2full, const double* Are
 double unet_residual_loss_backward(Plan& P, UNet& N, const double* vals_sell, const double* const* r,
                                    const double* const* e, double w_e, int mode, hipStream_t st) {
   const int64_t n = P.n_free;
+  for (int b = 0; mode == 2 && b < N.batch; ++b)
+    APX_REQUIRE(e && e[b], APX_ERR_ARG, "the A-norm loss needs the exact errors e");
   if (P.tw.n < (size_t)(4 * n)) P.tw.alloc(4 * n);
   double *z = P.tw.p, *w = z + n, *res = z + 2 * n, *Ares = z + 3 * n;
-  if (P.tpart.n < (size_t)(4 * kRedBlocks)) P.tpart.alloc(4 * kRedBlocks);
-  std::vector<double> hp(4 * kRedBlocks);
+  const size_t at = kLossSums * kRedBlocks, want = at + 3 * (size_t)N.batch;
+  if (P.tpart.n < want) P.tpart.alloc(want);
+  double *cr = P.tpart.p + at, *ce = cr + N.batch, *losses = ce + N.batch;
   int g;
   grid1d(n, g);
   const int gr = std::min(g, kRedBlocks);
   APX_HIP(hipMemsetAsync(N.gy.p, 0, N.gy.bytes(), st));
-  net_set_diag_scaling(P, vals_sell, APX_FP64, st);  // the network sees D^-1/2 A D^-1/2
-  // sign of the (definite) matrix from its first diagonal entry
-  double d0 = 1.0;
-  {
-    int32_t slot0 = 0;
-    APX_HIP(hipMemcpy(&slot0, P.diag_slot.p, sizeof(int32_t), hipMemcpyDeviceToHost));
-    APX_HIP(hipMemcpy(&d0, vals_sell + slot0, sizeof(double), hipMemcpyDeviceToHost));
-  }
-  const double sA = d0 < 0.0 ? -1.0 : 1.0;
-  std::vector<float> hscale(N.batch);
-  APX_HIP(hipMemcpy(hscale.data(), N.scale.p, N.batch * sizeof(float), hipMemcpyDeviceToHost));
-  double loss = 0.0;
   for (int b = 0; b < N.batch; ++b) {
+    const double* eb = e ? e[b] : nullptr;
+    const LossArgs A{P.tpart.p, vals_sell, P.diag_slot.p, N.scale.p + b, (double)n, w_e, gr, eb != nullptr,
+                     cr + b, ce + b, losses + b};
     net_output_to_reduced_img(P, N, r[b], z, 1, b, st);
     spmv(P, vals_sell, z, w, APX_FP64, st);
-    hipLaunchKernelGGL(k_res_terms, dim3(gr), dim3(256), 0, st, n, r[b], w, z, e ? e[b] : nullptr, res,
-                       P.tpart.p);
-    APX_HIP(hipMemcpyAsync(hp.data(), P.tpart.p, hp.size() * sizeof(double), hipMemcpyDeviceToHost, st));
-    APX_HIP(hipStreamSynchronize(st));
-    double t[4] = {0, 0, 0, 0};
-    for (int j = 0; j < 4; ++j)
-      for (int k = 0; k < gr; ++k) t[j] += hp[j * kRedBlocks + k];
-    const double rr = std::max(t[1], 1e-300), ee = std::max(t[3], 1e-300);
-    const double* eb = (e && e[b]) ? e[b] : nullptr;
-    if (mode == 1 || mode == 2) {
-      double d[3] = {0.0, 0.0, 0.0};
-      auto dots = [&](const double* a0, const double* b0, const double* a1, const double* b1, const double* a2,
-                      const double* b2) {
-        hipLaunchKernelGGL(k_dots3, dim3(gr), dim3(256), 0, st, n, a0, b0, a1, b1, a2, b2, P.tpart.p);
-        APX_HIP(hipMemcpyAsync(hp.data(), P.tpart.p, 3 * kRedBlocks * sizeof(double), hipMemcpyDeviceToHost, st));
-        APX_HIP(hipStreamSynchronize(st));
-        for (int j = 0; j < 3; ++j)
-          for (int k = 0; k < gr; ++k) d[j] += hp[j * kRedBlocks + k];
-      };
-      double cr;
-      if (mode == 1) {
-        // energy functional J(z) = sA (z.Az / 2 - z.r) / (s^2 n), gradient sA (A z - r) / (s^2 n)
-        const double sb = hscale[b], norm = sb * sb * (double)n;
-        dots(z, w, z, r[b], nullptr, nullptr);
-        loss += sA * (0.5 * d[0] - d[1]) / norm + (eb ? w_e * t[2] / ee : 0.0);
-        cr = sA / norm;
-      } else {
-        // relative A-norm error (z - e).Ahat(z - e) / e.Ahat e, Ahat = sA A SPD, A e = r:
-        // Ahat (z - e) = -sA res, so the value is -sA (z - e).res / E and the gradient -2 sA res / E
-        APX_REQUIRE(eb != nullptr, APX_ERR_ARG, "the A-norm loss needs the exact errors e");
-        dots(z, res, eb, res, eb, r[b]);
-        const double E = std::max(sA * d[2], 1e-300);
-        loss += -sA * (d[0] - d[1]) / E + w_e * t[2] / ee;
-        cr = 2.0 * sA / E;
-      }
-      // g = -cr res (+ the error term) through the Ares slot of k_grad_out
-      hipLaunchKernelGGL(k_grad_out, dim3(g), dim3(256), 0, st, n, P.red2full.p, res, z, eb, cr, 2.0 * w_e / ee,
-                         P.net_dsq.p, N.scale.p, b, 1.f / N.batch, P.n_dofs, N.gy.p);
+    auto terms = [&](auto m) {
+      constexpr int MODE = decltype(m)::value;
+      hipLaunchKernelGGL(k_loss_sums<MODE>, dim3(gr), dim3(256), 0, st, n, r[b], (const double*)w, (const double*)z,
+                         eb, res, P.tpart.p);
+      hipLaunchKernelGGL(k_loss_coefficients<MODE>, dim3(1), dim3(64 * kLossSums), 0, st, A);
+    };
+    const double* grad = res;  // the functionals' gradients are multiples of the residual
+    if (mode == 1) {
+      terms(std::integral_constant<int, 1>{});
+    } else if (mode == 2) {
+      terms(std::integral_constant<int, 2>{});
     } else {
-      loss += t[0] / rr + (eb ? w_e * t[2] / ee : 0.0);
+      terms(std::integral_constant<int, 0>{});
       spmv(P, vals_sell, res, Ares, APX_FP64, st);
-      // d/dz: -2 A (r - A z) / ||r||^2 + 2 w_e (z - e) / ||e||^2 ; d/dy = s d/dz
-      hipLaunchKernelGGL(k_grad_out, dim3(g), dim3(256), 0, st, n, P.red2full.p, Ares, z, eb, 2.0 / rr,
-                         2.0 * w_e / ee, P.net_dsq.p, N.scale.p, b, 1.f / N.batch, P.n_dofs, N.gy.p);
+      grad = Ares;
     }
+    hipLaunchKernelGGL(k_grad_out, dim3(g), dim3(256), 0, st, n, P.red2full.p, grad, z, eb, cr + b, ce + b,
+                       P.net_dsq.p, N.scale.p, b, 1.f / N.batch, P.n_dofs, N.gy.p);
     APX_LAUNCH_CHECK();
   }
   N.backward(st);
+  std::vector<double> host(N.batch);
+  APX_HIP(hipMemcpyAsync(host.data(), losses, N.batch * sizeof(double), hipMemcpyDeviceToHost, st));
   APX_HIP(hipStreamSynchronize(st));
+  double loss = 0.0;
+  for (double v : host) loss += v;
   return loss / N.batch;
 }
 

@@ -137,6 +137,7 @@ void net_target_from_reduced_img(Plan& P, UNet& N, const double* e, float* targe
 // mode 0: residual loss ||r - A z||^2 / ||r||^2; mode 1: energy functional
 // sA (z.Az/2 - z.r) / (s^2 n) with sA the sign of A (minimizer z = A^-1 r);
 // mode 2: relative A-norm error (z-e).sA A (z-e) / e.sA A e (needs e = A^-1 r).
+// The plan's diagonal scaling is that of this matrix (net_set_diag_scaling).
 double unet_residual_loss_backward(Plan& P, UNet& N, const double* vals_sell, const double* const* r,
                                    const double* const* e, double w_e, int mode, hipStream_t st);
 
