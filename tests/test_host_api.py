@@ -114,3 +114,32 @@ def test_fit_rejects_self_fraction_outside_unit_interval(frac):
     from autopdex_amd import learned
     with pytest.raises(ValueError, match="self_fraction"):
         learned.fit(None, 9, 9, self_fraction=frac)
+
+
+@pytest.mark.parametrize("values,ok", [
+    ([2.0, 2.0, 2.0], True), ([2, 2.0, np.float64(2.0)], True), ([2.0, 2.0 * (1 + 4e-15), 2.0], True),
+    ([2.0, 2.0, 2.0 * (1 + 1e-12)], False), ([1 + 1e-30j] * 3, True), ([1 + 1e-30j, 1 + 2e-30j, 1 + 1e-30j], True),
+    ([1 + 1e-10j, 1 + 2e-10j, 1 + 1e-10j], False), ([float("nan")] * 3, False), ([float("inf")] * 3, True),
+    ([np.array([1.0, 2.0])] * 3, True), ([np.array([1.0, 2.0]), np.array([1.0, 2.0]), np.array([1.0, 2.1])], False),
+    ([1.0, np.array([1.0]), 1.0], False), ([[0.0, -0.0], [0.0, 0.0], (0.0, 0.0)], True), ([True, 1.0, 1], True)])
+def test_uniform_parameters_as_allclose_decides(values, ok):
+    """Equal values, values within the tolerance and others, as numbers, arrays and mixtures, with and
+    without settings: the same decision at every point as np.allclose alone, and every point asked."""
+    from autopdex_amd import models
+    x = np.arange(6.0).reshape(3, 2)
+    arrays = [np.asarray(v) for v in values]
+    assert ok == all(a.shape == arrays[0].shape and np.allclose(a, arrays[0], rtol=1e-14, atol=0.0) for a in arrays)
+    for two in (False, True):
+        asked = []
+
+        def at(p):
+            asked.append(int(p[0]) // 2)
+            return values[asked[-1]]
+
+        fun = (lambda p, s: at(p)) if two else (lambda p: at(p))
+        if ok:
+            got = models._uniform(fun, x, {}, "value")
+            assert np.array_equal(got, arrays[0]) and got.dtype in (np.float64, np.complex128) and asked == [0, 1, 2]
+        else:
+            with pytest.raises(NotImplementedError, match="value varies"):
+                models._uniform(fun, x, {}, "value")
