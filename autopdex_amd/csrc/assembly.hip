@@ -185,10 +185,6 @@ static void dispatch(Plan& P, ElemSet& S, const double* u, double* r, void* vals
   }
 }
 
-void assemble_set_colour_residual(Plan& P, ElemSet& S, const double* u, double* r, hipStream_t st) {
-  dispatch<double, MODE_RES>(P, S, u, r, nullptr, st);
-}
-
 // Algorithmic (compulsory) bytes of one assembly: what the kernels that run
 // must move at least once -- coordinates and DOFs read, outputs written; the
 // colour path also reads the connectivity (and, for the tangent, the slot

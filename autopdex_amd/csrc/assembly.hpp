@@ -22,8 +22,6 @@ int64_t tangent_coo_entries(const Plan& P);
 void assemble_tangent_coo(Plan& P, const double* u, void* data, int precision, hipStream_t st);
 int64_t residual_bytes(const Plan& P);
 int64_t tangent_bytes(const Plan& P, int precision);
-// one set's residual through the colour kernels (r += ...)
-void assemble_set_colour_residual(Plan& P, ElemSet& S, const double* u, double* r, hipStream_t st);
 
 // structured.hip: owner-tile kernels for structured Q1 grids
 // mode: 0 residual, 1 tangent, 2 diagonal

@@ -253,7 +253,7 @@ __global__ __launch_bounds__(kTBS) void k_tile(TileArgs A) {
     gx[q][0] = in ? A.cx[node] : 0.0;
     gx[q][1] = in ? A.cy[node] : 0.0;
 #pragma unroll
-    for (int c = 0; c < D; ++c) gu[q][c] = (MODE == TILE_RES && in) ? A.u[node * D + c] : 0.0;
+    for (int c = 0; c < D; ++c) gu[q][c] = (MODE == TILE_RES && in && A.u) ? A.u[node * D + c] : 0.0;
     gn[q][0] = (M::NODAL && in) ? A.mp.nodal[0][node] : 0.0;
     gn[q][1] = (M::NODAL && in) ? A.mp.nodal[1][node] : 0.0;
     gm[q] = (MODE == TILE_TAN && in) ? (A.dmask[node] ? 1 : 0) : 2;  // 2: outside the grid
@@ -540,18 +540,18 @@ void run_tile(Plan& P, ElemSet& S, const double* u, double* r, void* vals, const
 }
 }  // namespace
 
-// The u-independent part of a precomputed-source model's residual (its value
-// at u = 0), assembled once per parameter set by the colour kernels.
+// The u-independent part of a precomputed-source model's residual (its value at u = 0), assembled
+// once per parameter set, which for the solvers is once a call: one launch of the residual kernel
+// without u.  (A launch per colour into a cleared vector, with a vector of zeros allocated, waited
+// for and freed, took 4 x 72 us at 2049^2 nodes instead of 148, and at 17^2 nodes 35
+// of a Newton solve's 286 us.)  Waited for, since the next call may come on another stream.
 static const double* source_load(Plan& P, ElemSet& S, hipStream_t st) {
   if (S.model != APX_MODEL_POISSON_SOURCE) return nullptr;
   if (!S.load_valid) {
     if (S.load.n < (size_t)P.n_dofs) S.load.alloc(P.n_dofs);
-    DevBuf<double> zero;
-    zero.alloc(P.n_dofs);
-    fill<double>(zero.p, P.n_dofs, 0.0, st);
-    fill<double>(S.load.p, P.n_dofs, 0.0, st);
-    assemble_set_colour_residual(P, S, zero.p, S.load.p, st);
-    APX_HIP(hipStreamSynchronize(st));  // `zero` is freed on return
+    APX_REQUIRE(P.d == 1, APX_ERR_ARG, "Poisson model needs one DOF per node");
+    run_tile<PoissonSource<4, 2>, double, TILE_RES>(P, S, nullptr, S.load.p, nullptr, nullptr, true, st);
+    APX_HIP(hipStreamSynchronize(st));
     S.load_valid = true;
   }
   return S.load.p;
