@@ -40,7 +40,6 @@ bool gather_residual(Plan& P, ElemSet& S, const double* u, double* r, bool overw
 // krylov.hip
 struct KState {
   double gamma, gamma_prev, pAp, alpha, beta, rr, atol2, bb, rr0, rmax2, delta2;
-  double dot_out;  // scratch result of dot / norm kernels
   double rsq;      // flexible CG: sum of squares of the network's input, r scaled by D^-1/2
   int k, maxiter, done, reliable;  // contiguous: copied to the host as one block
 };
@@ -112,7 +111,8 @@ struct PcgRun {
   // state = one KState (its fields are all written by init before they are read)
   PcgRun(Plan& P, const M* vals, const T* inv, hipStream_t st, T* work, double* partials, KState* state);
   ~PcgRun();
-  void init(const T* b, T* x, double tol, double atol, int maxiter, double delta);
+  // right-hand side b, or (r_full given) -r_full on the free DOFs
+  void init(const T* b, const double* r_full, T* x, double tol, double atol, int maxiter, double delta);
   bool extract_lines();
   void launch_iteration();
   KState run();
@@ -127,7 +127,7 @@ apx_krylov_stats pcg(Plan& P, const void* vals, const void* inv_diag, const void
                      double tol, double atol, int maxiter, hipStream_t st);
 // ||r[red2full]||_2 of a full-length FP64 vector (deterministic).
 double free_norm(Plan& P, const double* r_full, hipStream_t st);
-void gather_rhs(Plan& P, const double* r_full, void* b, int precision, hipStream_t st);
+void gather_rhs(Plan& P, const double* r_full, double* b, hipStream_t st);
 void scatter_update(Plan& P, double* u, const void* x, double damping, int precision, hipStream_t st);
 void impose_dirichlet(Plan& P, double* u, const double* values, hipStream_t st);
 

@@ -251,14 +251,45 @@ __device__ __forceinline__ bool halted(const KState* S) { return S->done | S->re
     }                                                                                       \
   }
 
-template <class T>
-__global__ __launch_bounds__(kBS) void k_pcg_init(int64_t n, const T* __restrict__ b, const T* __restrict__ inv,
+// the slots of a resident run start at zero (its meetings count from 1)
+template <int BS>
+__device__ __forceinline__ void clear_resident_slots(double* partials) {
+  static_assert(kResidentSlotsAt == 2 * kMaxBlocks && kResidentClearWords <= 2 * kMaxBlocks, "slots behind two rows");
+  for (int i = threadIdx.x; i < kResidentClearWords; i += BS) partials[kResidentSlotsAt + i] = 0.0;
+}
+
+struct PcgStart {
+  double tol, atol, delta;
+  int maxiter;
+};
+// the scalars of a run from r.z and r.r
+__device__ __forceinline__ void pcg_start(KState* S, double rz, double rr, const PcgStart& A) {
+  S->gamma = rz;
+  S->gamma_prev = rz;
+  S->rr = rr;
+  S->rr0 = rr;
+  S->bb = rr;
+  S->rmax2 = rr;
+  S->delta2 = A.delta * A.delta;
+  S->atol2 = fmax(A.tol * A.tol * rr, A.atol * A.atol);
+  S->beta = 0.0;
+  S->k = 0;
+  S->maxiter = A.maxiter;
+  S->reliable = 0;
+  S->done = !(rr > S->atol2 && 0 < A.maxiter);
+}
+
+// FULL: the right-hand side is -rfull on the free DOFs, else b.  ONE: the launch is one block, which
+// finishes the sums itself (a second launch and its wait were 5 us of a small solve).
+template <class T, bool FULL, bool ONE>
+__global__ __launch_bounds__(kBS) void k_pcg_init(int64_t n, const T* __restrict__ b,
+                                                  const int32_t* __restrict__ red2full,
+                                                  const double* __restrict__ rfull, const T* __restrict__ inv,
                                                   T* __restrict__ x, T* __restrict__ r, T* __restrict__ z,
-                                                  T* __restrict__ pa, KState* S, double* partials, double tol,
-                                                  double atol, int maxiter, double delta) {
+                                                  T* __restrict__ pa, KState* S, double* partials, PcgStart A) {
   double v[2] = {0.0, 0.0};
   T bv[kUnroll], iv[kUnroll];
-  APX_FOR_ELEMENTS(n, { bv[j] = b[i]; iv[j] = inv[i]; }, {
+  APX_FOR_ELEMENTS(n, { bv[j] = FULL ? (T)(-rfull[red2full[i]]) : b[i]; iv[j] = inv[i]; }, {
     const T zi = iv[j] * bv[j];
     x[i] = 0;
     r[i] = bv[j];
@@ -267,35 +298,21 @@ __global__ __launch_bounds__(kBS) void k_pcg_init(int64_t n, const T* __restrict
     v[0] += (double)bv[j] * (double)zi;
     v[1] += (double)bv[j] * (double)bv[j];
   })
-  block_partials<kBS, 2>(v, partials);
+  if constexpr (ONE) {
+    __shared__ double lds[kBS / 64];
+    clear_resident_slots<kBS>(partials);
+    const double rz = block_sum<kBS>(v[0], lds), rr = block_sum<kBS>(v[1], lds);
+    if (threadIdx.x == 0) pcg_start(S, rz, rr, A);
+  } else {
+    block_partials<kBS, 2>(v, partials);
+  }
 }
 
-// the slots of a resident run start at zero (its meetings count from 1)
-__device__ __forceinline__ void clear_resident_slots(double* partials) {
-  static_assert(kResidentSlotsAt == 2 * kMaxBlocks && kResidentClearWords <= 2 * kMaxBlocks, "slots behind two rows");
-  for (int i = threadIdx.x; i < kResidentClearWords; i += kFinBS) partials[kResidentSlotsAt + i] = 0.0;
-}
-
-__global__ __launch_bounds__(kFinBS) void k_pcg_init_fin(KState* S, double* partials, int nb, double tol,
-                                                         double atol, int maxiter, double delta) {
+__global__ __launch_bounds__(kFinBS) void k_pcg_init_fin(KState* S, double* partials, int nb, PcgStart A) {
   double s[2];
   finalize_sums<2>(partials, nb, s);
-  clear_resident_slots(partials);
-  if (threadIdx.x == 0) {
-    S->gamma = s[0];
-    S->gamma_prev = s[0];
-    S->rr = s[1];
-    S->rr0 = s[1];
-    S->bb = s[1];
-    S->rmax2 = s[1];
-    S->delta2 = delta * delta;
-    S->atol2 = fmax(tol * tol * s[1], atol * atol);
-    S->beta = 0.0;
-    S->k = 0;
-    S->maxiter = maxiter;
-    S->reliable = 0;
-    S->done = !(s[1] > S->atol2 && 0 < maxiter);
-  }
+  clear_resident_slots<kFinBS>(partials);
+  if (threadIdx.x == 0) pcg_start(S, s[0], s[1], A);
 }
 
 template <class M, class T, int U, class C>
@@ -605,7 +622,7 @@ __global__ __launch_bounds__(kBS) void k_pcg_reanchor(int64_t n, const int32_t* 
 __global__ __launch_bounds__(kFinBS) void k_pcg_reanchor_fin(KState* S, double* partials, int nb) {
   double s[2];
   finalize_sums<2>(partials, nb, s);
-  clear_resident_slots(partials);
+  clear_resident_slots<kFinBS>(partials);
   if (threadIdx.x == 0) {
     S->beta = s[0] / S->gamma_prev;
     S->gamma = s[0];
@@ -654,16 +671,23 @@ PcgRun<M, T>::~PcgRun() {
 }
 
 template <class M, class T>
-void PcgRun<M, T>::init(const T* b, T* x_, double tol, double atol, int maxiter_, double delta) {
+void PcgRun<M, T>::init(const T* b, const double* r_full, T* x_, double tol, double atol, int maxiter_, double delta) {
   x = x_ ? x_ : xw;
   start_k = 0;
   upper = nullptr;  // the matrix may be another one
   upper_known = false;
   maxiter = maxiter_ <= 0 ? (int)std::min<int64_t>(10 * n, INT32_MAX / 2) : maxiter_;
+  const PcgStart A{tol, atol, delta, maxiter};
   const int g = grid_for(n);
-  hipLaunchKernelGGL(k_pcg_init<T>, dim3(g), dim3(kBS), 0, st, n, b, inv, x, r, z, pa, S, part, tol, atol,
-                     maxiter, delta);
-  hipLaunchKernelGGL(k_pcg_init_fin, dim3(1), dim3(kFinBS), 0, st, S, part, g, tol, atol, maxiter, delta);
+  auto start = [&](auto full, auto one) {
+    hipLaunchKernelGGL((k_pcg_init<T, decltype(full)::value, decltype(one)::value>), dim3(g), dim3(kBS), 0, st, n, b,
+                       P.red2full.p, r_full, inv, x, r, z, pa, S, part, A);
+  };
+  if (r_full)
+    g == 1 ? start(std::true_type{}, std::true_type{}) : start(std::true_type{}, std::false_type{});
+  else
+    g == 1 ? start(std::false_type{}, std::true_type{}) : start(std::false_type{}, std::false_type{});
+  if (g > 1) hipLaunchKernelGGL(k_pcg_init_fin, dim3(1), dim3(kFinBS), 0, st, S, part, g, A);
   APX_LAUNCH_CHECK();
 }
 
@@ -884,7 +908,7 @@ static apx_krylov_stats pcg_t(Plan& P, const T* vals, const T* inv, const T* b, 
                               int maxiter, hipStream_t st) {
   auto t0 = std::chrono::steady_clock::now();
   PcgRun<T> run(P, vals, inv, st);
-  run.init(b, x, tol, atol, maxiter, 0.0);
+  run.init(b, nullptr, x, tol, atol, maxiter, 0.0);
   KState hs = run.run();
   run.collect_timing();
   apx_krylov_stats out{};
@@ -905,44 +929,52 @@ apx_krylov_stats pcg(Plan& P, const void* vals, const void* inv, const void* b, 
 }
 
 // ---- Newton helpers -----------------------------------------------------------------
-__global__ __launch_bounds__(kBS) void k_free_norm(int64_t n, const int32_t* red2full, const double* r, KState* S,
+// The norm goes to the host's pinned word by the kernel itself (a copy behind it took 6 us).  ONE:
+// one block, which finishes the sum.
+template <bool ONE>
+__global__ __launch_bounds__(kBS) void k_free_norm(int64_t n, const int32_t* red2full, const double* r, double* host,
                                                    double* partials) {
   double v[1] = {0.0};
   double rv[kUnroll];
   APX_FOR_ELEMENTS(n, { rv[j] = r[red2full[i]]; }, { v[0] += rv[j] * rv[j]; })
-  block_partials<kBS, 1>(v, partials);
+  if constexpr (ONE) {
+    __shared__ double lds[kBS / 64];
+    const double s = block_sum<kBS>(v[0], lds);
+    if (threadIdx.x == 0) *host = sqrt(s);
+  } else {
+    block_partials<kBS, 1>(v, partials);
+  }
 }
 
-__global__ __launch_bounds__(kFinBS) void k_norm_fin(KState* S, const double* partials, int nb) {
+__global__ __launch_bounds__(kFinBS) void k_norm_fin(double* host, const double* partials, int nb) {
   double s[1];
   finalize_sums<1>(partials, nb, s);
-  if (threadIdx.x == 0) S->dot_out = sqrt(s[0]);
+  if (threadIdx.x == 0) *host = sqrt(s[0]);
 }
 
 double free_norm(Plan& P, const double* r_full, hipStream_t st) {
   ensure_krylov_scratch(P, st);
-  KState* S = (KState*)P.kstate.p;
+  double* host = P.pinned + 16;
   const int g = grid_for(P.n_free);
-  hipLaunchKernelGGL(k_free_norm, dim3(g), dim3(kBS), 0, st, P.n_free, P.red2full.p, r_full, S, P.partials.p);
-  hipLaunchKernelGGL(k_norm_fin, dim3(1), dim3(kFinBS), 0, st, S, P.partials.p, g);
+  if (g == 1) {
+    hipLaunchKernelGGL(k_free_norm<true>, dim3(1), dim3(kBS), 0, st, P.n_free, P.red2full.p, r_full, host,
+                       P.partials.p);
+  } else {
+    hipLaunchKernelGGL(k_free_norm<false>, dim3(g), dim3(kBS), 0, st, P.n_free, P.red2full.p, r_full, host,
+                       P.partials.p);
+    hipLaunchKernelGGL(k_norm_fin, dim3(1), dim3(kFinBS), 0, st, host, (const double*)P.partials.p, g);
+  }
   APX_LAUNCH_CHECK();
-  APX_HIP(hipMemcpyAsync(P.pinned + 16, &S->dot_out, sizeof(double), hipMemcpyDeviceToHost, st));
   APX_HIP(hipStreamSynchronize(st));
-  return P.pinned[16];
+  return *(volatile double*)host;
 }
-
-template <class T>
-__global__ void k_gather_rhs(int64_t n, const int32_t* red2full, const double* r, T* b) {
+__global__ void k_gather_rhs(int64_t n, const int32_t* red2full, const double* r, double* b) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    b[i] = (T)(-r[red2full[i]]);
+    b[i] = -r[red2full[i]];
 }
-
-void gather_rhs(Plan& P, const double* r_full, void* b, int precision, hipStream_t st) {
+void gather_rhs(Plan& P, const double* r_full, double* b, hipStream_t st) {
   const int g = std::max(1, (int)std::min<int64_t>((P.n_free + 255) / 256, 65536));
-  if (precision == APX_FP64)
-    hipLaunchKernelGGL(k_gather_rhs<double>, dim3(g), dim3(256), 0, st, P.n_free, P.red2full.p, r_full, (double*)b);
-  else
-    hipLaunchKernelGGL(k_gather_rhs<float>, dim3(g), dim3(256), 0, st, P.n_free, P.red2full.p, r_full, (float*)b);
+  hipLaunchKernelGGL(k_gather_rhs, dim3(g), dim3(256), 0, st, P.n_free, P.red2full.p, r_full, b);
   APX_LAUNCH_CHECK();
 }
 

@@ -147,9 +147,8 @@ static void newton_standard(NewtonCtx& C, const double* dvals, const apx_newton_
   apx_newton_stats& s = C.s;
   const int vprec = sizeof(V) == 8 ? APX_FP64 : APX_FP32;
   DevBuf<V> vecs;
-  vecs.alloc(2 * P.n_free);
+  vecs.alloc(P.n_free);
   V* inv = vecs.p;
-  V* b = vecs.p + P.n_free;
   M* vals = matrix_buffer<M>(P);
   impose_dirichlet(P, C.u, dvals, C.st);
   C.residual();
@@ -182,7 +181,7 @@ static void newton_standard(NewtonCtx& C, const double* dvals, const apx_newton_
     if (learned && sizeof(M) == 4 && o.reliable_delta > 0.0) eta = std::max(eta, o.reliable_delta);
     auto t0 = std::chrono::steady_clock::now();
     if (learned) {
-      gather_rhs(P, C.r, b64.p, APX_FP64, C.st);
+      gather_rhs(P, C.r, b64.p, C.st);
       FcgResult fr = fcg_solve<M>(P, *P.net, vals, P.net_g, b64.p, x64.p, eta, o.lin_atol, o.lin_maxiter, C.st);
       s.krylov_iterations += fr.iterations;
       if (fr.stagnated) {
@@ -193,12 +192,11 @@ static void newton_standard(NewtonCtx& C, const double* dvals, const apx_newton_
       }
       scatter_update(P, C.u, x64.p, o.damping, APX_FP64, C.st);
     } else {
-      gather_rhs(P, C.r, b, vprec, C.st);
       // after a fallback the iteration budget is Jacobi-PCG's own (at least jax cg's default
       // 10 n_free): 'linear maxiter' was sized for flexible CG with the network
       const int fb_max = (int)std::min<int64_t>(10 * P.n_free, 2000000000);
       const int maxit = fell_back && o.lin_maxiter > 0 ? std::max(o.lin_maxiter, fb_max) : o.lin_maxiter;
-      pcg.init(b, nullptr, eta, o.lin_atol, maxit, 0.0);
+      pcg.init(nullptr, C.r, nullptr, eta, o.lin_atol, maxit, 0.0);
       pcg.iterations = 0;
       pcg.counted = 0;
       KState hs = pcg.run();
@@ -223,9 +221,8 @@ static void newton_reliable(NewtonCtx& C, const double* dvals, const apx_newton_
   apx_newton_stats& s = C.s;
   const int vprec = sizeof(V) == 8 ? APX_FP64 : APX_FP32;
   DevBuf<V> vecs;
-  vecs.alloc(2 * P.n_free);
+  vecs.alloc(P.n_free);
   V* inv = vecs.p;
-  V* b = vecs.p + P.n_free;
   float* vals = matrix_buffer<float>(P);
   impose_dirichlet(P, C.u, dvals, C.st);
   C.residual();
@@ -233,12 +230,11 @@ static void newton_reliable(NewtonCtx& C, const double* dvals, const apx_newton_
   s.initial_residual = res0;
   const double thr = o.relative ? o.newton_tol * res0 : o.newton_tol;
   C.tangent(vals, inv, o.precond);
-  gather_rhs(P, C.r, b, vprec, C.st);
   auto t0 = std::chrono::steady_clock::now();
   PcgRun<float, V> pcg(P, vals, inv, C.st);
   // the FP32 recursion stops on its own at half the Newton threshold; the
   // FP64 residual decides at every anchor
-  pcg.init(b, nullptr, 0.0, 0.5 * thr, o.lin_maxiter, o.reliable_delta);
+  pcg.init(nullptr, C.r, nullptr, 0.0, 0.5 * thr, o.lin_maxiter, o.reliable_delta);
   NewtonTest test;
   double res = res0;
   bool go = true;

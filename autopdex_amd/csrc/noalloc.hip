@@ -88,7 +88,7 @@ apx_krylov_stats pcg_noalloc(Plan& P, const T* vals_csr, const T* b, T* x, int p
   else
     fill<T>(inv, P.n_free, T(1), st);
   PcgRun<T> run(P, sell, inv, st, work, part, state);
-  run.init(b, x, tol, atol, maxiter, 0.0);
+  run.init(b, nullptr, x, tol, atol, maxiter, 0.0);
   KState hs = run.run();
   apx_krylov_stats out{};
   out.iterations = hs.k;

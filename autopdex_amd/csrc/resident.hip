@@ -32,7 +32,9 @@
 // workgroup that waits longer raises ResidentOut::aborted and leaves, and so do those that wait for
 // it.  What the run started from (r, z, p, the scalars) is not written, so the caller then starts
 // the streaming kernels from there, whatever the other workgroups have done.
+#include <atomic>
 #include <condition_variable>
+#include <cstring>
 #include <cstring>
 #include <mutex>
 #include <type_traits>
@@ -54,7 +56,8 @@ struct ResidentArgs {
   const KState* S;
   u64* slots;  // [p.q: G x 2 words][r.z, r.r: G x 4 words], zero before the launch
   u64* zt;     // tagged z of the rows that other workgroups read (2 words a row, FP32: 1)
-  ResidentOut* out;
+  ResidentOut* out;   // on the device
+  ResidentOut* host;  // the same in the host's pinned memory (a copy behind the run took 6 us)
   long long wait_ticks;
 };
 
@@ -121,6 +124,7 @@ struct Tagged {
 // Bounded wait: true while the caller may try again.
 struct Patience {
   ResidentOut* out;
+  ResidentOut* host;
   long long ticks;
   long long t0 = wall_clock64();
   int tries = 0;
@@ -130,6 +134,7 @@ struct Patience {
         __hip_atomic_load(&out->aborted, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
       return true;
     __hip_atomic_store(&out->aborted, 1LL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&host->aborted, 1LL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     *fail = 1;
     return false;
   }
@@ -193,15 +198,16 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs A, const M* __r
   };
   if (S->done | S->reliable) {
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-      KState* o = &A.out->state;
-      report(o);
-      o->gamma = S->gamma;
-      o->gamma_prev = S->gamma_prev;
-      o->beta = S->beta;
-      o->rr = S->rr;
-      o->k = S->k;
-      o->done = S->done;
-      o->reliable = S->reliable;
+      for (KState* o : {&A.out->state, &A.host->state}) {
+        report(o);
+        o->gamma = S->gamma;
+        o->gamma_prev = S->gamma_prev;
+        o->beta = S->beta;
+        o->rr = S->rr;
+        o->k = S->k;
+        o->done = S->done;
+        o->reliable = S->reliable;
+      }
     }
     return;
   }
@@ -313,7 +319,7 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs A, const M* __r
     if (lane == 0) redA[w] = v1;
     __syncthreads();
     if (G > 1) {
-      if (w == 0) meet<NW, 1>(redA, totA, &fail, A.slots, G, number, Patience{A.out, A.wait_ticks});
+      if (w == 0) meet<NW, 1>(redA, totA, &fail, A.slots, G, number, Patience{A.out, A.host, A.wait_ticks});
       __syncthreads();
       if (fail) return;
       pAp = totA[0];
@@ -351,9 +357,9 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs A, const M* __r
     if (G > 1) {
       // the first wave meets the others while the rest fetch the halo
       if (w == 0) {
-        meet<NW, 2>(redB, totB, &fail, A.slots + 2 * G, G, number, Patience{A.out, A.wait_ticks});
+        meet<NW, 2>(redB, totB, &fail, A.slots + 2 * G, G, number, Patience{A.out, A.host, A.wait_ticks});
       } else {
-        Patience wait{A.out, A.wait_ticks};
+        Patience wait{A.out, A.host, A.wait_ticks};
         for (int j = tid - 64; j < n_halo; j += T - 64) {
           const int row = j < n_lo ? w0 + j : row1 + (j - n_lo);
           V v;
@@ -398,17 +404,18 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs A, const M* __r
     p_new[row0 + at(i)] = pw[row0 - w0 + at(i)];
   }
   if (blockIdx.x == 0 && tid == 0) {
-    KState* o = &A.out->state;
-    report(o);
-    o->gamma = gamma;
-    o->gamma_prev = gamma_prev;
-    o->beta = beta;
-    o->alpha = alpha;
-    o->pAp = pAp;
-    o->rr = rr;
-    o->k = k;
-    o->done = done;
-    o->reliable = reliable;
+    for (KState* o : {&A.out->state, &A.host->state}) {
+      report(o);
+      o->gamma = gamma;
+      o->gamma_prev = gamma_prev;
+      o->beta = beta;
+      o->alpha = alpha;
+      o->pAp = pAp;
+      o->rr = rr;
+      o->k = k;
+      o->done = done;
+      o->reliable = reliable;
+    }
   }
 }
 
@@ -561,6 +568,8 @@ bool pcg_resident(Plan& P, const M* vals, const V* inv, V* x, const V* r, const 
   on(std::integral_constant<int, T>{}, std::integral_constant<int, K>{}, std::integral_constant<int, RW>{}, \
      std::integral_constant<bool, XL>{})
   ResidentOut* host = (ResidentOut*)host_state;
+  A.host = host;
+  std::memset(host, 0, sizeof(ResidentOut));
   {
     ResidentLease lease(dev, s.G, P.cus);
     const bool launched = APX_SHAPE(1024, 1, 9, false) || APX_SHAPE(1024, 2, 9, false) || APX_SHAPE(512, 6, 9, true) || APX_SHAPE(512, 8, 9, true) ||
@@ -570,10 +579,10 @@ bool pcg_resident(Plan& P, const M* vals, const V* inv, V* x, const V* r, const 
                           APX_SHAPE(512, 1, 81, false) || APX_SHAPE(1024, 1, 0, false) ||
                           APX_SHAPE(1024, 2, 0, false) || APX_SHAPE(1024, 4, 0, false);
     APX_REQUIRE(launched, APX_ERR_INTERNAL, "resident PCG: no kernel of this shape");
-    APX_HIP(hipMemcpyAsync(host, A.out, sizeof(ResidentOut), hipMemcpyDeviceToHost, st));
     APX_HIP(hipStreamSynchronize(st));
   }
 #undef APX_SHAPE
+  std::atomic_thread_fence(std::memory_order_acquire);  // written by the kernel
   if (host->aborted) {
     fill<V>(x, P.n_free, V(0), st);
     return false;
