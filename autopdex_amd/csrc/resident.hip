@@ -10,11 +10,13 @@
 // What bounds it: the latency of the two meetings, 1 to 2 us each across the 8 XCDs, growing with
 // the number of workgroups, where the four launches of the streaming kernels cost 14 to 20 us an
 // iteration however small the system is.  us per iteration, streaming -> resident (MI355X):
-//   Q1 Poisson FP64: 229 rows 14.3 -> 1.7, 9,805: 17.0 -> 4.0, 39,605: 16.9 -> 5.2,
-//     195,717: 21.8 -> 7.0, 510,565: 33.2 -> 10.2, 1,046,533: 51.7 -> 21.7
-//   panel (18 entries a row): 6,272: 17.4 -> 4.1, 320,800: 36.8 -> 12.0, 524,288: 45.4 -> 18.6
-//   Q2 (50): 1,600: 23.2 -> 3.6, 96,480: 29.2 -> 9.4
-//   Hex8 (81): 26,019: 31.9 -> 10.2 (FP32 22.0 -> 7.0), 123,725: 38.9 -> 21.4 (FP32 26.7 -> 12.5)
+//   Q1 Poisson FP64: 229 rows 14.2 -> 1.7, 9,805: 17.4 -> 3.7, 39,605: 17.3 -> 5.0,
+//     195,717: 23.0 -> 7.0, 510,565: 29.6 -> 10.2, 1,046,533: 39.8 -> 16.6
+//   panel (18 entries a row): 6,272: 18.6 -> 3.8, 320,800: 36.6 -> 10.1, 524,288: 46.1 -> 14.2
+//   Q2 (50): 1,600: 23.2 -> 3.5, 96,480: 29.2 -> 8.6, 320,800: 60.7 -> 28.3
+//   Hex8 (81): 26,019: 32.4 -> 11.2 (FP32 21.9 -> 6.0), 123,725: 39.6 -> 18.3 (FP32 27.0 -> 10.3)
+// Of 14.0 us at 786,944 rows 6 are the products (matrix entries spilled from the registers), 2 the
+// halo, 2 a meeting, the rest updates and sums; of 11 us of the smaller Hex8 4.5, 2.5 and 2.
 //
 // Meeting: a workgroup writes its partial sums into its own slots and reads everybody's, so a
 // sum costs one write and one read of memory that all XCDs see.  A slot is a 64-bit word holding the
@@ -34,7 +36,6 @@
 // the streaming kernels from there, whatever the other workgroups have done.
 #include <atomic>
 #include <condition_variable>
-#include <cstring>
 #include <cstring>
 #include <mutex>
 #include <type_traits>
@@ -107,17 +108,25 @@ struct Tagged {
       store_agent(p, tag | __float_as_uint(v));
     }
   }
+  struct Raw {
+    u64 w[words];
+  };
+  static __device__ __forceinline__ Raw load(const u64* p) {
+    Raw r;
+#pragma unroll
+    for (int i = 0; i < words; ++i) r.w[i] = load_agent(p + i);
+    return r;
+  }
   // false: not there yet
-  static __device__ __forceinline__ bool load(const u64* p, V& v, uint32_t number) {
-    if constexpr (words == 2) {
-      const u64 a = load_agent(p), b = load_agent(p + 1);
-      v = __hiloint2double((int)(uint32_t)a, (int)(uint32_t)b);
-      return (uint32_t)(a >> 32) == number && (uint32_t)(b >> 32) == number;
-    } else {
-      const u64 a = load_agent(p);
-      v = __uint_as_float((uint32_t)a);
-      return (uint32_t)(a >> 32) == number;
-    }
+  static __device__ __forceinline__ bool value(const Raw& r, V& v, uint32_t number) {
+    bool here = true;
+#pragma unroll
+    for (int i = 0; i < words; ++i) here &= (uint32_t)(r.w[i] >> 32) == number;
+    if constexpr (words == 2)
+      v = __hiloint2double((int)(uint32_t)r.w[0], (int)(uint32_t)r.w[1]);
+    else
+      v = __uint_as_float((uint32_t)r.w[0]);
+    return here;
   }
 };
 
@@ -140,6 +149,22 @@ struct Patience {
   }
 };
 
+// N tagged values, value i at p(i), until all are there; all loads of a try are in flight together
+// (each try is a trip past the L2).  false: given up.
+template <class V, int N, class P>
+__device__ __forceinline__ bool collect(V (&v)[N], P p, uint32_t number, Patience& wait, int* fail) {
+  for (;;) {
+    typename Tagged<V>::Raw raw[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) raw[i] = Tagged<V>::load(p(i));
+    bool here = true;
+#pragma unroll
+    for (int i = 0; i < N; ++i) here &= Tagged<V>::value(raw[i], v[i], number);
+    if (here) return true;
+    if (!wait.again(fail)) return false;
+  }
+}
+
 // The first wave's part of a meeting: add up the waves' sums in red (NV x NW), publish them, collect
 // everybody's and leave the totals in out.
 template <int NW, int NV>
@@ -154,19 +179,24 @@ __device__ __forceinline__ void meet(const double* red, double* out, int* fail, 
   double got[NV];
 #pragma unroll
   for (int j = 0; j < NV; ++j) got[j] = 0.0;
-  for (int g = lane; g < G; g += 64) {
-    for (;;) {
-      double v[NV];
-      bool here = true;
+  auto take = [&](auto u, int g0) {
+    constexpr int U = decltype(u)::value;
+    double v[U * NV];
+    if (!collect<double, U * NV>(
+            v, [&](int i) { return slots + ((size_t)min(g0 + lane + 64 * (i / NV), G - 1) * NV + i % NV) * 2; }, number,
+            wait, fail))
+      return false;
 #pragma unroll
-      for (int j = 0; j < NV; ++j) here &= Tagged<double>::load(slots + ((size_t)g * NV + j) * 2, v[j], number);
-      if (here) {
-#pragma unroll
-        for (int j = 0; j < NV; ++j) got[j] += v[j];
-        break;
-      }
-      if (!wait.again(fail)) return;
-    }
+    for (int i = 0; i < U * NV; ++i)
+      if (g0 + lane + 64 * (i / NV) < G) got[i % NV] += v[i];
+    return true;
+  };
+  constexpr int kTwo = NW < 16 ? 2 : 1;  // 1,024 threads have no registers for a second slot
+  if (G <= 64) {
+    if (!take(std::integral_constant<int, 1>{}, 0)) return;
+  } else {
+    for (int g0 = 0; g0 < G; g0 += 64 * kTwo)
+      if (!take(std::integral_constant<int, kTwo>{}, g0)) return;
   }
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
@@ -184,6 +214,16 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs A, const M* __r
                                                     const V* __restrict__ r, const V* __restrict__ z,
                                                     const V* __restrict__ p_old, V* __restrict__ p_new) {
   constexpr int NW = T / 64;
+  // halo entries that a thread asks for at once: as registers are left beside the matrix (1,024 threads
+  // have few and rarely a second entry)
+  constexpr int kRegs = T > 256 ? 131072 / T : 512;
+  constexpr int kLeft = kRegs - K * (RW * (int)(sizeof(M) / 4) + (RW + 1) / 2) - 4 * K * (int)(sizeof(V) / 4);
+  // The positions are unpacked in every iteration where, hoisted by the compiler to a register each,
+  // they would spill the matrix (which is then read back from scratch in every iteration): 81 entries
+  // of FP64 20 x 19 x 21 Hex8 11.9 -> 9.8 us an iteration, 8 x 9 entries 18.3 -> 14.9 us; elsewhere
+  // the unpacking costs up to 0.2 us.
+  constexpr bool kPacked = 5 * K * RW * (int)(sizeof(M) / 4 + 1) > 4 * kRegs;
+  constexpr int kHalo = T == 1024 ? 1 : kLeft >= 128 ? 8 : kLeft >= 96 ? 4 : kLeft >= 64 ? 2 : 1;
   extern __shared__ __align__(16) unsigned char lds_raw[];
   __shared__ double redA[NW], redB[2 * NW], totA[1], totB[2];
   __shared__ int fail;
@@ -284,6 +324,9 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs A, const M* __r
       if constexpr (RW > 0) {
 #pragma unroll
         for (int e = 0; e < RW; ++e) {
+          // the positions are unpacked here: hoisted, each would take a register of its own
+          if constexpr (kPacked)
+            if ((e & 1) == 0) asm volatile("" : "+v"(ci[i][e >> 1]));
           const uint32_t pos = (e & 1) ? ci[i][e >> 1] >> 16 : ci[i][e >> 1] & 0xffffu;
           // FP32 entries of an FP64 run are widened here: hoisted, they would take two registers each
           if constexpr (sizeof(M) < sizeof(V)) asm volatile("" : "+v"(a[i][e]));
@@ -329,23 +372,23 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs A, const M* __r
     alpha = gamma / pAp;
     const V al = (V)alpha;
     double v2[2] = {0.0, 0.0};
-    V zv[K];
+    V zv[XL ? 1 : K];  // XL: formed again from r where it is needed
 #pragma unroll
     for (int i = 0; i < K; ++i) {
-      zv[i] = 0;
       if (!on(i)) continue;
       const int o = at(i);
       const V p = pw[row0 - w0 + o];
       rv[i] -= al * q[i];
+      V zi;
       if constexpr (XL) {
         xl[o] += al * p;
-        zv[i] = il[o] * rv[i];
+        zi = il[o] * rv[i];
       } else {
-        xv[i] += al * p;
-        zv[i] = iv[i] * rv[i];
+        xv[XL ? 0 : i] += al * p;
+        zi = zv[XL ? 0 : i] = iv[XL ? 0 : i] * rv[i];
       }
-      if (seen(i)) Tagged<V>::store(A.zt + (size_t)(row0 + o) * Tagged<V>::words, zv[i], number);
-      v2[0] += (double)rv[i] * (double)zv[i];
+      if (seen(i)) Tagged<V>::store(A.zt + (size_t)(row0 + o) * Tagged<V>::words, zi, number);
+      v2[0] += (double)rv[i] * (double)zi;
       v2[1] += (double)rv[i] * (double)rv[i];
     }
 #pragma unroll
@@ -360,12 +403,19 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs A, const M* __r
         meet<NW, 2>(redB, totB, &fail, A.slots + 2 * G, G, number, Patience{A.out, A.host, A.wait_ticks});
       } else {
         Patience wait{A.out, A.host, A.wait_ticks};
-        for (int j = tid - 64; j < n_halo; j += T - 64) {
-          const int row = j < n_lo ? w0 + j : row1 + (j - n_lo);
-          V v;
-          while (!Tagged<V>::load(A.zt + (size_t)row * Tagged<V>::words, v, number))
-            if (!wait.again(&fail)) break;
-          zh[j] = v;
+        for (int j0 = tid - 64; j0 < n_halo; j0 += kHalo * (T - 64)) {
+          auto entry = [&](int i) { return min(j0 + i * (T - 64), n_halo - 1); };
+          V v[kHalo];
+          if (!collect<V, kHalo>(
+                  v,
+                  [&](int i) {
+                    const int j = entry(i), row = j < n_lo ? w0 + j : row1 + (j - n_lo);
+                    return A.zt + (size_t)row * Tagged<V>::words;
+                  },
+                  number, wait, &fail))
+            break;
+#pragma unroll
+          for (int i = 0; i < kHalo; ++i) zh[entry(i)] = v[i];
         }
       }
       __syncthreads();
@@ -393,7 +443,7 @@ __global__ __launch_bounds__(T) void k_pcg_resident(ResidentArgs A, const M* __r
     for (int i = 0; i < K; ++i)
       if (on(i)) {
         V* p = pw + (row0 - w0) + at(i);
-        *p = zv[i] + be * *p;
+        *p = (XL ? il[at(i)] * rv[i] : zv[XL ? 0 : i]) + be * *p;
       }
     __syncthreads();
   }
