@@ -73,6 +73,18 @@ template <class M, class V>
 bool pcg_resident(Plan& P, const M* vals, const V* inv, V* x, const V* r, const V* z, const V* p_old, V* p_new,
                   unsigned long long* zt, KState* S, double* part, KState* host_state, hipStream_t st);
 
+// Symmetric 9-point matrices by grid lines (krylov.hip): the upper diagonals of SELL values for
+// line_product, with P.asymmetric set on the device where they are not the whole matrix; null: not
+// applicable.  vector_bytes: of an entry of the vectors.
+template <class M>
+const M* line_matrix(Plan& P, const M* vals, size_t vector_bytes, hipStream_t st);
+// p_new = z + beta p_old, q = A p_new, block partials of p.q and (r given) p.r; exits at once when S
+// has a stop flag
+template <class M, class T>
+void line_product(Plan& P, const M* upper, const M* vals, const T* z, T* pa, T* pb, T* q, const T* r, KState* S,
+                  double* part, hipStream_t st);
+int line_blocks(const Plan& P);  // its workgroups
+
 // One preconditioned-CG solve on the plan's SELL matrix with values of type M
 // and Krylov vectors and scalars of type T (M = float, T = double: an FP32
 // matrix with FP64 vectors).  Workspace (r, z, two directions, q, x) comes
@@ -113,7 +125,6 @@ struct PcgRun {
   ~PcgRun();
   // right-hand side b, or (r_full given) -r_full on the free DOFs
   void init(const T* b, const double* r_full, T* x, double tol, double atol, int maxiter, double delta);
-  bool extract_lines();
   void launch_iteration();
   KState run();
   void reanchor(const double* r_full);

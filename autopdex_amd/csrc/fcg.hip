@@ -198,8 +198,12 @@ __global__ void k_fcg_update(int64_t n, const double* pa, const double* pb, cons
   partials_out<kBS, 2>(v, partials);
 }
 
-__global__ __launch_bounds__(kFinBS) void k_fcg_update_fin(KState* S, const double* partials, int nb) {
-  if (S->done) return;
+// The scalars after the iteration go to the host's pinned slot from here (a copy behind took 5 us).
+__global__ __launch_bounds__(kFinBS) void k_fcg_update_fin(KState* S, const double* partials, int nb, KState* host) {
+  if (S->done) {
+    if (threadIdx.x == 0) *host = *S;
+    return;
+  }
   double s[2];
   sums_in<2>(partials, nb, s);
   if (threadIdx.x == 0) {
@@ -207,6 +211,7 @@ __global__ __launch_bounds__(kFinBS) void k_fcg_update_fin(KState* S, const doub
     S->rsq = s[1];
     S->k += 1;
     S->done = !(s[0] > S->atol2 && S->k < S->maxiter);
+    *host = *S;
   }
 }
 }  // namespace
@@ -244,7 +249,8 @@ FcgResult fcg_solve(Plan& P, UNet& N, const T* vals, const double* g_nodal, cons
   } net_scope{N};
   N.timer_plan = P.timing ? &P : nullptr;
   N.stop = &S->done;
-  auto iteration = [&] {
+  const T* upper = line_matrix<T>(P, vals, sizeof(double), st);
+  auto iteration = [&](KState* host) {
     EventPair e0 = timing_begin(P, st);
     net_input_from_reduced_img(P, N, r, 1, g_nodal, &S->rsq, 0, st);  // its scale from the last update
     N.forward(st, false);
@@ -255,15 +261,18 @@ FcgResult fcg_solve(Plan& P, UNet& N, const T* vals, const double* g_nodal, cons
     // timed: the pair takes the SpMV's own start and end timestamps
     const EventPair e1 = P.timing ? timing_pair(P) : EventPair{};
     t_launch_events = P.timing ? &e1 : nullptr;
-    if (P.sell_dcol.p)
+    const int gp = upper ? line_blocks(P) : gs;
+    if (upper)
+      line_product<T, double>(P, upper, vals, z, pa, pb, q, r, S, P.partials.p, st);
+    else if (P.sell_dcol.p)
       launch_kernel(k_fcg_spmv<T, int16_t>, dim3(gs), dim3(kSpmvBS), 0, st, n, P.n_chunks, P.sell_ptr.p,
                     (const int16_t*)P.sell_dcol.p, vals, z, pa, pb, q, r, S, P.partials.p);
     else
       launch_kernel(k_fcg_spmv<T, int32_t>, dim3(gs), dim3(kSpmvBS), 0, st, n, P.n_chunks, P.sell_ptr.p,
                     (const int32_t*)P.sell_cols.p, vals, z, pa, pb, q, r, S, P.partials.p);
-    hipLaunchKernelGGL(k_fcg_alpha_fin, dim3(1), dim3(kFinBS), 0, st, S, P.partials.p, gs);
+    hipLaunchKernelGGL(k_fcg_alpha_fin, dim3(1), dim3(kFinBS), 0, st, S, P.partials.p, gp);
     hipLaunchKernelGGL(k_fcg_update, dim3(gv), dim3(kBS), 0, st, n, pa, pb, q, dsq, x, r, S, P.partials.p);
-    hipLaunchKernelGGL(k_fcg_update_fin, dim3(1), dim3(kFinBS), 0, st, S, P.partials.p, gv);
+    hipLaunchKernelGGL(k_fcg_update_fin, dim3(1), dim3(kFinBS), 0, st, S, P.partials.p, gv, host);
     APX_LAUNCH_CHECK();
     if (P.timing) {
       ev_net.push_back(e0);
@@ -284,14 +293,16 @@ FcgResult fcg_solve(Plan& P, UNet& N, const T* vals, const double* g_nodal, cons
   APX_HIP(hipEventCreateWithFlags(&evs[0], hipEventDisableTiming));
   APX_HIP(hipEventCreateWithFlags(&evs[1], hipEventDisableTiming));
   auto enqueue = [&](int slot) {
-    for (int i = 0; i < kBatch; ++i) iteration();
-    APX_HIP(hipMemcpyAsync((void*)(pin + 128 * slot), S, sizeof(KState), hipMemcpyDeviceToHost, st));
+    for (int i = 0; i < kBatch; ++i) iteration((KState*)(pin + 128 * slot));
     APX_HIP(hipEventRecord(evs[slot], st));
   };
   FcgResult res;
   KState hs;
+  volatile int* flag = (volatile int*)P.pinned;
+  if (upper) APX_HIP(hipMemcpyAsync((void*)flag, P.asymmetric.p, sizeof(int), hipMemcpyDeviceToHost, st));
   APX_HIP(hipMemcpyAsync(&hs, S, sizeof(KState), hipMemcpyDeviceToHost, st));
   APX_HIP(hipStreamSynchronize(st));
+  if (upper && *flag) upper = nullptr;
   res.rr0 = hs.rr0;
   std::vector<double> hist;  // rr after each polled batch
   std::vector<int> hist_k;
@@ -348,7 +359,7 @@ FcgResult fcg_solve(Plan& P, UNet& N, const T* vals, const double* g_nodal, cons
   if (P.timing) {
     const size_t k = (size_t)hs.k;
     const int64_t spmv_bytes =
-        P.sell_total * (int64_t)(sizeof(T) + (P.sell_dcol.p ? 2 : 4)) + (P.n_chunks + 1) * 4 + n * 6 * 8;
+        upper ? n * (5 * (int64_t)sizeof(T) + 5 * 8) : P.sell_total * (int64_t)(sizeof(T) + (P.sell_dcol.p ? 2 : 4)) + (P.n_chunks + 1) * 4 + n * 6 * 8;
     timing_collect(P, "fcg_precond", ev_net, 0, k);
     timing_collect(P, sizeof(T) == 8 ? "fcg_spmv_f64" : "fcg_spmv_f32", ev_spmv, spmv_bytes, k);
     N.collect_timing(k);  // the forward passes of the executed iterations

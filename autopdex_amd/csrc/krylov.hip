@@ -441,13 +441,14 @@ __global__ __launch_bounds__(kBS) void k_lines_check(int64_t n, int m, const int
   if (differs) *asymmetric = 1;
 }
 
-template <class M, class T, class C>
+// DOT: flexible CG, which wants p.r (second partial) beside p.q
+template <class M, class T, class C, bool DOT>
 __global__ __launch_bounds__(kLineBS) void k_pcg_lines(int64_t n, LineGrid L, const M* __restrict__ A,
                                                        const uint32_t* __restrict__ irregular,
                                                        const int32_t* __restrict__ sptr, const C* __restrict__ cols,
                                                        const M* __restrict__ vals, const T* __restrict__ z,
                                                        T* __restrict__ pa, T* __restrict__ pb, T* __restrict__ q,
-                                                       KState* S, double* partials) {
+                                                       const T* __restrict__ res, KState* S, double* partials) {
   if (halted(S)) return;
   const T beta = (T)S->beta;
   const bool odd = S->k & 1;
@@ -456,7 +457,7 @@ __global__ __launch_bounds__(kLineBS) void k_pcg_lines(int64_t n, LineGrid L, co
   const int lane = threadIdx.x & 63, N = (int)n;
   const int64_t block = xcd_block(blockIdx.x, gridDim.x);
   const int64_t task = block * (kLineBS / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  double v[1] = {0.0};
+  double v[DOT ? 2 : 1] = {};
   if (task < L.tasks) {
     const int seg = (int)(task % L.segments), l0 = (int)(task / L.segments) * L.lines;
     const int j0 = seg * L.width, width = min(L.width, L.m - j0);
@@ -465,7 +466,7 @@ __global__ __launch_bounds__(kLineBS) void k_pcg_lines(int64_t n, LineGrid L, co
     int64_t first = (int64_t)l0 * L.m + j0;  // row of lane 1
     const int last = min(l0 + L.lines, (N + L.m - 1) / L.m);
     struct Line {
-      T z, po;
+      T z, po, r;
       M d[5];
     } next;
     // row of this lane `lines` lines further on, or out of range
@@ -483,7 +484,9 @@ __global__ __launch_bounds__(kLineBS) void k_pcg_lines(int64_t n, LineGrid L, co
       const int64_t r = at(lines);
 #pragma unroll
       for (int d = 0; d < 5; ++d) next.d[d] = M(0);
+      next.r = T(0);
       if (inside(r)) {
+        if constexpr (DOT) next.r = res[r];
 #pragma unroll
         for (int d = 0; d < 5; ++d) next.d[d] = __builtin_nontemporal_load(A + d * n + r);
       }
@@ -530,6 +533,7 @@ __global__ __launch_bounds__(kLineBS) void k_pcg_lines(int64_t n, LineGrid L, co
         pn[row] = pc;
         q[row] = s;
         v[0] += (double)pc * (double)s;
+        if constexpr (DOT) v[DOT] += (double)pc * (double)now.r;
       }
       u2 = from_lane_above((T)now.d[2]);
       u3 = (T)now.d[3];
@@ -542,7 +546,7 @@ __global__ __launch_bounds__(kLineBS) void k_pcg_lines(int64_t n, LineGrid L, co
       pcR = pdR;
     }
   }
-  block_partials_at<kLineBS, 1>(v, partials, block);
+  block_partials_at<kLineBS, DOT ? 2 : 1>(v, partials, block);
 }
 
 __global__ __launch_bounds__(kFinBS) void k_pcg_alpha_fin(KState* S, const double* partials, int nb) {
@@ -704,7 +708,7 @@ static LineGrid line_grid(const Plan& P) {
   L.tasks = (lines + L.lines - 1) / L.lines * L.segments;
   return L;
 }
-static int line_blocks(const Plan& P) {
+int line_blocks(const Plan& P) {
   constexpr int wpb = kLineBS / 64;
   return (int)round_xcd((line_grid(P).tasks + wpb - 1) / wpb);
 }
@@ -716,25 +720,22 @@ static bool lines_pay(const Plan& P, size_t value_bytes) {
   return P.line >= 32 && !noalloc_accepts(P, value_bytes);
 }
 
-// The upper diagonals of the run's matrix into the plan's buffer for them, and the flag that tells
-// whether they are not the whole of it (copied to the host with the stop flags); false: another
-// pattern, or no memory (the run then reads the SELL matrix).
-template <class M, class T>
-bool PcgRun<M, T>::extract_lines() {
-  if (external || !lines_pay(P, sizeof(T))) return false;
+// The upper diagonals of a SELL matrix into the plan's buffer for them, and the flag P.asymmetric that
+// tells whether they are not the whole of it (copied to the host with the first stop flags); null:
+// another pattern, or no memory (the run then reads the SELL matrix).
+template <class M>
+const M* line_matrix(Plan& P, const M* vals, size_t vector_bytes, hipStream_t st) {
+  if (!lines_pay(P, vector_bytes)) return nullptr;
+  const int64_t n = P.n_free;
   const size_t want = (size_t)(5 * n);
-  M* A;
-  auto room = [&](auto& buf) {
-    if (buf.n < want && !buf.try_alloc(want)) return false;
-    A = (M*)buf.p;
-    return true;
-  };
-  bool have;
-  if constexpr (sizeof(M) == 8)
-    have = room(P.lines64);
-  else
-    have = room(P.lines32);
-  if (!have) return false;
+  auto room = [&](auto& buf) { return buf.n >= want || buf.try_alloc(want); };
+  M* A = nullptr;
+  if constexpr (sizeof(M) == 8) {
+    if (room(P.lines64)) A = P.lines64.p;
+  } else {
+    if (room(P.lines32)) A = P.lines32.p;
+  }
+  if (!A) return nullptr;
   if (!P.asymmetric.p) P.asymmetric.alloc(1);
   const int g = (int)std::min<int64_t>((n + kBS - 1) / kBS, 65536);
   auto run = [&](auto cols) {
@@ -749,9 +750,31 @@ bool PcgRun<M, T>::extract_lines() {
   else
     run((const int32_t*)P.sell_cols.p);
   APX_LAUNCH_CHECK();
-  upper = A;
-  return true;
+  return A;
 }
+template const float* line_matrix<float>(Plan&, const float*, size_t, hipStream_t);
+template const double* line_matrix<double>(Plan&, const double*, size_t, hipStream_t);
+
+template <class M, class T>
+void line_product(Plan& P, const M* upper, const M* vals, const T* z, T* pa, T* pb, T* q, const T* r, KState* S,
+                  double* part, hipStream_t st) {
+  auto run = [&](auto cols, auto dot) {
+    using C = std::remove_const_t<std::remove_pointer_t<decltype(cols)>>;
+    launch_kernel(k_pcg_lines<M, T, C, decltype(dot)::value>, dim3(line_blocks(P)), dim3(kLineBS), 0, st, P.n_free,
+                  line_grid(P), upper, P.irregular.p, P.sell_ptr.p, cols, vals, z, pa, pb, q, r, S, part);
+  };
+  auto with = [&](auto cols) { r ? run(cols, std::true_type{}) : run(cols, std::false_type{}); };
+  if (P.sell_dcol.p)
+    with((const int16_t*)P.sell_dcol.p);
+  else
+    with((const int32_t*)P.sell_cols.p);
+}
+template void line_product<double, double>(Plan&, const double*, const double*, const double*, double*, double*,
+                                           double*, const double*, KState*, double*, hipStream_t);
+template void line_product<float, double>(Plan&, const float*, const float*, const double*, double*, double*, double*,
+                                          const double*, KState*, double*, hipStream_t);
+template void line_product<float, float>(Plan&, const float*, const float*, const float*, float*, float*, float*,
+                                         const float*, KState*, double*, hipStream_t);
 
 template <class M, class T>
 void PcgRun<M, T>::launch_iteration() {
@@ -769,15 +792,8 @@ void PcgRun<M, T>::launch_iteration() {
       launch_kernel((k_pcg_spmv<M, T, 4, C>), dim3(gs), dim3(kSpmvBS), 0, st, n, P.n_chunks, P.sell_ptr.p, cols, vals,
                     z, pa, pb, q, S, part);
   };
-  auto by_lines = [&](auto cols) {
-    using C = std::remove_const_t<std::remove_pointer_t<decltype(cols)>>;
-    launch_kernel(k_pcg_lines<M, T, C>, dim3(gs), dim3(kLineBS), 0, st, n, line_grid(P), upper, P.irregular.p,
-                  P.sell_ptr.p, cols, vals, (const T*)z, pa, pb, q, S, part);
-  };
-  if (upper && P.sell_dcol.p)
-    by_lines((const int16_t*)P.sell_dcol.p);
-  else if (upper)
-    by_lines((const int32_t*)P.sell_cols.p);
+  if (upper)
+    line_product<M, T>(P, upper, vals, z, pa, pb, q, nullptr, S, part, st);
   else if (P.sell_dcol.p)
     spmv((const int16_t*)P.sell_dcol.p);
   else
@@ -833,7 +849,8 @@ KState PcgRun<M, T>::run() {
   };
   auto halted_host = [&](int slot) { return flag[4 * slot + 2] != 0 || flag[4 * slot + 3] != 0; };
   // flags after init / reanchor
-  const bool extracted = !upper_known && extract_lines();
+  if (!upper_known && !external) upper = line_matrix<M>(P, vals, sizeof(T), st);
+  const bool extracted = !upper_known && upper;
   if (extracted) APX_HIP(hipMemcpyAsync((void*)(flag + 12), P.asymmetric.p, sizeof(int), hipMemcpyDeviceToHost, st));
   APX_HIP(hipMemcpyAsync((void*)(flag + 8), &S->k, 4 * sizeof(int), hipMemcpyDeviceToHost, st));
   APX_HIP(hipStreamSynchronize(st));

@@ -1326,29 +1326,30 @@ __global__ void k_sq_partials(int64_t n, const T* r, const double* dsq, double* 
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-__global__ void k_scale_fin(const double* part, int nb, const double* rr_src, int64_t n, float* scale, int img,
-                            const int* stop) {
+// root mean square of the network's n inputs from their sum of squares
+__device__ __forceinline__ float input_scale(double sum, int64_t n) {
+  const double rms = sqrt(sum / (double)(n > 0 ? n : 1));
+  return rms > 0.0 ? (float)rms : 1.f;
+}
+__global__ void k_scale_fin(const double* part, int nb, int64_t n, float* scale, int img, const int* stop) {
   __shared__ double lds[4];
   if (stop && *stop) return;
   double s = 0.0;
-  if (rr_src) {
-    s = *rr_src;
-  } else {
-    for (int i = threadIdx.x; i < nb; i += 256) s += part[i];
-    s = block_sum<256>(s, lds);
-  }
-  if (threadIdx.x == 0) {
-    const double rms = sqrt(s / (double)(n > 0 ? n : 1));
-    scale[img] = rms > 0.0 ? (float)rms : 1.f;
-  }
+  for (int i = threadIdx.x; i < nb; i += 256) s += part[i];
+  s = block_sum<256>(s, lds);
+  if (threadIdx.x == 0) scale[img] = input_scale(s, n);
 }
 
 template <class T>
 __global__ void k_to_grid(int64_t n_nodes, int d, int cin, const uint8_t* dmask, const int32_t* full2red, const T* r,
-                          const double* dsq, const double* g, const float* scale, int img, uint16_t* x,
-                          const int* stop) {
-  const float inv = 1.f / scale[img];  // issued together with the stop flag's load
+                          const double* dsq, const double* g, float* scale, int img, uint16_t* x,
+                          const int* stop, const double* rr, int64_t n_red) {
+  // rr given: the scale is formed here, by every block, and kept for the network's output by one
+  // (k_scale_fin is a launch more); its loads are issued together with the stop flag's
+  const float s = rr ? input_scale(*rr, n_red) : scale[img];
   if (stop && *stop) return;
+  const float inv = 1.f / s;
+  if (rr && blockIdx.x == 0 && threadIdx.x == 0) scale[img] = s;
   for (int64_t node = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; node < n_nodes;
        node += (int64_t)gridDim.x * blockDim.x) {
     uint16_t* xo = x + ((int64_t)img * n_nodes + node) * cin;
@@ -1422,17 +1423,16 @@ void net_input_from_reduced_img(Plan& P, UNet& N, const void* r, int r_f64, cons
     else
       hipLaunchKernelGGL(k_sq_partials<float>, dim3(nb), dim3(256), 0, st, P.n_free, (const float*)r, dsq,
                          P.partials.p, N.stop);
+    hipLaunchKernelGGL(k_scale_fin, dim3(1), dim3(256), 0, st, P.partials.p, nb, P.n_free, N.scale.p, img, N.stop);
   }
-  hipLaunchKernelGGL(k_scale_fin, dim3(1), dim3(256), 0, st, P.partials.p, nb, rr_src, P.n_free, N.scale.p, img,
-                     N.stop);
   int g;
   grid1d(P.n_nodes, g);
   if (r_f64)
     hipLaunchKernelGGL(k_to_grid<double>, dim3(g), dim3(256), 0, st, P.n_nodes, P.d, N.c_in, P.dmask.p, P.full2red.p,
-                       (const double*)r, dsq, g_nodal, N.scale.p, img, N.x0.p, N.stop);
+                       (const double*)r, dsq, g_nodal, N.scale.p, img, N.x0.p, N.stop, rr_src, P.n_free);
   else
     hipLaunchKernelGGL(k_to_grid<float>, dim3(g), dim3(256), 0, st, P.n_nodes, P.d, N.c_in, P.dmask.p, P.full2red.p,
-                       (const float*)r, dsq, g_nodal, N.scale.p, img, N.x0.p, N.stop);
+                       (const float*)r, dsq, g_nodal, N.scale.p, img, N.x0.p, N.stop, rr_src, P.n_free);
   APX_LAUNCH_CHECK();
 }
 

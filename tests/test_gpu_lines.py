@@ -98,3 +98,33 @@ def test_newton_by_lines(torch_gpu, precision):
     assert not infos[2]
     r = OA.residual(o["sets"], o["coords"], np.asarray(sol).ravel(), 1)
     assert np.linalg.norm(r[~o["mask"]]) <= 1.1e-9
+
+
+# A network of zero weights with its Jacobi part is the preconditioner D^-1, and flexible CG with it the
+# iterations of _reference; tolerance as above times five for its own recurrence of beta.
+@pytest.mark.parametrize("kind,size,precision", [("side", (521, 530), "fp64"), ("corners", (600, 470), "fp64"),
+                                                 ("corners", (520, 533), "fp32"), ("side", (8500, 31), "fp32")])
+def test_flexible_cg_by_lines(torch_gpu, kind, size, precision):
+    torch = torch_gpu
+    import scipy.sparse as sp
+    from autopdex_amd import learned
+    prob = _problem(kind, size)
+    print(f"[case] flexible cg by lines {kind} {size} {precision}: {prob.n_free} rows", flush=True)
+    net = learned.UNetPreconditioner(size[0] + 1, size[1] + 1, 2, (16, 16), 1, 1, relu=False, batch=1, jacobi_skip=True)
+    net.set_params(np.zeros(net.n_params))
+    net.attach(prob)
+    dt = torch.float64 if precision == "fp64" else torch.float32
+    vals = learned.tangent(prob).to(dt)
+    indptr, indices = prob.csr_pattern()
+    rng = np.random.default_rng(prob.n_free)
+    b = torch.from_numpy(rng.standard_normal(prob.n_free)).cuda()
+    rows = np.repeat(np.arange(prob.n_free), np.diff(indptr))
+    skew = vals.clone()
+    below = np.flatnonzero(np.asarray(indices) < rows)
+    skew[torch.from_numpy(rng.choice(below, 50)).cuda()] *= 1 + 1e-12 if precision == "fp64" else 1 + 1e-6
+    for v in (vals, skew):
+        x, ks = learned.fcg(prob, v, b, tol=0.0, maxiter=7, precision=precision)
+        A = sp.csr_matrix((v.double().cpu().numpy(), indices, indptr), shape=(prob.n_free,) * 2)
+        ref = _reference(A, b.cpu().numpy(), 7)
+        assert ks.iterations == 7
+        assert np.abs(x.cpu().numpy() - ref).max() <= 25 * 3.7e-14 * np.abs(ref).max() + 1e-5 * (v is skew and precision == "fp32")
