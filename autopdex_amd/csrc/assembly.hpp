@@ -78,11 +78,11 @@ bool pcg_resident(Plan& P, const M* vals, const V* inv, V* x, const V* r, const 
 // applicable.  vector_bytes: of an entry of the vectors.
 template <class M>
 const M* line_matrix(Plan& P, const M* vals, size_t vector_bytes, hipStream_t st);
-// p_new = z + beta p_old, q = A p_new, block partials of p.q and (r given) p.r; exits at once when S
-// has a stop flag
+// p_new = z + beta p_old, q = A p_new, block partials of p.q; r given: also of p.r; else x += alpha p_old
+// from the second iteration after k0 on.  Exits at once when S has a stop flag.
 template <class M, class T>
-void line_product(Plan& P, const M* upper, const M* vals, const T* z, T* pa, T* pb, T* q, const T* r, KState* S,
-                  double* part, hipStream_t st);
+void line_product(Plan& P, const M* upper, const M* vals, const T* z, T* pa, T* pb, T* q, const T* r, T* x, int k0,
+                  KState* S, double* part, hipStream_t st);
 int line_blocks(const Plan& P);  // its workgroups
 
 // One preconditioned-CG solve on the plan's SELL matrix with values of type M
@@ -110,6 +110,7 @@ struct PcgRun {
   // streaming run on it
   const M* upper = nullptr;
   bool upper_known = false;
+  int k0 = 0;  // iterations before the present streaming run
   int start_k = 0;         // iterations before the present resident run
   int maxiter = 0, iterations = 0;
   int64_t launched = 0;

@@ -263,7 +263,7 @@ FcgResult fcg_solve(Plan& P, UNet& N, const T* vals, const double* g_nodal, cons
     t_launch_events = P.timing ? &e1 : nullptr;
     const int gp = upper ? line_blocks(P) : gs;
     if (upper)
-      line_product<T, double>(P, upper, vals, z, pa, pb, q, r, S, P.partials.p, st);
+      line_product<T, double>(P, upper, vals, z, pa, pb, q, r, nullptr, 0, S, P.partials.p, st);
     else if (P.sell_dcol.p)
       launch_kernel(k_fcg_spmv<T, int16_t>, dim3(gs), dim3(kSpmvBS), 0, st, n, P.n_chunks, P.sell_ptr.p,
                     (const int16_t*)P.sell_dcol.p, vals, z, pa, pb, q, r, S, P.partials.p);

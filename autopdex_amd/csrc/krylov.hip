@@ -356,7 +356,8 @@ __global__ __launch_bounds__(kSpmvBS) void k_pcg_spmv(int64_t n, int64_t n_chunk
 // (non-temporal), which leaves them to the vectors: the update kernel after it 43.9 -> 41.4 us.
 //
 // Bound by HBM: at 2047^2 rows, FP64, 302 MB in 56.5 us (5.3 TB/s) against 512 MB in 109 us for
-// k_pcg_spmv; the iteration 157 -> 114 us.  The same diagonals read without the walk (27 loads a
+// k_pcg_spmv; with x's update 369 MB in 64.5 us (5.7 TB/s) and the update kernel 41.4 -> 26.1 us; the
+// iteration 157 -> 104 us.  The same diagonals read without the walk (27 loads a
 // row, neighbours' lines from L2) took 89 us.  Which rows form a line is arithmetic
 // only: entries that a grid's end takes out of the pattern are stored zeros.  Rows of the chunks
 // with entries elsewhere (Plan::irregular) are summed from the SELL values.
@@ -441,17 +442,20 @@ __global__ __launch_bounds__(kBS) void k_lines_check(int64_t n, int m, const int
   if (differs) *asymmetric = 1;
 }
 
-// DOT: flexible CG, which wants p.r (second partial) beside p.q
+// DOT: flexible CG, which wants p.r (second partial) beside p.q.  Else the last iteration's x += alpha p
+// is made up for here (where there was one since iteration k0), whose p is at hand: the update kernel
+// then reads neither x nor p, 8 of an iteration's 136 bytes a row less in FP64.
 template <class M, class T, class C, bool DOT>
 __global__ __launch_bounds__(kLineBS) void k_pcg_lines(int64_t n, LineGrid L, const M* __restrict__ A,
                                                        const uint32_t* __restrict__ irregular,
                                                        const int32_t* __restrict__ sptr, const C* __restrict__ cols,
                                                        const M* __restrict__ vals, const T* __restrict__ z,
                                                        T* __restrict__ pa, T* __restrict__ pb, T* __restrict__ q,
-                                                       const T* __restrict__ res, KState* S, double* partials) {
+                                                       const T* __restrict__ res, T* __restrict__ x, int k0, KState* S,
+                                                       double* partials) {
   if (halted(S)) return;
-  const T beta = (T)S->beta;
-  const bool odd = S->k & 1;
+  const T beta = (T)S->beta, alpha = (T)S->alpha;
+  const bool odd = S->k & 1, behind = !DOT && S->k > k0;
   const T* __restrict__ po = odd ? pb : pa;
   T* __restrict__ pn = odd ? pa : pb;
   const int lane = threadIdx.x & 63, N = (int)n;
@@ -466,7 +470,7 @@ __global__ __launch_bounds__(kLineBS) void k_pcg_lines(int64_t n, LineGrid L, co
     int64_t first = (int64_t)l0 * L.m + j0;  // row of lane 1
     const int last = min(l0 + L.lines, (N + L.m - 1) / L.m);
     struct Line {
-      T z, po, r;
+      T z, po, r, x;
       M d[5];
     } next;
     // row of this lane `lines` lines further on, or out of range
@@ -484,9 +488,12 @@ __global__ __launch_bounds__(kLineBS) void k_pcg_lines(int64_t n, LineGrid L, co
       const int64_t r = at(lines);
 #pragma unroll
       for (int d = 0; d < 5; ++d) next.d[d] = M(0);
-      next.r = T(0);
+      next.r = next.x = T(0);
       if (inside(r)) {
-        if constexpr (DOT) next.r = res[r];
+        if constexpr (DOT)
+          next.r = res[r];
+        else if (behind)
+          next.x = x[r];
 #pragma unroll
         for (int d = 0; d < 5; ++d) next.d[d] = __builtin_nontemporal_load(A + d * n + r);
       }
@@ -494,7 +501,7 @@ __global__ __launch_bounds__(kLineBS) void k_pcg_lines(int64_t n, LineGrid L, co
     load_p(-1);
     T pm = next.z + beta * next.po;
     load_p(0);
-    T pc = next.z + beta * next.po;
+    T pc = next.z + beta * next.po, poc = next.po;
     load_d(-1);
     T u2 = from_lane_above((T)next.d[2]), u3 = (T)next.d[3], u4 = from_lane_below((T)next.d[4]);
     load_p(1);
@@ -533,8 +540,12 @@ __global__ __launch_bounds__(kLineBS) void k_pcg_lines(int64_t n, LineGrid L, co
         pn[row] = pc;
         q[row] = s;
         v[0] += (double)pc * (double)s;
-        if constexpr (DOT) v[DOT] += (double)pc * (double)now.r;
+        if constexpr (DOT)
+          v[DOT] += (double)pc * (double)now.r;
+        else if (behind)
+          x[row] = now.x + alpha * poc;
       }
+      poc = now.po;
       u2 = from_lane_above((T)now.d[2]);
       u3 = (T)now.d[3];
       u4 = from_lane_below((T)now.d[4]);
@@ -559,7 +570,8 @@ __global__ __launch_bounds__(kFinBS) void k_pcg_alpha_fin(KState* S, const doubl
   }
 }
 
-template <class T>
+// WITH_X: or the next k_pcg_lines (after the last iteration k_pcg_finish_x) adds alpha p to x.
+template <class T, bool WITH_X>
 __global__ __launch_bounds__(kBS) void k_pcg_update(int64_t n, const T* __restrict__ inv, const T* __restrict__ pa,
                                                     const T* __restrict__ pb, const T* __restrict__ q,
                                                     T* __restrict__ x, T* __restrict__ r, T* __restrict__ z,
@@ -570,13 +582,15 @@ __global__ __launch_bounds__(kBS) void k_pcg_update(int64_t n, const T* __restri
   double v[2] = {0.0, 0.0};
   T pv[kUnroll], qv[kUnroll], xv[kUnroll], rv[kUnroll], iv[kUnroll];
   APX_FOR_ELEMENTS(n, {
-    pv[j] = p[i];
+    if constexpr (WITH_X) {
+      pv[j] = p[i];
+      xv[j] = x[i];
+    }
     qv[j] = q[i];
-    xv[j] = x[i];
     rv[j] = r[i];
     iv[j] = inv[i];
   }, {
-    x[i] = xv[j] + alpha * pv[j];
+    if constexpr (WITH_X) x[i] = xv[j] + alpha * pv[j];
     const T ri = rv[j] - alpha * qv[j];
     const T zi = iv[j] * ri;
     r[i] = ri;
@@ -600,6 +614,15 @@ __global__ __launch_bounds__(kFinBS) void k_pcg_beta_fin(KState* S, const double
     S->done = !(s[1] > S->atol2 && S->k < S->maxiter);
     if (!S->done && S->delta2 > 0.0 && s[1] < S->delta2 * S->rmax2) S->reliable = 1;
   }
+}
+
+template <class T>
+__global__ __launch_bounds__(kBS) void k_pcg_finish_x(int64_t n, const T* __restrict__ pa, const T* __restrict__ pb,
+                                                      T* __restrict__ x, const KState* S) {
+  const T alpha = (T)S->alpha;
+  const T* __restrict__ p = ((S->k - 1) & 1) ? pa : pb;  // of the last iteration
+  T pv[kUnroll], xv[kUnroll];
+  APX_FOR_ELEMENTS(n, { pv[j] = p[i]; xv[j] = x[i]; }, { x[i] = xv[j] + alpha * pv[j]; })
 }
 
 // Replace the recursive residual by b_new = -r_full[free] (a true residual
@@ -756,12 +779,12 @@ template const float* line_matrix<float>(Plan&, const float*, size_t, hipStream_
 template const double* line_matrix<double>(Plan&, const double*, size_t, hipStream_t);
 
 template <class M, class T>
-void line_product(Plan& P, const M* upper, const M* vals, const T* z, T* pa, T* pb, T* q, const T* r, KState* S,
-                  double* part, hipStream_t st) {
+void line_product(Plan& P, const M* upper, const M* vals, const T* z, T* pa, T* pb, T* q, const T* r, T* x, int k0,
+                  KState* S, double* part, hipStream_t st) {
   auto run = [&](auto cols, auto dot) {
     using C = std::remove_const_t<std::remove_pointer_t<decltype(cols)>>;
     launch_kernel(k_pcg_lines<M, T, C, decltype(dot)::value>, dim3(line_blocks(P)), dim3(kLineBS), 0, st, P.n_free,
-                  line_grid(P), upper, P.irregular.p, P.sell_ptr.p, cols, vals, z, pa, pb, q, r, S, part);
+                  line_grid(P), upper, P.irregular.p, P.sell_ptr.p, cols, vals, z, pa, pb, q, r, x, k0, S, part);
   };
   auto with = [&](auto cols) { r ? run(cols, std::true_type{}) : run(cols, std::false_type{}); };
   if (P.sell_dcol.p)
@@ -770,11 +793,11 @@ void line_product(Plan& P, const M* upper, const M* vals, const T* z, T* pa, T* 
     with((const int32_t*)P.sell_cols.p);
 }
 template void line_product<double, double>(Plan&, const double*, const double*, const double*, double*, double*,
-                                           double*, const double*, KState*, double*, hipStream_t);
+                                           double*, const double*, double*, int, KState*, double*, hipStream_t);
 template void line_product<float, double>(Plan&, const float*, const float*, const double*, double*, double*, double*,
-                                          const double*, KState*, double*, hipStream_t);
+                                          const double*, double*, int, KState*, double*, hipStream_t);
 template void line_product<float, float>(Plan&, const float*, const float*, const float*, float*, float*, float*,
-                                         const float*, KState*, double*, hipStream_t);
+                                         const float*, float*, int, KState*, double*, hipStream_t);
 
 template <class M, class T>
 void PcgRun<M, T>::launch_iteration() {
@@ -793,14 +816,17 @@ void PcgRun<M, T>::launch_iteration() {
                     z, pa, pb, q, S, part);
   };
   if (upper)
-    line_product<M, T>(P, upper, vals, z, pa, pb, q, nullptr, S, part, st);
+    line_product<M, T>(P, upper, vals, z, pa, pb, q, nullptr, x, k0, S, part, st);
   else if (P.sell_dcol.p)
     spmv((const int16_t*)P.sell_dcol.p);
   else
     spmv((const int32_t*)P.sell_cols.p);
   hipLaunchKernelGGL(k_pcg_alpha_fin, dim3(1), dim3(kFinBS), 0, st, S, part, gs);
   t_launch_events = timed ? &e2 : nullptr;
-  launch_kernel(k_pcg_update<T>, dim3(gu), dim3(kBS), 0, st, n, inv, pa, pb, q, x, r, z, S, part);
+  if (upper)
+    launch_kernel(k_pcg_update<T, false>, dim3(gu), dim3(kBS), 0, st, n, inv, pa, pb, q, x, r, z, S, part);
+  else
+    launch_kernel(k_pcg_update<T, true>, dim3(gu), dim3(kBS), 0, st, n, inv, pa, pb, q, x, r, z, S, part);
   hipLaunchKernelGGL(k_pcg_beta_fin, dim3(1), dim3(kFinBS), 0, st, S, part, gu);
   if (timed) {
     ev_spmv.push_back(e1);
@@ -856,6 +882,7 @@ KState PcgRun<M, T>::run() {
   APX_HIP(hipStreamSynchronize(st));
   if (extracted && flag[12]) upper = nullptr;
   upper_known = true;
+  k0 = flag[8];
   if (external && !halted_host(2)) {
     // no events: enqueue a batch, copy the flags, wait for the stream, test
     const int64_t limit = (int64_t)launched + maxiter + kBatch;
@@ -888,6 +915,11 @@ KState PcgRun<M, T>::run() {
   } else {
     APX_HIP(hipStreamSynchronize(st));
     APX_HIP(hipMemcpy(&hs, S, sizeof(KState), hipMemcpyDeviceToHost));
+    if (upper && hs.k > k0) {
+      hipLaunchKernelGGL(k_pcg_finish_x<T>, dim3(grid_for(n)), dim3(kBS), 0, st, n, pa, pb, x, S);
+      APX_LAUNCH_CHECK();
+      APX_HIP(hipStreamSynchronize(st));  // x is complete on return, on whatever stream it is read
+    }
   }
   iterations = hs.k;
   return hs;
@@ -907,11 +939,11 @@ void PcgRun<M, T>::collect_timing() {
   const bool f64 = sizeof(T) == 8;
   // only launches that executed an iteration are counted; the rest exited at entry
   const size_t k = (size_t)iterations - counted;
-  // by lines: the upper values; z and p_old read, p_new and q written
-  const int64_t line_bytes = n * (5 * (int64_t)sizeof(M) + 4 * (int64_t)sizeof(T));
+  // by lines: the upper values; z, p_old and x read, p_new, q and x written; D^-1, q, r read, r, z written
+  const int64_t line_bytes = n * (5 * (int64_t)sizeof(M) + 6 * (int64_t)sizeof(T));
   timing_collect(P, sizeof(M) == sizeof(T) ? (f64 ? "pcg_spmv_f64" : "pcg_spmv_f32") : "pcg_spmv_f32m_f64v", ev_spmv,
                  upper ? line_bytes : spmv_bytes, k);
-  timing_collect(P, f64 ? "pcg_update_f64" : "pcg_update_f32", ev_upd, upd_bytes, k);
+  timing_collect(P, f64 ? "pcg_update_f64" : "pcg_update_f32", ev_upd, upper ? n * 5 * (int64_t)sizeof(T) : upd_bytes, k);
   timing_collect(P, f64 ? "pcg_resident_f64" : "pcg_resident_f32", ev_res, 0, ev_res.size());
   counted = iterations;
 }
