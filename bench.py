@@ -70,9 +70,8 @@ HBM_PEAK = 8.0e12
 # reading of a 512 MiB device copy (FETCH_SIZE x2.000, WRITE_SIZE x1.000).
 # The convolution's figure is the average over the launches of one network application (two at
 # 513 x 513, four at 257 x 257), the mix its timer averages over.
-PMC_TRAFFIC_BYTES = {("k_pcg_spmv<double, double, 4, short>", 2048): 584.8e6,
-                     ("k_pcg_spmv<float, double, 4, short>", 2048): 434.1e6,
-                     ("k_pcg_spmv<float, float, 4, short>", 2048): 333.1e6, ("k_fcg_spmv<float, short>", 2048): 467.7e6,
+PMC_TRAFFIC_BYTES = {("k_pcg_lines<double, double, short, false>", 2048): 413.5e6,
+                     ("k_pcg_lines<float, double, short, true>", 2048): 287.3e6,
                      ("k_conv3x3<64, 64, false, 4, 2, false>", 2048): 37.33e6,
                      ("k_conv3x3_ws<16, 16, 4, 0>", 2048): 292.1e6}
 
@@ -158,12 +157,14 @@ def all_timers(prob):
 
 
 # single-kernel solver timers and the kernel each one times (rocprofv3 names)
-# (the SpMVs of the 2048^2 grid read int16 column offsets: template argument "short")
-SOLVER_KERNELS = {"fcg_spmv_f32": "k_fcg_spmv<float, short>", "fcg_spmv_f64": "k_fcg_spmv<double, short>",
-                  "pcg_spmv_f64": "k_pcg_spmv<double, double, 4, short>",
-                  "pcg_spmv_f32": "k_pcg_spmv<float, float, 4, short>",
-                  "pcg_spmv_f32m_f64v": "k_pcg_spmv<float, double, 4, short>", "pcg_update_f64": "k_pcg_update<double>",
-                  "pcg_update_f32": "k_pcg_update<float>"}
+# (the products of the 2048^2 grid walk its lines over the upper diagonals; the chunks beside them
+# read int16 column offsets: template argument "short")
+SOLVER_KERNELS = {"fcg_spmv_f32": "k_pcg_lines<float, double, short, true>",
+                  "fcg_spmv_f64": "k_pcg_lines<double, double, short, true>",
+                  "pcg_spmv_f64": "k_pcg_lines<double, double, short, false>",
+                  "pcg_spmv_f32": "k_pcg_lines<float, float, short, false>",
+                  "pcg_spmv_f32m_f64v": "k_pcg_lines<float, double, short, false>",
+                  "pcg_update_f64": "k_pcg_update<double, false>", "pcg_update_f32": "k_pcg_update<float, false>"}
 
 
 def dominant_kernel(timers):
