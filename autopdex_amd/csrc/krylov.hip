@@ -736,7 +736,9 @@ int line_blocks(const Plan& P) {
   return (int)round_xcd((line_grid(P).tasks + wpb - 1) / wpb);
 }
 
-// Lines of fewer than 32 rows would leave more than half of a wavefront's lanes idle.  Systems that
+// Lines of fewer than 32 rows would leave more than half of a wavefront's lanes idle, where it no longer
+// pays (FP64, us an iteration: 557,973 rows in lines of 31, SELL kernel 35.1; 575,972 in lines of 32
+// 34.8, of 64 31.5; 571,377 in lines of 127 29.6).  Systems that
 // apx_pcg_noalloc takes keep the SELL kernel, whose sums it shares bit by bit (and where the launches'
 // latency, not the bytes, sets the pace).
 static bool lines_pay(const Plan& P, size_t value_bytes) {
