@@ -1,5 +1,5 @@
-// Element-loop assembly kernels: residual and tangent diagonal by colours, the tangent's element
-// matrices, and the dispatch between these, the owner tiles and the row-owner kernels.
+// Element-loop assembly kernels: the tangent's diagonal by colours and its element matrices in the
+// reference's BCOO order, and the dispatch between these, the owner tiles and the row-owner kernels.
 //
 // Replaces jacrev / jacfwd(jacrev) of the element potential under lax.map and
 // the .at[].add scatter (assembler.py:1064-1149, :219-436).
@@ -13,7 +13,7 @@
 
 namespace apx {
 
-enum { MODE_RES = 0, MODE_DIAG = 2, MODE_COO = 3 };
+enum { MODE_DIAG = 2, MODE_COO = 3 };
 
 struct AsmArgs {
   const double* coords;  // SoA, dim x n_nodes
@@ -22,7 +22,7 @@ struct AsmArgs {
   int64_t e0, e1;        // element range of one colour
   const double* u;       // n_dofs
   ModelParams mp;
-  double* r;             // residual or diagonal output (n_dofs)
+  double* r;             // diagonal output (n_dofs)
   void* vals;            // element matrices (BCOO)
 };
 
@@ -52,29 +52,22 @@ __global__ __launch_bounds__(BS) void k_team(AsmArgs A) {
     }
   }
   __syncthreads();
-  if (active) M::template qp<T>(t, sx[le], su[le], sn[le], A.mp, MODE == MODE_RES, sq[le][t]);
+  if (active) M::template qp<T>(t, sx[le], su[le], sn[le], A.mp, false, sq[le][t]);
   __syncthreads();
   if (!active) return;
 
-  if constexpr (MODE == MODE_RES) {
-    double out[D];
-    M::res_row(t, (const typename M::template QP<double>*)sq[le], A.mp, out);
+  T out[D][ND];
+  M::template tan_rows<T>(t, sq[le], A.mp, out);
+  if constexpr (MODE == MODE_DIAG) {
 #pragma unroll
-    for (int i = 0; i < D; ++i) A.r[(int64_t)node * D + i] += out[i];
-  } else {
-    T out[D][ND];
-    M::template tan_rows<T>(t, sq[le], A.mp, out);
-    if constexpr (MODE == MODE_DIAG) {
+    for (int i = 0; i < D; ++i) A.r[(int64_t)node * D + i] += (double)out[i][t * D + i];
+  } else if constexpr (MODE == MODE_COO) {
+    // element-major, row-major block (the reference's BCOO order); every entry written once
+    T* data = (T*)A.vals + ((int64_t)e * ND + (int64_t)t * D) * ND;
 #pragma unroll
-      for (int i = 0; i < D; ++i) A.r[(int64_t)node * D + i] += (double)out[i][t * D + i];
-    } else if constexpr (MODE == MODE_COO) {
-      // element-major, row-major block (the reference's BCOO order); every entry written once
-      T* data = (T*)A.vals + ((int64_t)e * ND + (int64_t)t * D) * ND;
+    for (int i = 0; i < D; ++i)
 #pragma unroll
-      for (int i = 0; i < D; ++i)
-#pragma unroll
-        for (int B = 0; B < ND; ++B) data[i * ND + B] = out[i][B];
-    }
+      for (int B = 0; B < ND; ++B) data[i * ND + B] = out[i][B];
   }
 }
 
@@ -147,6 +140,11 @@ static void run_set(Plan& P, ElemSet& S, const double* u, double* r, void* vals,
   }
 }
 
+[[noreturn]] static void no_kernel(const Plan& P, const ElemSet& S) {
+  throw Error(APX_ERR_UNSUPPORTED, "no kernel for model " + std::to_string(S.model) + " with " +
+                                       std::to_string(S.npe) + "-node elements in " + std::to_string(P.dim) + "D");
+}
+
 template <class T, int MODE>
 static void dispatch(Plan& P, ElemSet& S, const double* u, double* r, void* vals, hipStream_t st) {
   const int key = S.model * 100 + S.npe * 10 + P.dim;
@@ -179,9 +177,7 @@ static void dispatch(Plan& P, ElemSet& S, const double* u, double* r, void* vals
       APX_REQUIRE(P.d == 2, APX_ERR_ARG, "line traction needs 2 DOFs per node");
       return run_set<LineTraction3, T, MODE>(P, S, u, r, vals, st);
     default:
-      throw Error(APX_ERR_UNSUPPORTED, "no kernel for model " + std::to_string(S.model) + " with " +
-                                           std::to_string(S.npe) + "-node elements in " +
-                                           std::to_string(P.dim) + "D");
+      no_kernel(P, S);
   }
 }
 
@@ -236,8 +232,9 @@ void assemble_residual(Plan& P, const double* u, double* r, hipStream_t st) {
     if (tile_supported(P, S, 0)) {
       tile_residual(P, S, u, r, !have, st);
     } else if (!gather_residual(P, S, u, r, !have, st)) {
-      if (!have) fill<double>(r, P.n_dofs, 0.0, st);
-      dispatch<double, MODE_RES>(P, S, u, r, nullptr, st);
+      APX_REQUIRE(S.model != APX_MODEL_LINE_TRACTION || P.dim != 2 || (S.npe != 2 && S.npe != 3), APX_ERR_ARG,
+                  "line traction needs 2 DOFs per node");
+      no_kernel(P, S);
     }
     have = true;
   }

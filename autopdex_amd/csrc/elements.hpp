@@ -189,21 +189,6 @@ struct PoissonSource {
       o.srcN = (T)(p.p[0] * (sin(p.p[1] * xx) - cos(p.p[1] * yy)));
     }
   }
-  __device__ static double nshape(int q, int a) {
-    double N[NPE], dN[NPE][DIM];
-    Shape<NPE, DIM>::eval(q, N, dN);
-    return N[a];
-  }
-  __device__ static void res_row(int a, const QP<double>* Q, const ModelParams&, double out[1]) {
-    double s = 0.0;
-    for (int q = 0; q < NQ; ++q) {
-      double gg = 0.0;
-#pragma unroll
-      for (int k = 0; k < DIM; ++k) gg += Q[q].G[a][k] * Q[q].grad[k];
-      s += Q[q].wdet * (gg - Q[q].srcN * nshape(q, a));
-    }
-    out[0] = s;
-  }
   template <class T>
   __device__ static void tan_rows(int a, const QP<T>* Q, const ModelParams&, T out[1][NPE]) {
 #pragma unroll
@@ -276,18 +261,6 @@ struct PoissonVarK {
       }
       o.grad[k] = (T)s;
     }
-  }
-  __device__ static void res_row(int a, const QP<double>* Q, const ModelParams&, double out[1]) {
-    double s = 0.0;
-    for (int q = 0; q < NQ; ++q) {
-      double N[NPE], dN[NPE][DIM];
-      Shape<NPE, DIM>::eval(q, N, dN);
-      double gg = 0.0;
-#pragma unroll
-      for (int k = 0; k < DIM; ++k) gg += Q[q].G[a][k] * Q[q].grad[k];
-      s += Q[q].wdet * (Q[q].kq * gg - Q[q].fq * N[a]);
-    }
-    out[0] = s;
   }
   template <class T>
   __device__ static void tan_rows(int a, const QP<T>* Q, const ModelParams&, T out[1][NPE]) {
@@ -406,14 +379,6 @@ struct NeoHooke {
     for (int a = 0; a < NPE; ++a)
 #pragma unroll
       for (int i = 0; i < DIM; ++i) out[a][i] += Q.wdet * (Q.FG[a][i] - Q.c1 * Q.H[a][i]);
-  }
-  // r_ai = sum_q w det (mu (F G_a)_i - c1 H_ai)
-  __device__ static void res_row(int a, const QP<double>* Q, const ModelParams&, double out[DIM]) {
-#pragma unroll
-    for (int i = 0; i < DIM; ++i) out[i] = 0.0;
-    for (int q = 0; q < NQ; ++q)
-#pragma unroll
-      for (int i = 0; i < DIM; ++i) out[i] += Q[q].wdet * (Q[q].FG[a][i] - Q[q].c1 * Q[q].H[a][i]);
   }
   template <class T>
   __device__ static void tan_rows(int a, const QP<T>* Q, const ModelParams& p, T out[DIM][NPE * DIM]) {

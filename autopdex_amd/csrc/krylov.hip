@@ -13,6 +13,8 @@
 //   k_pcg_update: x += alpha p, r -= alpha q, z = D^-1 r, partials of r.z and
 //                 r.r;  k_pcg_beta_fin forms beta, gamma, the stop flag and
 //                 the reliable-update request.
+// On symmetric 9-point matrices k_pcg_lines stands in for k_pcg_spmv and also updates x (below); systems
+// that fit on the compute units run all iterations in one launch (resident.hip).
 // Scalars live on the device.  Kernels exit at entry once a flag is set, so
 // the host enqueues iterations in batches and reads the flags one batch late.
 // The two direction buffers alternate by the device iteration counter.
