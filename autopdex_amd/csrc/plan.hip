@@ -14,6 +14,7 @@
 namespace apx {
 
 Plan::~Plan() {
+  if (scratch_done) (void)hipEventDestroy(scratch_done);
   if (pinned) (void)hipHostFree(pinned);
   if (ev0) (void)hipEventDestroy(ev0);
   if (ev1) (void)hipEventDestroy(ev1);
@@ -440,11 +441,15 @@ void plan_finalize(Plan& P) {
   if (P.line) P.irregular.upload(P.irregular_h.data(), P.irregular_h.size());
   std::vector<int32_t>().swap(P.sell_cols_h);
   std::vector<int32_t>().swap(P.csr2sell_h);
+  size_t words = 0;  // of element vectors
   for (size_t si = 0; si < P.sets.size(); ++si) {
     ElemSet& S = P.sets[si];
     S.conn.upload(conn_perm[si].data(), conn_perm[si].size());
+    const bool vectors = !S.inc_ptr_h.empty() && !tile_supported(P, S, 0) && S.model != APX_MODEL_LINE_TRACTION;
+    if (vectors) words = std::max(words, (size_t)(S.n_elems * S.npe * P.d));
     upload_rows(P, S);
   }
+  if (words) P.element_vectors.alloc(words);
   // pinned host scalars: [0, 512) B PCG flags and norms, [512, 768) B FCG state copies,
   // [768, 1024) B the final Krylov state of an allocation-free PCG run
   if (!P.pinned) APX_HIP(hipHostMalloc((void**)&P.pinned, 128 * sizeof(double), hipHostMallocDefault));

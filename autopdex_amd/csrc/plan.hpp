@@ -62,8 +62,12 @@ struct Plan {
   int dim = 0, d = 0;
   int64_t n_nodes = 0, n_dofs = 0, n_free = 0, nnz = 0;
   bool finalized = false;
-  // scratch of the row-owner kernels
+  // Scratch of the row-owner kernels, and the last work on it: a call on another stream waits for
+  // that on the device (rows.hip, ScratchUse).
   DevBuf<double> element_vectors, element_matrices;
+  hipEvent_t scratch_done = nullptr;
+  hipStream_t scratch_stream = nullptr;
+  bool scratch_used = false;
   double build_seconds = 0.0;
 
   std::vector<double> coords_host;   // n_nodes * dim row-major

@@ -649,6 +649,28 @@ __global__ void k_line_vectors(int64_t n_list, const int32_t* __restrict__ list,
   r[node * 2 + 1] += s[1];
 }
 
+// The plan's scratch is one: work on it from another stream than the last waits for that work.  (Under
+// capture neither is recorded: what a graph's replays overlap with is the caller's to order.)
+struct ScratchUse {
+  Plan& P;
+  hipStream_t st;
+  bool capturing = false;
+  ScratchUse(Plan& p, hipStream_t s) : P(p), st(s) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &status) != hipSuccess) (void)hipGetLastError();
+    capturing = status != hipStreamCaptureStatusNone;
+    if (capturing) return;
+    if (!P.scratch_done) APX_HIP(hipEventCreateWithFlags(&P.scratch_done, hipEventDisableTiming));
+    if (P.scratch_used && P.scratch_stream != st) APX_HIP(hipStreamWaitEvent(st, P.scratch_done, 0));
+  }
+  ~ScratchUse() {
+    if (capturing) return;
+    (void)hipEventRecord(P.scratch_done, st);
+    P.scratch_stream = st;
+    P.scratch_used = true;
+  }
+};
+
 template <class M, class T, class TO, bool CSR>
 void run_rows(Plan& P, ElemSet& S, const double* u, void* vals, bool accumulate, hipStream_t st) {
   if constexpr (M::NODAL) {
@@ -658,6 +680,7 @@ void run_rows(Plan& P, ElemSet& S, const double* u, void* vals, bool accumulate,
   constexpr int EPB = elements_per_block<M>(), NPW = 64 / M::NPE;
   const size_t words = ((size_t)S.n_elems * M::NPE * kBlocks<M::NPE> * M::D * M::D * sizeof(T) + 7) / 8;
   if (P.element_matrices.n < words) P.element_matrices.alloc(words);
+  ScratchUse use(P, st);
   hipLaunchKernelGGL((k_element_matrices<M, T>), dim3((unsigned)((S.n_elems + EPB - 1) / EPB)), dim3(EPB * M::NPE), 0, st,
                      S.conn_orig.p, S.n_elems, P.coords.p, P.n_nodes, u, S.params, (T*)P.element_matrices.p);
   RowArgs A;
@@ -771,8 +794,8 @@ bool gather_residual(Plan& P, ElemSet& S, const double* u, double* r, bool overw
       APX_REQUIRE(S.params.nodal[0] && S.params.nodal[1], APX_ERR_STATE,
                   "variable-coefficient Poisson set needs nodal fields g and f bound");
     }
-    const size_t words = (size_t)S.n_elems * M::NPE * M::D;
-    if (P.element_vectors.n < words) P.element_vectors.alloc(words);
+    // (element_vectors: allocated with the plan)
+    ScratchUse use(P, st);
     if (overwrite && !S.touched_all) fill<double>(r, P.n_dofs, 0.0, st);
     hipLaunchKernelGGL((k_element_vectors<M, EPB>), dim3((unsigned)((S.n_elems + EPB - 1) / EPB)), dim3(EPB * M::NPE), 0,
                        st, S.conn_orig.p, S.n_elems, P.coords.p, P.n_nodes, u, S.params, P.element_vectors.p);

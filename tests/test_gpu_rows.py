@@ -200,3 +200,48 @@ def test_newton_on_row_owner_tangent(torch_gpu, kind, size, precision):
     assert not infos[2]
     r = OA.residual(sets, settings["node coordinates"], sol.ravel(), d)
     assert np.linalg.norm(r[~settings["dirichlet dofs"].ravel()]) <= 1.1e-10
+
+
+def _residual(N, prob, u, r, stream):
+    N.call("apx_assemble_residual", prob.plan, C.c_void_p(u.data_ptr()), C.c_void_p(r.data_ptr()),
+           C.c_void_p(stream.cuda_stream))
+
+
+def test_residuals_on_two_streams_and_in_a_graph(torch_gpu):
+    """One plan, calls alternating between streams without waits, and a captured first call replayed between
+    eager ones: every residual is the one that a call alone gives (the same bits)."""
+    torch = torch_gpu
+    from autopdex_amd import _native as N
+    from autopdex_amd import backend
+    u, settings, static, sets, d = _problem("hex", (9, 8, 7), 1, seed=11)
+    prob = backend.get_problem(u, settings, static)
+    print("[case] rows on two streams", flush=True)
+    rng = np.random.default_rng(1)
+    us = [torch.from_numpy(0.05 * rng.standard_normal(prob.n_dofs)).cuda() for _ in range(8)]
+    graph, stream = torch.cuda.CUDAGraph(), [torch.cuda.Stream(), torch.cuda.Stream()]
+    static_u, static_r = us[0].clone(), torch.empty_like(us[0])
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):  # the plan's first residual
+        _residual(N, prob, static_u, static_r, torch.cuda.current_stream())
+    alone = []
+    for v in us:
+        r = torch.full_like(v, float("nan"))
+        torch.cuda.synchronize()
+        _residual(N, prob, v, r, torch.cuda.current_stream())
+        torch.cuda.synchronize()
+        alone.append(r)
+    rs = [torch.full_like(us[0], float("nan")) for _ in range(40)]
+    torch.cuda.synchronize()
+    for i, r in enumerate(rs):
+        _residual(N, prob, us[i % 8], r, stream[i % 2])
+    torch.cuda.synchronize()
+    for i, r in enumerate(rs):
+        assert torch.equal(r, alone[i % 8])
+    for i in (3, 1, 6):
+        static_u.copy_(us[i])
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(static_r, alone[i])
+        _residual(N, prob, us[0], rs[0], torch.cuda.current_stream())
+        torch.cuda.synchronize()
+        assert torch.equal(rs[0], alone[0])
