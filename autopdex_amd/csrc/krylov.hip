@@ -740,11 +740,11 @@ int line_blocks(const Plan& P) {
 
 // Lines of fewer than 32 rows would leave more than half of a wavefront's lanes idle, where it no longer
 // pays (FP64, us an iteration: 557,973 rows in lines of 31, SELL kernel 35.1; 575,972 in lines of 32
-// 34.8, of 64 31.5; 571,377 in lines of 127 29.6).  Systems that
-// apx_pcg_noalloc takes keep the SELL kernel, whose sums it shares bit by bit (and where the launches'
-// latency, not the bytes, sets the pace).
+// 34.8, of 64 31.5; 571,377 in lines of 127 29.6).  Lines of over two million rows would need more
+// workgroups than a row of partial sums holds.  Systems that apx_pcg_noalloc takes keep the SELL kernel,
+// whose sums it shares bit by bit (and where the launches' latency, not the bytes, sets the pace).
 static bool lines_pay(const Plan& P, size_t value_bytes) {
-  return P.line >= 32 && !noalloc_accepts(P, value_bytes);
+  return P.line >= 32 && line_blocks(P) <= kMaxBlocks && !noalloc_accepts(P, value_bytes);
 }
 
 // The upper diagonals of a SELL matrix into the plan's buffer for them, and the flag P.asymmetric that
