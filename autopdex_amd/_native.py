@@ -25,6 +25,11 @@ class KrylovStats(C.Structure):
                 ("final_residual", C.c_double), ("seconds", C.c_double)]
 
 
+class ResidentLayout(C.Structure):
+    _fields_ = [("threads", C.c_int), ("rows_per_thread", C.c_int), ("row_entries", C.c_int),
+                ("vectors_in_lds", C.c_int), ("chunks", C.c_int), ("workgroups", C.c_int), ("lds_bytes", C.c_int64)]
+
+
 class NewtonOptions(C.Structure):
     _fields_ = [("newton_tol", C.c_double), ("relative", C.c_int), ("maxiter", C.c_int),
                 ("damping", C.c_double), ("precision", C.c_int), ("precond", C.c_int),
@@ -63,6 +68,7 @@ _SIGS = {
     "apx_spmv": (_int, [_vp, _vp, _vp, _vp, _int, _vp]),
     "apx_pcg": (_int, [_vp, _vp, _vp, _vp, _int, _int, _dbl, _dbl, _int, C.POINTER(KrylovStats), _vp]),
     "apx_plan_set_resident_wait": (_int, [_vp, _dbl]),
+    "apx_resident_shape": (_int, [_i64, _i64, _int, _int, _int, C.POINTER(ResidentLayout)]),
     "apx_pcg_noalloc": (_int, [_vp, _vp, _vp, _vp, _int, _int, _dbl, _dbl, _int, C.POINTER(KrylovStats), _vp]),
     "apx_newton": (_int, [_vp, _vp, _vp, C.POINTER(NewtonOptions), C.POINTER(NewtonStats), _vp]),
     "apx_unet_create": (_int, [C.POINTER(_vp), _int, _vp, _int, _int, _int, _int, _int, _int]),

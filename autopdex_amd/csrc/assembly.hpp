@@ -73,6 +73,17 @@ template <class M, class V>
 bool pcg_resident(Plan& P, const M* vals, const V* inv, V* x, const V* r, const V* z, const V* p_old, V* p_new,
                   unsigned long long* zt, KState* S, double* part, KState* host_state, hipStream_t st);
 
+// How a resident run deals out a system of n rows of at most `row` entries, bandwidth bw: T threads a
+// workgroup, K rows a thread, rows of up to RW entries in registers (0: read in every iteration), xl:
+// x and D^-1 in LDS, cpw 64-row chunks a workgroup, G workgroups, bytes of dynamic LDS each.  T = 0: it
+// does not fit on `cus` compute units.
+struct ResidentShape {
+  int T = 0, K = 0, RW = 0, cpw = 0, G = 0;
+  bool xl = false;
+  size_t lds = 0;
+};
+ResidentShape resident_shape(int64_t n, int64_t bw, int row, size_t vector_bytes, int cus);
+
 // Symmetric 9-point matrices by grid lines (krylov.hip): the upper diagonals of SELL values for
 // line_product, with P.asymmetric set on the device where they are not the whole matrix; null: not
 // applicable.  vector_bytes: of an entry of the vectors.

@@ -270,6 +270,17 @@ int apx_plan_set_resident_wait(apx_plan* plan, double seconds) {
   });
 }
 
+int apx_resident_shape(int64_t n_free, int64_t bandwidth, int max_row, int precision, int compute_units,
+                       apx_resident_layout* out) {
+  return guarded([&] {
+    APX_REQUIRE(out, APX_ERR_ARG, "null argument");
+    APX_REQUIRE(n_free >= 0 && n_free < INT32_MAX && bandwidth >= 0 && max_row >= 0, APX_ERR_ARG, "invalid system");
+    APX_REQUIRE(precision == APX_FP64 || precision == APX_FP32, APX_ERR_ARG, "precision must be FP64 or FP32");
+    const ResidentShape s = resident_shape(n_free, bandwidth, max_row, precision == APX_FP64 ? 8 : 4, compute_units);
+    *out = apx_resident_layout{s.T, s.K, s.RW, s.xl ? 1 : 0, s.cpw, s.G, (int64_t)s.lds};
+  });
+}
+
 int apx_set_timing(apx_plan* plan, int enabled) {
   return guarded([&] {
     APX_REQUIRE(plan, APX_ERR_ARG, "null plan");

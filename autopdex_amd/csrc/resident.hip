@@ -499,18 +499,13 @@ struct ResidentLease {
   }
 };
 
-// How the rows are dealt out; T = 0: the system does not fit.
-struct Shape {
-  int T = 0, K = 0, RW = 0, cpw = 0, G = 0;
-  bool xl = false;
-  size_t lds = 0;
-};
-
 int device_cus(int dev) {
   int cus = 0;
   APX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   return cus;
 }
+
+}  // namespace
 
 // LDS for the vectors: it leaves room for the reduction words in 160 KB.
 constexpr size_t kResidentLds = 156 * 1024;
@@ -524,17 +519,24 @@ constexpr size_t kResidentLds = 156 * 1024;
 // take 2.0 against 3.6 in two.  Wide rows: 1,600 of 50 take 3.6 with 256 threads and 3.8 with 512,
 // 19,440 take 6.7 and 5.5; 1,863 of 81 5.8 and 8.2 (82 registers spill), 25,960 11.9 and 10.4.
 // Wherever a shape fits it was faster than the streaming kernels, up to the largest (see above).
-template <class M, class V>
-Shape resident_shape(const Plan& P, int cus) {
-  const int64_t chunks = P.n_chunks, bw = P.bandwidth;
-  Shape s;
-  if (!P.sell_dcol.p || P.n_free < 1 || cus < 1) return s;
+ResidentShape resident_shape(int64_t n, int64_t bw, int row, size_t vector_bytes, int cus) {
+  const int64_t chunks = (n + kSellC - 1) / kSellC;
+  ResidentShape s;
+  if (bw > INT16_MAX || n < 1 || cus < 1) return s;
   // cpw chunks per workgroup of T threads, rows of up to RW entries in registers
   auto take = [&](int T, int K, int RW, bool xl, int64_t cpw) {
-    const int64_t G = (chunks + cpw - 1) / cpw, own = std::min<int64_t>(P.n_free, cpw * 64);
-    const int64_t halo = G > 1 ? std::min<int64_t>(P.n_free - own, 2 * bw) : 0;
-    const size_t lds = (size_t)(own + 2 * halo + (xl ? 2 * own : 0)) * sizeof(V);
-    if (G > cus || own + halo > 65535 || lds > kResidentLds) return false;
+    const int64_t G = (chunks + cpw - 1) / cpw, own = std::min<int64_t>(n, cpw * 64);
+    if (G > cus) return false;
+    // The largest need of a workgroup, as the kernel lays out its LDS: the window of p, the halo's z, and
+    // with xl the own rows' x and D^-1.  A last workgroup of a few rows has the whole bandwidth before it.
+    int64_t words = 0, window = 0;
+    for (int64_t row0 = 0; row0 < n; row0 += own) {
+      const int64_t rows = std::min(own, n - row0), halo = std::min(bw, row0) + std::min(bw, n - row0 - rows);
+      window = std::max(window, rows + halo);
+      words = std::max(words, rows + 2 * halo + (xl ? 2 * rows : 0));
+    }
+    const size_t lds = (size_t)words * vector_bytes;
+    if (window > 65536 || lds > kResidentLds) return false;
     s.T = T;
     s.K = K;
     s.RW = RW;
@@ -544,7 +546,6 @@ Shape resident_shape(const Plan& P, int cus) {
     s.lds = lds;
     return true;
   };
-  const int row = P.max_row;
   if (row <= 9) {
     if (chunks <= 16 && take(1024, 1, 9, false, chunks)) return s;
     if (chunks <= 32 && take(1024, 2, 9, false, chunks)) return s;
@@ -571,8 +572,9 @@ Shape resident_shape(const Plan& P, int cus) {
   return s;
 }
 
+namespace {
 template <class M, class V, int T, int K, int RW, bool XL>
-bool launch_if(const Shape& s, const ResidentArgs& A, const M* vals, const V* inv, V* x, const V* r, const V* z,
+bool launch_if(const ResidentShape& s, const ResidentArgs& A, const M* vals, const V* inv, V* x, const V* r, const V* z,
                const V* p_old, V* p_new, hipStream_t st) {
   if (s.T != T || s.K != K || s.RW != RW || s.xl != XL) return false;
   const auto kernel = k_pcg_resident<M, V, T, K, RW, XL>;
@@ -596,7 +598,8 @@ bool pcg_resident(Plan& P, const M* vals, const V* inv, V* x, const V* r, const 
     APX_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
     P.clock_khz = khz > 0 ? khz : 100000;
   }
-  const Shape s = resident_shape<M, V>(P, std::min(P.cus, kResidentMaxGroups));
+  if (!P.sell_dcol.p) return false;
+  const ResidentShape s = resident_shape(P.n_free, P.bandwidth, P.max_row, sizeof(V), std::min(P.cus, kResidentMaxGroups));
   if (s.T == 0) return false;
   ResidentArgs A;
   A.n = (int)P.n_free;

@@ -162,6 +162,21 @@ int apx_pcg(apx_plan* plan, const void* vals_dev, const void* b_dev, void* x_dev
  * negative: always one launch per kernel.  The two agree to rounding.       */
 int apx_plan_set_resident_wait(apx_plan* plan, double seconds);
 
+/* How such a solve would deal out a system (no device is asked): rows of at most max_row entries, all
+ * within `bandwidth` of the diagonal, vectors in `precision`, a device of that many compute units.
+ * threads = 0: the system does not fit.  No counterpart in the reference (for sizing and tests).      */
+typedef struct apx_resident_layout {
+  int threads;          /* per workgroup                                              */
+  int rows_per_thread;
+  int row_entries;      /* entries of a row held in registers; 0: read in every iteration */
+  int vectors_in_lds;   /* 1: x and D^-1 in LDS instead of registers                  */
+  int chunks;           /* 64-row chunks per workgroup                                */
+  int workgroups;
+  int64_t lds_bytes;    /* dynamic LDS per workgroup                                  */
+} apx_resident_layout;
+int apx_resident_shape(int64_t n_free, int64_t bandwidth, int max_row, int precision, int compute_units,
+                       apx_resident_layout* out);
+
 /* Allocation-free apx_pcg.  No counterpart in the reference: it is for callers that
  * cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  Same arguments, kernels, iterates and
