@@ -48,7 +48,8 @@ void ensure_krylov_scratch(Plan& P, hipStream_t st);
 // reduction partials of the Krylov kernels: 4 rows of kMaxBlocks = 8192 doubles
 constexpr int64_t kKrylovPartials = 4 * 8192;
 // A resident run's slots and its ResidentOut lie behind the rows of partials that the kernels before
-// it use; the kernels that finish those partials clear them.
+// it use; the kernels that finish those partials clear them.  What comes between a run and its
+// re-anchoring (free_norm) uses the first row only.
 constexpr int kResidentMaxGroups = 256;
 constexpr int64_t kResidentSlotsAt = 2 * 8192;
 constexpr int kResidentSlotWords = 6 * kResidentMaxGroups;
@@ -66,9 +67,9 @@ void jacobi_inverse_f32_to_f64(Plan& P, const float* vals, double* inv_diag, hip
 
 // The iterations of a PCG run from x = 0, r, z = D^-1 r, p_old and the scalars S to a stop flag in one
 // launch, waited for (resident.hip).  x and p_new receive the solution and the last direction,
-// host_state (pinned, sizeof(ResidentOut)) the scalars; S follows when the run asks for a reliable
-// update.  zt: 2 n_free words of scratch of the vectors' type.  false: the system does not fit, or
-// the run was given up; x is 0, r, z, p_old and S are as they were.
+// host_state (pinned, sizeof(ResidentOut)) and the ResidentOut in part the scalars; S stays as it was (a
+// re-anchored run goes on from the latter).  zt: 2 n_free words of scratch of the vectors' type.  false:
+// the system does not fit, or the run was given up; x is 0, r, z and p_old are as they were.
 template <class M, class V>
 bool pcg_resident(Plan& P, const M* vals, const V* inv, V* x, const V* r, const V* z, const V* p_old, V* p_new,
                   unsigned long long* zt, KState* S, double* part, KState* host_state, hipStream_t st);
@@ -123,6 +124,7 @@ struct PcgRun {
   bool upper_known = false;
   int k0 = 0;  // iterations before the present streaming run
   int start_k = 0;         // iterations before the present resident run
+  bool resident_last = false;  // the last run was resident: S still holds the scalars from before it
   int maxiter = 0, iterations = 0;
   int64_t launched = 0;
   size_t counted = 0;

@@ -648,7 +648,13 @@ __global__ __launch_bounds__(kBS) void k_pcg_reanchor(int64_t n, const int32_t* 
   block_partials<kBS, 2>(v, partials);
 }
 
+// RESIDENT: the last run left its scalars with its slots, not in S (a copy behind every run would be 10 us).
+template <bool RESIDENT>
 __global__ __launch_bounds__(kFinBS) void k_pcg_reanchor_fin(KState* S, double* partials, int nb) {
+  if constexpr (RESIDENT) {
+    if (threadIdx.x == 0) *S = ((const ResidentOut*)(partials + kResidentSlotsAt + kResidentSlotWords))->state;
+    __syncthreads();  // before they are cleared
+  }
   double s[2];
   finalize_sums<2>(partials, nb, s);
   clear_resident_slots<kFinBS>(partials);
@@ -703,6 +709,7 @@ template <class M, class T>
 void PcgRun<M, T>::init(const T* b, const double* r_full, T* x_, double tol, double atol, int maxiter_, double delta) {
   x = x_ ? x_ : xw;
   start_k = 0;
+  resident_last = false;
   upper = nullptr;  // the matrix may be another one
   upper_known = false;
   maxiter = maxiter_ <= 0 ? (int)std::min<int64_t>(10 * n, INT32_MAX / 2) : maxiter_;
@@ -857,12 +864,14 @@ KState PcgRun<M, T>::run() {
     t_launch_events = nullptr;
     if (ran) {
       iterations = pinned_state->k;
+      resident_last = true;
       // the last direction was written beside p_old; iteration k reads it from pb (k odd) or pa
-      if (((iterations ^ start_k) & 1) == 0) std::swap(pa, pb);
+      if (iterations != start_k && ((iterations ^ start_k) & 1) == 0) std::swap(pa, pb);
       start_k = iterations;
       return *pinned_state;
     }
     streaming = true;
+    resident_last = false;
   }
   if (!external && !evs[0]) {
     APX_HIP(hipEventCreateWithFlags(&evs[0], hipEventDisableTiming));
@@ -933,7 +942,10 @@ template <class M, class T>
 void PcgRun<M, T>::reanchor(const double* r_full) {
   const int g = grid_for(n);
   hipLaunchKernelGGL(k_pcg_reanchor<T>, dim3(g), dim3(kBS), 0, st, n, P.red2full.p, r_full, inv, x, r, z, S, part);
-  hipLaunchKernelGGL(k_pcg_reanchor_fin, dim3(1), dim3(kFinBS), 0, st, S, part, g);
+  if (resident_last)
+    hipLaunchKernelGGL(k_pcg_reanchor_fin<true>, dim3(1), dim3(kFinBS), 0, st, S, part, g);
+  else
+    hipLaunchKernelGGL(k_pcg_reanchor_fin<false>, dim3(1), dim3(kFinBS), 0, st, S, part, g);
   APX_LAUNCH_CHECK();
 }
 

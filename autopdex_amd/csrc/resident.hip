@@ -640,8 +640,6 @@ bool pcg_resident(Plan& P, const M* vals, const V* inv, V* x, const V* r, const 
     fill<V>(x, P.n_free, V(0), st);
     return false;
   }
-  // what a further run or a reliable update reads
-  if (host->state.reliable) APX_HIP(hipMemcpyAsync(S, &A.out->state, sizeof(KState), hipMemcpyDeviceToDevice, st));
   return true;
 }
 
