@@ -82,6 +82,7 @@ int64_t Plan::device_bytes() const {
   for (auto& s : sets)
     b += s.conn.bytes() + s.conn_orig.bytes() + s.inc_ptr.bytes() + s.inc.bytes() + s.touched.bytes() + s.rn_ptr.bytes() +
          s.rn.bytes() + s.code.bytes();
+  for (auto& c : captured) b += c.vectors.bytes();
   return b;
 }
 

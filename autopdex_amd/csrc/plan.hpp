@@ -2,6 +2,7 @@
 #pragma once
 #include <map>
 #include <memory>
+#include <mutex>
 #include <string>
 
 #include <hip/hip_ext.h>
@@ -68,6 +69,13 @@ struct Plan {
   hipEvent_t scratch_done = nullptr;
   hipStream_t scratch_stream = nullptr;
   bool scratch_used = false;
+  struct Captured {  // element vectors of a capture's residuals on one stream (rows.hip)
+    unsigned long long id;
+    hipStream_t stream;
+    DevBuf<double> vectors;
+  };
+  std::vector<Captured> captured;
+  std::mutex scratch_mutex;  // of `captured`
   double build_seconds = 0.0;
 
   std::vector<double> coords_host;   // n_nodes * dim row-major

@@ -618,6 +618,70 @@ __global__ void k_gather_vectors(int64_t n_list, const int32_t* __restrict__ lis
   r[dof] = overwrite ? s : r[dof] + s;
 }
 
+// The same sums, bit by bit, without element vectors in memory: NPB nodes per workgroup, NPE threads each,
+// which evaluate the node's elements one after the other, every element as often as it has nodes.
+// For captured calls that get no scratch (captured_scratch).  64^3 Hex8: 306 us a replay, with scratch 87;
+// 512^2 plane-strain quads 19 either way.
+template <class M, int NPB>
+__global__ __launch_bounds__(NPB * M::NPE) void k_node_residuals(int64_t n_list, const int32_t* __restrict__ list,
+                                                                 const int32_t* __restrict__ ptr,
+                                                                 const int32_t* __restrict__ inc,
+                                                                 const int32_t* __restrict__ conn,
+                                                                 const double* __restrict__ coords, int64_t n_nodes,
+                                                                 const double* __restrict__ u, ModelParams mp,
+                                                                 int overwrite, double* __restrict__ r) {
+  constexpr int NPE = M::NPE, DIM = M::DIM, D = M::D, NQ = M::NQ, SW = (D * DIM + 1) | 1;
+  __shared__ double dn[NQ * NPE * DIM], sn[NQ * NPE];
+  __shared__ double xs[NPB][NPE][DIM], us[NPB][NPE][D], ns[M::NODAL ? NPB : 1][NPE][2];
+  __shared__ double sq[NPB * NPE][SW];
+  const int ln = threadIdx.x / NPE, t = threadIdx.x % NPE;
+  const int64_t l = blockIdx.x * (int64_t)NPB + ln;
+  const int64_t node = l >= n_list ? -1 : list ? list[l] : l;
+  const int32_t p0 = node < 0 ? 0 : ptr[node], p1 = node < 0 ? 0 : ptr[node + 1];
+  fill_gradients<M>(dn, sn);
+  double s = 0.0;  // thread i < D: component i
+  for (int32_t p = p0; __syncthreads_or(p < p1); ++p) {
+    const bool on = p < p1;
+    const int32_t ea = on ? inc[p] : 0, a = ea % NPE;
+    if (on) {
+      const int32_t c = conn[(int64_t)(ea / NPE) * NPE + t];
+#pragma unroll
+      for (int k = 0; k < DIM; ++k) xs[ln][t][k] = coords[k * n_nodes + c];
+#pragma unroll
+      for (int i = 0; i < D; ++i) us[ln][t][i] = u[(int64_t)c * D + i];
+      if constexpr (M::NODAL) {
+        ns[ln][t][0] = mp.nodal[0][c];
+        ns[ln][t][1] = mp.nodal[1][c];
+      }
+    }
+    __syncthreads();
+    if (on) {
+      double S[D][DIM];
+      const double f = ResModel<M>::eval(
+          t, dn + t * NPE * DIM, sn + t * NPE, [&](int b, int i) { return xs[ln][b][i]; },
+          [&](int b, int i) { return us[ln][b][i]; }, ns[M::NODAL ? ln : 0], mp, S);
+#pragma unroll
+      for (int i = 0; i < D; ++i)
+#pragma unroll
+        for (int j = 0; j < DIM; ++j) sq[threadIdx.x][i * DIM + j] = S[i][j];
+      sq[threadIdx.x][D * DIM] = f;
+    }
+    __syncthreads();
+    if (on && t < D) {
+      double row = 0.0;
+      for (int q = 0; q < NQ; ++q) {
+#pragma unroll
+        for (int j = 0; j < DIM; ++j) row += sq[ln * NPE + q][t * DIM + j] * dn[(q * NPE + a) * DIM + j];
+        if constexpr (D == 1) row -= sq[ln * NPE + q][DIM] * sn[q * NPE + a];
+      }
+      s += row;
+    }
+  }
+  if (node < 0 || t >= D) return;
+  double& out = r[node * D + t];
+  out = overwrite ? s : out + s;
+}
+
 // Boundary lines: every listed node evaluates its own (one or two) lines; one launch, nothing stored
 template <class M>
 __global__ void k_line_vectors(int64_t n_list, const int32_t* __restrict__ list, const int32_t* __restrict__ ptr,
@@ -649,16 +713,41 @@ __global__ void k_line_vectors(int64_t n_list, const int32_t* __restrict__ list,
   r[node * 2 + 1] += s[1];
 }
 
+bool is_capturing(hipStream_t st, unsigned long long* id = nullptr) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long ignored;
+  if (hipStreamGetCaptureInfo(st, &status, id ? id : &ignored) != hipSuccess) (void)hipGetLastError();
+  return status != hipStreamCaptureStatusNone;
+}
+
+// Element vectors of captured residuals: replays may overlap with anything else of the plan, other
+// graphs and other branches of their own graph among it, so every capture has its own on each of its streams
+// (whose calls follow one another in the graph).  A graph may be replayed as long as the plan lives, so
+// they stay with the plan, and it makes at most kMost; null: no more of them, or no memory.
+double* captured_scratch(Plan& P, hipStream_t st, unsigned long long id) {
+  constexpr size_t kMost = 16;
+  std::lock_guard<std::mutex> lock(P.scratch_mutex);
+  for (auto& c : P.captured)
+    if (c.id == id && c.stream == st) return c.vectors.p;
+  if (P.captured.size() == kMost) return nullptr;
+  Plan::Captured c{id, st, {}};
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // an allocation is no part of the capture
+  APX_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+  const bool room = c.vectors.try_alloc(P.element_vectors.n);
+  APX_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+  if (!room) return nullptr;
+  P.captured.push_back(std::move(c));
+  return P.captured.back().vectors.p;
+}
+
 // The plan's scratch is one: work on it from another stream than the last waits for that work.  (Under
-// capture neither is recorded: what a graph's replays overlap with is the caller's to order.)
+// capture, of a tangent, neither is recorded: what a graph's replays overlap with is the caller's to order.)
 struct ScratchUse {
   Plan& P;
   hipStream_t st;
   bool capturing = false;
   ScratchUse(Plan& p, hipStream_t s) : P(p), st(s) {
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &status) != hipSuccess) (void)hipGetLastError();
-    capturing = status != hipStreamCaptureStatusNone;
+    capturing = is_capturing(st);
     if (capturing) return;
     if (!P.scratch_done) APX_HIP(hipEventCreateWithFlags(&P.scratch_done, hipEventDisableTiming));
     if (P.scratch_used && P.scratch_stream != st) APX_HIP(hipStreamWaitEvent(st, P.scratch_done, 0));
@@ -794,13 +883,24 @@ bool gather_residual(Plan& P, ElemSet& S, const double* u, double* r, bool overw
       APX_REQUIRE(S.params.nodal[0] && S.params.nodal[1], APX_ERR_STATE,
                   "variable-coefficient Poisson set needs nodal fields g and f bound");
     }
-    // (element_vectors: allocated with the plan)
-    ScratchUse use(P, st);
     if (overwrite && !S.touched_all) fill<double>(r, P.n_dofs, 0.0, st);
-    hipLaunchKernelGGL((k_element_vectors<M, EPB>), dim3((unsigned)((S.n_elems + EPB - 1) / EPB)), dim3(EPB * M::NPE), 0,
-                       st, S.conn_orig.p, S.n_elems, P.coords.p, P.n_nodes, u, S.params, P.element_vectors.p);
-    hipLaunchKernelGGL(k_gather_vectors, dim3((unsigned)((n * M::D + 255) / 256)), dim3(256), 0, st, n, list, S.inc_ptr.p,
-                       S.inc.p, P.element_vectors.p, (int)M::D, overwrite && S.touched_all ? 1 : 0, r);
+    const int set = overwrite && S.touched_all ? 1 : 0;
+    auto by_elements = [&](double* vectors) {
+      hipLaunchKernelGGL((k_element_vectors<M, EPB>), dim3((unsigned)((S.n_elems + EPB - 1) / EPB)), dim3(EPB * M::NPE),
+                         0, st, S.conn_orig.p, S.n_elems, P.coords.p, P.n_nodes, u, S.params, vectors);
+      hipLaunchKernelGGL(k_gather_vectors, dim3((unsigned)((n * M::D + 255) / 256)), dim3(256), 0, st, n, list,
+                         S.inc_ptr.p, S.inc.p, vectors, (int)M::D, set, r);
+    };
+    unsigned long long capture = 0;
+    if (!is_capturing(st, &capture)) {
+      ScratchUse use(P, st);
+      by_elements(P.element_vectors.p);  // (allocated with the plan)
+    } else if (double* vectors = captured_scratch(P, st, capture)) {
+      by_elements(vectors);
+    } else {
+      hipLaunchKernelGGL((k_node_residuals<M, EPB>), dim3((unsigned)((n + EPB - 1) / EPB)), dim3(EPB * M::NPE), 0, st, n,
+                         list, S.inc_ptr.p, S.inc.p, S.conn_orig.p, P.coords.p, P.n_nodes, u, S.params, set, r);
+    }
     APX_LAUNCH_CHECK();
     return true;
   });

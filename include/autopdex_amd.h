@@ -112,7 +112,11 @@ int apx_plan_free_dofs(const apx_plan* plan, int32_t* red2full_host);
 
 /* assembler.assemble_residual (assembler.py:587-637, user potential
  * :1064-1088): r_dev (n_dofs, FP64, full length incl. Dirichlet rows)
- * = sum over sets of the scattered element residuals at u_dev (n_dofs).     */
+ * = sum over sets of the scattered element residuals at u_dev (n_dofs).
+ * Calls may be captured into a graph (also a plan's first one), and replays may
+ * overlap with other calls: the captures of a plan hold element vectors of their
+ * own, which live as long as the plan, up to 16 of them; later captures form the
+ * same bits without (64^3 Hex8: 306 us a replay instead of 87).              */
 int apx_assemble_residual(apx_plan* plan, const double* u_dev, double* r_dev, void* stream);
 
 /* assembler.assemble_tangent (assembler.py:682-777, :1115-1149) followed by the
