@@ -78,7 +78,8 @@ int64_t Plan::device_bytes() const {
   int64_t b = coords.bytes() + dmask.bytes() + full2red.bytes() + red2full.bytes() + indptr.bytes() +
               indices.bytes() + diag_slot.bytes() + sell_ptr.bytes() + sell_cols.bytes() + sell_dcol.bytes() +
               csr2sell.bytes() + vals64.bytes() + vals32.bytes() + w64.bytes() + w32.bytes() + r_full.bytes() +
-              diag_full.bytes() + partials.bytes() + lines64.bytes() + lines32.bytes() + element_vectors.bytes() + element_matrices.bytes();
+              diag_full.bytes() + partials.bytes() + lines64.bytes() + lines32.bytes() + element_vectors.bytes() +
+              element_matrices64.bytes() + element_matrices32.bytes();
   for (auto& s : sets)
     b += s.conn.bytes() + s.conn_orig.bytes() + s.inc_ptr.bytes() + s.inc.bytes() + s.touched.bytes() + s.rn_ptr.bytes() +
          s.rn.bytes() + s.code.bytes();

@@ -65,7 +65,8 @@ struct Plan {
   bool finalized = false;
   // Scratch of the row-owner kernels, and the last work on it: a call on another stream waits for
   // that on the device (rows.hip, ScratchUse).
-  DevBuf<double> element_vectors, element_matrices;
+  DevBuf<double> element_vectors, element_matrices64;
+  DevBuf<float> element_matrices32;
   hipEvent_t scratch_done = nullptr;
   hipStream_t scratch_stream = nullptr;
   bool scratch_used = false;

@@ -741,7 +741,8 @@ double* captured_scratch(Plan& P, hipStream_t st, unsigned long long id) {
 }
 
 // The plan's scratch is one: work on it from another stream than the last waits for that work.  (Under
-// capture, of a tangent, neither is recorded: what a graph's replays overlap with is the caller's to order.)
+// capture, of a tangent, neither is recorded: replays that overlap with tangents of the same type are the
+// caller's to order.)
 struct ScratchUse {
   Plan& P;
   hipStream_t st;
@@ -760,6 +761,25 @@ struct ScratchUse {
   }
 };
 
+// Element matrices of the plan's largest set, one buffer per type: allocated by the first tangent of that
+// type and kept with the plan, so a captured tangent's pointer stays good.
+template <class T>
+T* element_matrices(Plan& P) {
+  DevBuf<T>* buf;
+  if constexpr (sizeof(T) == 8)
+    buf = &P.element_matrices64;
+  else
+    buf = &P.element_matrices32;
+  if (!buf->p) {
+    size_t words = 0;
+    for (const auto& S : P.sets)
+      if (S.model != APX_MODEL_LINE_TRACTION)
+        words = std::max(words, (size_t)S.n_elems * S.npe * (S.npe / 2 + 1) * P.d * P.d);  // kBlocks per node
+    buf->alloc(words);
+  }
+  return buf->p;
+}
+
 template <class M, class T, class TO, bool CSR>
 void run_rows(Plan& P, ElemSet& S, const double* u, void* vals, bool accumulate, hipStream_t st) {
   if constexpr (M::NODAL) {
@@ -767,11 +787,10 @@ void run_rows(Plan& P, ElemSet& S, const double* u, void* vals, bool accumulate,
                 "variable-coefficient Poisson set needs nodal fields g and f bound");
   }
   constexpr int EPB = elements_per_block<M>(), NPW = 64 / M::NPE;
-  const size_t words = ((size_t)S.n_elems * M::NPE * kBlocks<M::NPE> * M::D * M::D * sizeof(T) + 7) / 8;
-  if (P.element_matrices.n < words) P.element_matrices.alloc(words);
+  T* matrices = element_matrices<T>(P);
   ScratchUse use(P, st);
   hipLaunchKernelGGL((k_element_matrices<M, T>), dim3((unsigned)((S.n_elems + EPB - 1) / EPB)), dim3(EPB * M::NPE), 0, st,
-                     S.conn_orig.p, S.n_elems, P.coords.p, P.n_nodes, u, S.params, (T*)P.element_matrices.p);
+                     S.conn_orig.p, S.n_elems, P.coords.p, P.n_nodes, u, S.params, matrices);
   RowArgs A;
   A.rn_ptr = S.rn_ptr.p;
   A.rn = S.rn.p;
@@ -786,7 +805,7 @@ void run_rows(Plan& P, ElemSet& S, const double* u, void* vals, bool accumulate,
   A.stride = A.window | 1;
   A.accumulate = accumulate ? 1 : 0;
   A.n_elems = S.n_elems;
-  A.matrices = P.element_matrices.p;
+  A.matrices = matrices;
   A.vals = vals;
   const int waves = std::max(1, std::min(4, (S.rn_max + NPW - 1) / NPW));
   const size_t bytes = ((size_t)64 * A.stride + 1) * sizeof(T);

@@ -122,7 +122,10 @@ int apx_assemble_residual(apx_plan* plan, const double* u_dev, double* r_dev, vo
 /* assembler.assemble_tangent (assembler.py:682-777, :1115-1149) followed by the
  * reduction of scipy_assembling: values of the reduced CSR (nnz) in FP64, FP32
  * or FP32 rounded from FP64 arithmetic (precision = apx_precision), pattern
- * from apx_plan_csr_pattern.                                                */
+ * from apx_plan_csr_pattern.  The plan keeps scratch of its own for FP64 (and
+ * rounded) and for FP32 tangents, allocated by the first of each; later ones may
+ * be captured into a graph.  Eager calls are ordered on it across streams; replays
+ * that overlap with other tangents of the same scratch are the caller's to order. */
 int apx_assemble_tangent(apx_plan* plan, const double* u_dev, void* vals_dev, int precision, void* stream);
 
 /* assembler.assemble_tangent_diagonal (assembler.py:639-680, :1090-1113):

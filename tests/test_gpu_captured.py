@@ -90,3 +90,48 @@ def test_replays_overlap_with_other_residuals(torch_gpu, kind, size):
         for i, rs in enumerate(out):
             for r in rs:
                 assert torch.equal(r, alone[i])
+
+
+def _tangent(prob, u, vals, precision, stream):
+    from autopdex_amd import _native as N
+    N.call("apx_assemble_tangent", prob.plan, C.c_void_p(u.data_ptr()), C.c_void_p(vals.data_ptr()), precision,
+           C.c_void_p(stream.cuda_stream))
+
+
+@pytest.mark.parametrize("kind,size,sets", [("hex", (12, 13, 14), 1), ("panel", (60, 61), 2), ("q2", (14, 15), 2)])
+@pytest.mark.parametrize("captured", ["fp32", "fp64"])
+def test_captured_tangent_beside_the_other_precision(torch_gpu, kind, size, sets, captured):
+    """A captured tangent keeps its scratch when the other precision comes later and when it runs beside it;
+    with two sets, the second is the larger one."""
+    torch = torch_gpu
+    from autopdex_amd import _native as N
+    from autopdex_amd import backend
+    u, settings, static, _, _ = _problem(kind, size, 1, seed=6)
+    if sets == 2:
+        elems = settings["connectivity"][0]
+        k = len(elems) // 4
+        settings["connectivity"] = (np.ascontiguousarray(elems[:k]), np.ascontiguousarray(elems[k:]))
+        static["model"], static["assembling mode"] = static["model"] * 2, static["assembling mode"] * 2
+    prob = backend.get_problem(u, settings, static)
+    print(f"[case] captured tangent {kind} {size} {captured}", flush=True)
+    ud = prob.to_device(u.ravel())
+    types = {"fp32": (N.APX_FP32, torch.float32), "fp64": (N.APX_FP64, torch.float64)}
+    (mine, dt), (other, odt) = types[captured], types["fp64" if captured == "fp32" else "fp32"]
+    vals = torch.empty(prob.nnz, dtype=dt, device="cuda")
+    _tangent(prob, ud, vals, mine, torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    want = vals.clone()
+    graph = _capture(torch, lambda st: _tangent(prob, ud, vals, mine, st))
+    beside = [torch.empty(prob.nnz, dtype=odt, device="cuda") for _ in range(9)]
+    _tangent(prob, ud, beside[0], other, torch.cuda.current_stream())
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for _ in range(4):
+        vals.fill_(float("nan"))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(streams[0]):
+            graph.replay()
+        for b in beside[1:]:
+            _tangent(prob, ud, b, other, streams[1])
+        torch.cuda.synchronize()
+        assert torch.equal(vals, want)
+        assert all(torch.equal(b, beside[0]) for b in beside)
