@@ -63,20 +63,18 @@ struct Plan {
   int dim = 0, d = 0;
   int64_t n_nodes = 0, n_dofs = 0, n_free = 0, nnz = 0;
   bool finalized = false;
-  // Scratch of the row-owner kernels, and the last work on it: a call on another stream waits for
-  // that on the device (rows.hip, ScratchUse).
+  // Scratch of the row-owner kernels, and the last work on it: every call waits for that on the
+  // device (rows.hip, ScratchUse).
   DevBuf<double> element_vectors, element_matrices64;
   DevBuf<float> element_matrices32;
   hipEvent_t scratch_done = nullptr;
-  hipStream_t scratch_stream = nullptr;
-  bool scratch_used = false;
   struct Captured {  // element vectors of a capture's residuals on one stream (rows.hip)
     unsigned long long id;
     hipStream_t stream;
     DevBuf<double> vectors;
   };
   std::vector<Captured> captured;
-  std::mutex scratch_mutex;  // of `captured`
+  std::mutex scratch_mutex;
   double build_seconds = 0.0;
 
   std::vector<double> coords_host;   // n_nodes * dim row-major

@@ -740,24 +740,26 @@ double* captured_scratch(Plan& P, hipStream_t st, unsigned long long id) {
   return P.captured.back().vectors.p;
 }
 
-// The plan's scratch is one: work on it from another stream than the last waits for that work.  (Under
-// capture, of a tangent, neither is recorded: replays that overlap with tangents of the same type are the
-// caller's to order.)
+// The plan's scratch is one: a call's work on it waits on the device for the last call's, from
+// whatever stream and thread that came, and no other call comes between its wait and its own event.  (The
+// wait is made on one stream too: a handle may be that of a stream made since, or of another thread's
+// default stream.)  Under capture, of a tangent, neither is recorded: replays that overlap with tangents
+// of the same type are the caller's to order.
 struct ScratchUse {
   Plan& P;
   hipStream_t st;
+  std::unique_lock<std::mutex> lock;
   bool capturing = false;
-  ScratchUse(Plan& p, hipStream_t s) : P(p), st(s) {
+  ScratchUse(Plan& p, hipStream_t s) : P(p), st(s), lock(p.scratch_mutex) {
     capturing = is_capturing(st);
     if (capturing) return;
-    if (!P.scratch_done) APX_HIP(hipEventCreateWithFlags(&P.scratch_done, hipEventDisableTiming));
-    if (P.scratch_used && P.scratch_stream != st) APX_HIP(hipStreamWaitEvent(st, P.scratch_done, 0));
+    if (P.scratch_done)
+      APX_HIP(hipStreamWaitEvent(st, P.scratch_done, 0));
+    else
+      APX_HIP(hipEventCreateWithFlags(&P.scratch_done, hipEventDisableTiming));
   }
   ~ScratchUse() {
-    if (capturing) return;
-    (void)hipEventRecord(P.scratch_done, st);
-    P.scratch_stream = st;
-    P.scratch_used = true;
+    if (!capturing) (void)hipEventRecord(P.scratch_done, st);
   }
 };
 
@@ -787,8 +789,8 @@ void run_rows(Plan& P, ElemSet& S, const double* u, void* vals, bool accumulate,
                 "variable-coefficient Poisson set needs nodal fields g and f bound");
   }
   constexpr int EPB = elements_per_block<M>(), NPW = 64 / M::NPE;
-  T* matrices = element_matrices<T>(P);
   ScratchUse use(P, st);
+  T* matrices = element_matrices<T>(P);
   hipLaunchKernelGGL((k_element_matrices<M, T>), dim3((unsigned)((S.n_elems + EPB - 1) / EPB)), dim3(EPB * M::NPE), 0, st,
                      S.conn_orig.p, S.n_elems, P.coords.p, P.n_nodes, u, S.params, matrices);
   RowArgs A;
