@@ -130,7 +130,7 @@ struct PcgRun {
   size_t counted = 0;
   int64_t spmv_bytes = 0, upd_bytes = 0;
   hipEvent_t evs[2] = {nullptr, nullptr};
-  std::vector<EventPair> ev_spmv, ev_upd, ev_res;
+  std::vector<EventPair> ev_spmv, ev_upd, ev_res, ev_given_up;
 
   PcgRun(Plan& P, const M* vals, const T* inv, hipStream_t st);
   // caller-provided workspace: work = 6 n_free vectors, partials = kKrylovPartials doubles,

@@ -267,6 +267,7 @@ int apx_plan_set_resident_wait(apx_plan* plan, double seconds) {
     APX_REQUIRE(plan, APX_ERR_ARG, "null plan");
     APX_REQUIRE(seconds <= 60.0, APX_ERR_ARG, "resident wait must be at most 60 seconds");
     plan->resident_wait = seconds;
+    plan->resident_given_up = plan->resident_skip = 0;
   });
 }
 

@@ -858,7 +858,7 @@ KState PcgRun<M, T>::run() {
     const bool ran = !streaming && pcg_resident<M, T>(P, vals, inv, x, r, z, odd ? pb : pa, odd ? pa : pb,
                                                       (unsigned long long*)q, S, part, pinned_state, st);
     if (timed && !t_launch_events)
-      ev_res.push_back(e);
+      (ran ? ev_res : ev_given_up).push_back(e);
     else if (timed)
       P.evpool.insert(P.evpool.end(), {e.a, e.b});
     t_launch_events = nullptr;
@@ -961,6 +961,7 @@ void PcgRun<M, T>::collect_timing() {
                  upper ? line_bytes : spmv_bytes, k);
   timing_collect(P, f64 ? "pcg_update_f64" : "pcg_update_f32", ev_upd, upper ? n * 5 * (int64_t)sizeof(T) : upd_bytes, k);
   timing_collect(P, f64 ? "pcg_resident_f64" : "pcg_resident_f32", ev_res, 0, ev_res.size());
+  timing_collect(P, "pcg_resident_given_up", ev_given_up, 0, ev_given_up.size());
   counted = iterations;
 }
 

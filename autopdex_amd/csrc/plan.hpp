@@ -133,6 +133,8 @@ struct Plan {
   // no resident runs).
   int cus = 0, clock_khz = 0;
   double resident_wait = 2.0;
+  int resident_given_up = 0;  // runs given up since one was completed (at most 4)
+  int resident_skip = 0;      // runs to go before the next is tried
   struct UNet* net = nullptr;  // attached learned preconditioner (not owned)
   const double* net_g = nullptr;  // nodal coefficient channel of the network input (device, optional)
   // Jacobi scaling of the network (1 / sqrt|A_ii| per free DOF): the network maps

@@ -601,6 +601,10 @@ bool pcg_resident(Plan& P, const M* vals, const V* inv, V* x, const V* r, const 
   if (!P.sell_dcol.p) return false;
   const ResidentShape s = resident_shape(P.n_free, P.bandwidth, P.max_row, sizeof(V), std::min(P.cus, kResidentMaxGroups));
   if (s.T == 0) return false;
+  if (P.resident_skip > 0) {
+    --P.resident_skip;
+    return false;
+  }
   ResidentArgs A;
   A.n = (int)P.n_free;
   A.n_chunks = (int)P.n_chunks;
@@ -638,8 +642,14 @@ bool pcg_resident(Plan& P, const M* vals, const V* inv, V* x, const V* r, const 
   std::atomic_thread_fence(std::memory_order_acquire);  // written by the kernel
   if (host->aborted) {
     fill<V>(x, P.n_free, V(0), st);
+    // Where the workgroups do not get onto the device together (another process's runs hold its compute
+    // units, a masked queue), every further run would wait as long in vain: the plan's next 16 runs go to the
+    // streaming kernels at once, after a second give-up 64, then 256, 1,024 and 4,096.
+    P.resident_skip = 16 << 2 * P.resident_given_up;
+    P.resident_given_up = std::min(P.resident_given_up + 1, 4);
     return false;
   }
+  P.resident_given_up = 0;
   return true;
 }
 

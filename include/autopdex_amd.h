@@ -165,8 +165,10 @@ int apx_pcg(apx_plan* plan, const void* vals_dev, const void* b_dev, void* x_dev
 
 /* A Jacobi-PCG solve whose vectors fit on the compute units runs all its iterations in one launch,
  * in which workgroups wait for each other.  A wait longer than `seconds` (default 2; at most 60)
- * gives that launch up, and the solve goes on with one launch per kernel, as larger systems do;
- * negative: always one launch per kernel.  The two agree to rounding.       */
+ * gives that launch up, and the solve goes on with one launch per kernel, as larger systems do, and so
+ * do the plan's next 16 solves (after a second give-up 64, then 256, 1,024, 4,096; a completed launch
+ * or a call of this starts the count anew).  0: given up at the first wait of some 60 tries; negative:
+ * always one launch per kernel.  The two agree to rounding.                  */
 int apx_plan_set_resident_wait(apx_plan* plan, double seconds);
 
 /* How such a solve would deal out a system (no device is asked): rows of at most max_row entries, all

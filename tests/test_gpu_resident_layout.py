@@ -80,20 +80,30 @@ class System:
     def solve(self, torch, precision, tol, wait=2.0):
         """(x, iterations, resident launches)"""
         from autopdex_amd import _native as N
+        N.call("apx_plan_set_resident_wait", self.plan, wait)
+        x, its, completed, given_up = self.run(torch, precision, tol)
+        assert given_up == 0
+        return x, its, completed
+
+    def run(self, torch, precision, tol):
+        """(x, iterations, completed resident launches, given up ones)"""
+        from autopdex_amd import _native as N
         from autopdex_amd.backend import current_stream
         dt = torch.float64 if precision == N.APX_FP64 else torch.float32
         vals, b = torch.from_numpy(self.A.data).to("cuda", dt), torch.from_numpy(self.b).to("cuda", dt)
         x = torch.full_like(b, float("nan"))
-        ks, ms, count, nbytes = N.KrylovStats(), C.c_double(), C.c_int64(), C.c_int64()
-        N.call("apx_plan_set_resident_wait", self.plan, wait)
+        ks, ms, nbytes = N.KrylovStats(), C.c_double(), C.c_int64()
         N.call("apx_set_timing", self.plan, 1)
         N.call("apx_pcg", self.plan, C.c_void_p(vals.data_ptr()), C.c_void_p(b.data_ptr()), C.c_void_p(x.data_ptr()),
                precision, N.APX_PRECOND_JACOBI, tol, 0.0, 0, C.byref(ks), current_stream())
-        name = b"pcg_resident_f64" if precision == N.APX_FP64 else b"pcg_resident_f32"
-        N.call("apx_get_timing", self.plan, name, C.byref(ms), C.byref(count), C.byref(nbytes))
+        counts = []
+        for name in (b"pcg_resident_f64" if precision == N.APX_FP64 else b"pcg_resident_f32", b"pcg_resident_given_up"):
+            count = C.c_int64()
+            N.call("apx_get_timing", self.plan, name, C.byref(ms), C.byref(count), C.byref(nbytes))
+            counts.append(count.value)
         N.call("apx_set_timing", self.plan, 0)
         assert ks.converged == 1
-        return x.double().cpu().numpy(), ks.iterations, count.value
+        return x.double().cpu().numpy(), ks.iterations, *counts
 
 
 # (mesh, size, random numbering, expected threads, rows per thread, entries in registers)
@@ -126,3 +136,24 @@ def test_resident_pcg_by_layout(torch_gpu, kind, size, shuffle, shape, precision
     xs, its_s, resident = s.solve(torch, prec, tol, wait=-1.0)  # one launch per kernel
     assert resident == 0 and abs(its - its_s) <= 1
     assert np.linalg.norm(s.A @ xs - s.b) <= most * norm
+
+
+def test_a_given_up_launch_is_remembered(torch_gpu):
+    """Without patience the launches of a large grid are given up: the solve is completed all the same, the
+    plan's next 16 solves do without, a further give-up counts for 64, and setting the wait starts anew."""
+    torch = torch_gpu
+    from autopdex_amd import _native as N
+    s = System("quad", (900, 901, 1), 0)
+    norm = np.linalg.norm(s.b)
+    N.call("apx_plan_set_resident_wait", s.plan, 0.0)
+    tried = []
+    for i in range(24):
+        x, its, completed, given_up = s.run(torch, N.APX_FP64, 1e-12)
+        assert np.linalg.norm(s.A @ x - s.b) <= 1.1e-12 * norm
+        if completed or given_up:
+            tried.append((i, given_up))
+    print(f"[case] resident launches without patience (solve, given up): {tried}", flush=True)
+    assert tried[0] == (0, 1)
+    assert [i for i, _ in tried] == [0, 17]
+    x, its, completed = s.solve(torch, N.APX_FP64, 1e-12)
+    assert completed == 1 and np.linalg.norm(s.A @ x - s.b) <= 1.1e-12 * norm
