@@ -38,6 +38,7 @@
 #include <condition_variable>
 #include <cstring>
 #include <mutex>
+#include <optional>
 #include <type_traits>
 
 #include "assembly.hpp"
@@ -628,7 +629,14 @@ bool pcg_resident(Plan& P, const M* vals, const V* inv, V* x, const V* r, const 
   A.host = host;
   std::memset(host, 0, sizeof(ResidentOut));
   {
-    ResidentLease lease(dev, s.G, P.cus);
+    // The compute units are held only while the run is on the device: what the stream has to do before it is
+    // waited for first, or a solve on another thread would wait for all of that (10 us a solve).  A
+    // single workgroup meets nobody and holds none; others at most wait for it to end.
+    std::optional<ResidentLease> lease;
+    if (s.G > 1) {
+      APX_HIP(hipStreamSynchronize(st));
+      lease.emplace(dev, s.G, P.cus);
+    }
     const bool launched = APX_SHAPE(1024, 1, 9, false) || APX_SHAPE(1024, 2, 9, false) || APX_SHAPE(512, 6, 9, true) || APX_SHAPE(512, 8, 9, true) ||
                           APX_SHAPE(1024, 1, 18, false) || APX_SHAPE(512, 3, 18, true) ||
                           APX_SHAPE(512, 4, 18, true) || APX_SHAPE(256, 1, 54, false) ||

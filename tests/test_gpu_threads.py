@@ -1,10 +1,12 @@
 """One plan, or one device, used from several threads and streams at once."""
+import ctypes as C
 import threading
 
 import numpy as np
 import pytest
 
 from tests.test_gpu_captured import _residual, _tangent
+from tests.test_gpu_resident_layout import System
 from tests.test_gpu_rows import _problem
 
 pytestmark = pytest.mark.gpu
@@ -63,3 +65,72 @@ def test_assembly_of_one_plan_from_three_threads(torch_gpu, kind, size):
     _in_threads(torch, 3, work)
     for i in range(3):
         assert all(torch.equal(r, rs[i]) and torch.equal(t, ts[i]) for r, t in got[i])
+
+
+def _solve(torch, s):
+    from autopdex_amd import _native as N
+    x, its, completed, given_up = s.run(torch, N.APX_FP64, 1e-12)
+    assert completed == 1 and given_up == 0
+    assert np.linalg.norm(s.A @ x - s.b) <= 1.1e-12 * np.linalg.norm(s.b)
+    return x
+
+
+def test_resident_solves_on_three_threads(torch_gpu):
+    """Systems that together have more workgroups than the device has compute units take turns: every run
+    is completed, with the bits that it has alone."""
+    torch = torch_gpu
+    systems = [System("quad", (900, 901, 1), 0), System("quad", (800, 799, 1), 0), System("brick", (10, 11, 12), 0),
+               System("quad", (20, 21, 1), 0)]
+    print("[case] resident solves on threads", flush=True)
+    alone = [_solve(torch, s) for s in systems]
+
+    def work(i):
+        for _ in range(6):
+            assert np.array_equal(_solve(torch, systems[i]), alone[i])
+
+    _in_threads(torch, len(systems), work)
+
+
+def test_a_solve_does_not_wait_for_another_threads_stream(torch_gpu):
+    """A solve whose stream still has half a second of other work to do holds no compute units meanwhile: a
+    solve on another thread (allocation-free, since freeing memory waits for the whole device) ends before."""
+    torch = torch_gpu
+    from autopdex_amd import _native as N
+    first, second = System("quad", (885, 886, 1), 0), System("quad", (300, 301, 1), 0)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert first.layout(0, cus).workgroups + second.layout(0, cus).workgroups > cus  # not both at once
+    vals, b = torch.from_numpy(second.A.data).cuda(), torch.from_numpy(second.b).cuda()
+    x = torch.empty_like(b)
+
+    def solve_second():
+        ks = N.KrylovStats()
+        N.call("apx_pcg_noalloc", second.plan, C.c_void_p(vals.data_ptr()), C.c_void_p(b.data_ptr()),
+               C.c_void_p(x.data_ptr()), N.APX_FP64, N.APX_PRECOND_JACOBI, 1e-12, 0.0, 0, C.byref(ks),
+               C.c_void_p(torch.cuda.current_stream().cuda_stream))
+        return ks.converged
+
+    _solve(torch, first)
+    assert solve_second() == 1
+    start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    start.record()
+    torch.cuda._sleep(10_000_000)
+    end.record()
+    end.synchronize()
+    cycles = int(10_000_000 * 500 / start.elapsed_time(end))
+    print(f"[case] two threads, one with a busy stream: {cycles} cycles", flush=True)
+    queued, busy, seen = threading.Event(), torch.cuda.Event(), []
+
+    def work(i):
+        if i == 0:
+            torch.cuda._sleep(cycles)
+            busy.record()
+            queued.set()
+            _solve(torch, first)
+        else:
+            assert queued.wait(10)
+            threading.Event().wait(0.1)  # the first solve has come to its run
+            seen.append((solve_second(), busy.query()))
+
+    _in_threads(torch, 2, work)
+    assert seen == [(1, False)]
+    assert np.linalg.norm(second.A @ x.cpu().numpy() - second.b) <= 1.1e-12 * np.linalg.norm(second.b)
