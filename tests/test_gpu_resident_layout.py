@@ -113,9 +113,19 @@ WIDE = [("clamped", (2, 256), 0, (1024, 1, 18)),     # a last workgroup of 4 row
         ("quad", (31, 40, 2), 1, (1024, 1, 18)), ("q2", (4, 8), 1, (256, 1, 54)), ("q2", (15, 17), 1, (512, 1, 54)),
         ("brick", (4, 4, 4), 1, (256, 1, 81)), ("brick", (10, 11, 12), 1, (512, 1, 81)),
         ("book", (30, 6), 1, (1024, 1, 0)), ("book", (30, 12), 1, (1024, 1, 0))]
+# the mesher's numberings: every layout with one or several workgroups, up to the largest sizes
+MESHED = [("quad", (20, 21, 1), 0, (1024, 1, 9)), ("quad", (44, 43, 1), 0, (1024, 2, 9)),
+          ("quad", (47, 46, 1), 0, (1024, 1, 9)), ("quad", (120, 121, 1), 0, (1024, 2, 9)),
+          ("quad", (800, 801, 1), 0, (512, 6, 9)), ("quad", (900, 901, 1), 0, (512, 8, 9)),
+          ("quad", (22, 20, 2), 0, (1024, 1, 18)), ("quad", (60, 61, 2), 0, (1024, 1, 18)),
+          ("quad", (362, 362, 2), 0, (512, 3, 18)), ("quad", (450, 449, 2), 0, (512, 4, 18)),
+          ("q2", (10, 11), 0, (256, 1, 54)), ("q2", (30, 31), 0, (512, 1, 54)),
+          ("brick", (8, 9, 7), 0, (256, 1, 81)), ("brick", (15, 14, 16), 0, (512, 1, 81)),
+          ("book", (30, 20), 0, (1024, 1, 0)), ("q2", (130, 131), 0, (1024, 1, 0)), ("q2", (185, 186), 0, (1024, 2, 0)),
+          ("quad", (520, 521, 2), 0, (1024, 4, 0))]
 
 
-@pytest.mark.parametrize("kind,size,shuffle,shape", WIDE)
+@pytest.mark.parametrize("kind,size,shuffle,shape", WIDE + MESHED)
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
 def test_resident_pcg_by_layout(torch_gpu, kind, size, shuffle, shape, precision):
     torch = torch_gpu
