@@ -82,7 +82,7 @@ int64_t Plan::device_bytes() const {
               element_matrices64.bytes() + element_matrices32.bytes();
   for (auto& s : sets)
     b += s.conn.bytes() + s.conn_orig.bytes() + s.inc_ptr.bytes() + s.inc.bytes() + s.touched.bytes() + s.rn_ptr.bytes() +
-         s.rn.bytes() + s.code.bytes();
+         s.rn.bytes() + s.code.bytes() + s.code32.bytes();
   for (auto& c : captured) b += c.vectors.bytes();
   return b;
 }
@@ -131,9 +131,38 @@ static void build_incidence(const Plan& P, ElemSet& s) {
   for (int64_t k = 0; k < m; ++k) s.inc_h[at[s.conn_host[k]]++] = (int32_t)k;
 }
 
+// ElemSet::code: the first position of a node's columns in BITS bits, its free DOFs above.
+template <int BITS, class C>
+static void build_codes(const Plan& P, const ElemSet& s, std::vector<C>& code, const std::vector<int64_t>& adj_ptr,
+                        const std::vector<int32_t>& adj) {
+  const int d = P.d, npe = s.npe;
+  code.assign((size_t)s.n_elems * npe * npe, 0);
+  std::vector<C> place;
+  for (int64_t n = 0; n < P.n_nodes; ++n) {
+    if (s.inc_ptr_h[n + 1] == s.inc_ptr_h[n]) continue;
+    const int32_t *b = adj.data() + adj_ptr[n], *e = adj.data() + adj_ptr[n + 1];
+    place.clear();
+    uint32_t at = 0;
+    for (const int32_t* p = b; p != e; ++p) {
+      uint32_t free = 0, count = 0;
+      for (int k = 0; k < d; ++k)
+        if (!P.dmask_host[(int64_t)*p * d + k]) {
+          free |= 1u << k;
+          ++count;
+        }
+      place.push_back((C)((count ? at : 0) | free << BITS));
+      at += count;
+    }
+    for (int32_t k = s.inc_ptr_h[n]; k < s.inc_ptr_h[n + 1]; ++k) {
+      const int64_t* c = &s.conn_host[(int64_t)(s.inc_h[k] / npe) * npe];
+      for (int a = 0; a < npe; ++a) code[(size_t)k * npe + a] = place[std::lower_bound(b, e, (int32_t)c[a]) - b];
+    }
+  }
+}
+
 // The lists of a set's row-owner tangent (ElemSet::rn, code).  adj: sorted neighbours of a node.
 static void build_rows(const Plan& P, ElemSet& s, const std::vector<int64_t>& adj_ptr, const std::vector<int32_t>& adj) {
-  const int d = P.d, npe = s.npe;
+  const int d = P.d;
   s.rn_ptr_h.assign(1, 0);
   s.rn_h.clear();
   s.rn_max = 0;
@@ -149,30 +178,12 @@ static void build_rows(const Plan& P, ElemSet& s, const std::vector<int64_t>& ad
     s.rn_ptr_h.push_back((int32_t)(s.rn_h.size() / 3));
     s.rn_max = std::max(s.rn_max, s.rn_ptr_h[c + 1] - s.rn_ptr_h[c]);
   }
-  s.code_h.assign((size_t)s.n_elems * npe * npe, 0);
-  std::vector<uint16_t> place;
-  for (int64_t n = 0; n < P.n_nodes; ++n) {
-    if (s.inc_ptr_h[n + 1] == s.inc_ptr_h[n]) continue;
-    const int32_t *b = adj.data() + adj_ptr[n], *e = adj.data() + adj_ptr[n + 1];
-    place.clear();
-    int at = 0;
-    for (const int32_t* p = b; p != e; ++p) {
-      int free = 0, count = 0;
-      for (int k = 0; k < d; ++k)
-        if (!P.dmask_host[(int64_t)*p * d + k]) {
-          free |= 1 << k;
-          ++count;
-        }
-      APX_REQUIRE(at < 0x2000, APX_ERR_UNSUPPORTED, "a row of the reduced matrix has more than 8191 entries");
-      place.push_back((uint16_t)((count ? at : 0) | free << 13));
-      at += count;
-    }
-    for (int32_t k = s.inc_ptr_h[n]; k < s.inc_ptr_h[n + 1]; ++k) {
-      const int64_t* c = &s.conn_host[(int64_t)(s.inc_h[k] / npe) * npe];
-      for (int a = 0; a < npe; ++a)
-        s.code_h[(size_t)k * npe + a] = place[std::lower_bound(b, e, (int32_t)c[a]) - b];
-    }
-  }
+  s.code_h.clear();
+  s.code32_h.clear();
+  if (P.max_row <= 1 << 13)
+    build_codes<13>(P, s, s.code_h, adj_ptr, adj);
+  else
+    build_codes<29>(P, s, s.code32_h, adj_ptr, adj);
 }
 
 // Build the host-side reduced pattern, colours and row-owner lists (no device calls).
@@ -381,13 +392,17 @@ static void upload_rows(Plan& P, ElemSet& S) {
   if (!S.rn_ptr_h.empty()) {
     S.rn_ptr.upload(S.rn_ptr_h.data(), S.rn_ptr_h.size());
     S.rn.upload(S.rn_h.data(), S.rn_h.size());
-    S.code.upload(S.code_h.data(), S.code_h.size());
+    if (S.code32_h.empty())
+      S.code.upload(S.code_h.data(), S.code_h.size());
+    else
+      S.code32.upload(S.code32_h.data(), S.code32_h.size());
   }
   std::vector<int32_t>().swap(S.inc_ptr_h);
   std::vector<int32_t>().swap(S.inc_h);
   std::vector<int32_t>().swap(S.rn_ptr_h);
   std::vector<int32_t>().swap(S.rn_h);
   std::vector<uint16_t>().swap(S.code_h);
+  std::vector<uint32_t>().swap(S.code32_h);
 }
 
 void plan_finalize(Plan& P) {

@@ -34,12 +34,15 @@ struct ElemSet {
   bool touched_all = false;        // every node, in order: no list
   // Their tangent: per 64-row chunk of the reduced matrix the nodes of the set with rows in it (as
   // begin and end in inc and first DOF), and per pair of inc and node of its element where that
-  // node's columns lie in the row: first position | free DOFs << 13.
+  // node's columns lie in the row: first position | free DOFs << 13 (code32, << 29, where a row of the
+  // plan has more entries than 13 bits count).
   DevBuf<int32_t> rn_ptr, rn;
   int rn_max = 0;                  // most such nodes in a chunk
   DevBuf<uint16_t> code;
+  DevBuf<uint32_t> code32;
   std::vector<int32_t> inc_ptr_h, inc_h, rn_ptr_h, rn_h;  // until uploaded
   std::vector<uint16_t> code_h;
+  std::vector<uint32_t> code32_h;
   std::vector<int64_t> colour_offsets;  // n_colours + 1
   // Structured Q1 grid (the connectivity of mesher.structured_mesh): element
   // e = i * gny + j has nodes b, b + 1, b + gny + 2, b + gny + 1 with

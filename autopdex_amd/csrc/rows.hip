@@ -27,6 +27,7 @@
 // Both are bitwise reproducible.  Replaces jacfwd(jacrev) and the scatter of
 // user_potential_assemble_tangent / _residual (autopdex/assembler.py:1064-1149).
 #include <algorithm>
+#include <type_traits>
 
 #include "assembly.hpp"
 #include "elements.hpp"
@@ -353,7 +354,7 @@ struct RowArgs {
   const int32_t* rn_ptr;          // the chunk's row nodes
   const int32_t* rn;              // per row node: its pairs' range in inc, its first DOF
   const int32_t* inc;             // (element * NPE + local index), in element order
-  const uint16_t* code;           // per such pair and element node: where its columns lie in the row
+  const void* code;               // per such pair and element node: where its columns lie in the row
   const int32_t *full2red, *indptr, *sell_ptr;
   int n_free, stride;             // stride: words per row of the LDS rows
   int window;                     // columns formed at a time
@@ -367,10 +368,10 @@ struct RowArgs {
 // Rows of one chunk.  Lane (row node, b) adds the blocks K_ab of that node's elements one after the
 // other: within a step no two lanes of a wavefront touch the same entry, and a row belongs to one
 // wavefront, so LDS needs no ordering beyond the wavefront's own.  T: type of the element matrices and
-// of the sums, TO: of the stored values.
-template <int NPE, int D, class T, class TO, bool CSR>
+// of the sums, TO: of the stored values, C: of the codes (32 bits where a row has over 8,192 entries).
+template <int NPE, int D, class T, class TO, bool CSR, class C>
 __global__ __launch_bounds__(256) void k_gather_rows(RowArgs A) {
-  constexpr int NPW = 64 / NPE, KB = D * D, BATCH = 4;
+  constexpr int NPW = 64 / NPE, KB = D * D, BATCH = 4, BITS = sizeof(C) == 2 ? 13 : 29;
   extern __shared__ __align__(16) double lds[];
   T* rows = (T*)lds;
   __shared__ int ptr[65];
@@ -415,13 +416,13 @@ __global__ __launch_bounds__(256) void k_gather_rows(RowArgs A) {
       }
       for (int p = p0; __any(p < p1); p += BATCH) {
         T k[BATCH][KB];
-        int code[BATCH];
+        std::conditional_t<sizeof(C) == 2, int, uint32_t> code[BATCH];
         bool own[BATCH];
 #pragma unroll
         for (int j = 0; j < BATCH; ++j) {
           const bool in = p + j < p1;
           const int pp = in ? p + j : p0;
-          code[j] = in ? A.code[(int64_t)pp * NPE + b] : 0;
+          code[j] = in ? ((const C*)A.code)[(int64_t)pp * NPE + b] : 0;
           const int32_t ea = A.inc[pp], e = ea / NPE;
           int plane;
           own[j] = stored_block<NPE>(ea % NPE, b, plane);
@@ -435,13 +436,13 @@ __global__ __launch_bounds__(256) void k_gather_rows(RowArgs A) {
           // has no place in the rows goes to a spare word
           int word[KB];
           T old[KB];
-          const int at0 = (code[j] & 0x1fff) - win;
+          const int at0 = (int)(code[j] & ((1u << BITS) - 1)) - win;
 #pragma unroll
           for (int i = 0; i < D; ++i) {
             int at = at0;
 #pragma unroll
             for (int kk = 0; kk < D; ++kk) {
-              const bool free = code[j] >> (13 + kk) & 1;
+              const bool free = code[j] >> (BITS + kk) & 1;
               word[i * D + kk] = free && r[i] >= 0 && at >= 0 && at < A.window ? r[i] * A.stride + at : 64 * A.stride;
               old[i * D + kk] = rows[word[i * D + kk]];
               at += free ? 1 : 0;
@@ -797,7 +798,7 @@ void run_rows(Plan& P, ElemSet& S, const double* u, void* vals, bool accumulate,
   A.rn_ptr = S.rn_ptr.p;
   A.rn = S.rn.p;
   A.inc = S.inc.p;
-  A.code = S.code.p;
+  A.code = S.code32.p ? (const void*)S.code32.p : S.code.p;
   A.full2red = P.full2red.p;
   A.indptr = P.indptr.p;
   A.sell_ptr = P.sell_ptr.p;
@@ -811,7 +812,8 @@ void run_rows(Plan& P, ElemSet& S, const double* u, void* vals, bool accumulate,
   A.vals = vals;
   const int waves = std::max(1, std::min(4, (S.rn_max + NPW - 1) / NPW));
   const size_t bytes = ((size_t)64 * A.stride + 1) * sizeof(T);
-  const auto kernel = k_gather_rows<M::NPE, M::D, T, TO, CSR>;
+  const auto kernel =
+      S.code32.p ? k_gather_rows<M::NPE, M::D, T, TO, CSR, uint32_t> : k_gather_rows<M::NPE, M::D, T, TO, CSR, uint16_t>;
   if (bytes > 48 * 1024)
     APX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
   hipLaunchKernelGGL(kernel, dim3((unsigned)round_xcd(P.n_chunks)), dim3(waves * 64), (uint32_t)bytes, st, A);
