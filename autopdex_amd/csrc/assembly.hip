@@ -181,12 +181,11 @@ static void dispatch(Plan& P, ElemSet& S, const double* u, double* r, void* vals
   }
 }
 
-// Algorithmic (compulsory) bytes of one assembly: what the kernels that run
-// must move at least once -- coordinates and DOFs read, outputs written; the
-// colour path also reads the connectivity (and, for the tangent, the slot
-// map is not counted: it is an implementation choice), the owner-tile path
-// derives the connectivity from the grid and reads the precomputed source
-// part instead.
+// Algorithmic (compulsory) bytes of one assembly: inputs read once, outputs written once, in the type
+// that is stored.  Coordinates and DOFs, the values or the residual; the row owners also read the
+// connectivity, the owner tiles derive it from the grid and read the precomputed source part instead.
+// What the row owners keep in between is not counted: their element matrices (64^3 Hex8 FP64: 755 MB
+// written and read back, beside 528 MB of values) and vectors, and the lists of who owns what.
 int64_t residual_bytes(const Plan& P) {
   int64_t b = P.n_nodes * P.dim * 8 + P.n_dofs * 8 * 2;
   for (auto& s : P.sets) {

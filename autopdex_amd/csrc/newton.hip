@@ -97,9 +97,7 @@ struct NewtonCtx {
     else if (fp32_arith)
       timing_collect(P, "tangent_f32", ev_tan, tangent_bytes(P, APX_FP32), ev_tan.size());
     else
-      timing_collect(P, "tangent_f64_to_f32", ev_tan,
-                     tangent_by_tiles(P) ? tangent_bytes(P, APX_FP32) : tangent_bytes(P, APX_FP64) + P.sell_total * 12,
-                     ev_tan.size());
+      timing_collect(P, "tangent_f64_to_f32", ev_tan, tangent_bytes(P, APX_FP32), ev_tan.size());
   }
 };
 
