@@ -749,7 +749,10 @@ int line_blocks(const Plan& P) {
 // pays (FP64, us an iteration: 557,973 rows in lines of 31, SELL kernel 35.1; 575,972 in lines of 32
 // 34.8, of 64 31.5; 571,377 in lines of 127 29.6).  Lines of over two million rows would need more
 // workgroups than a row of partial sums holds.  Systems that apx_pcg_noalloc takes keep the SELL kernel,
-// whose sums it shares bit by bit (and where the launches' latency, not the bytes, sets the pace).
+// whose sums it shares bit by bit, and where the launches' latency, not the bytes, sets the pace.
+// Flexible CG has no allocation-free twin, but its break-even lies there too (a Newton solve with the
+// network, FP64, by lines against SELL: 65^2 nodes 8.47 and 8.24 ms, 129^2 14.23 and 14.08, 257^2 25.7 and
+// 25.1, 385^2 33.8 and 33.3, 513^2 46.5 and 46.3).
 static bool lines_pay(const Plan& P, size_t value_bytes) {
   return P.line >= 32 && line_blocks(P) <= kMaxBlocks && !noalloc_accepts(P, value_bytes);
 }

@@ -366,7 +366,7 @@ def probe_train(args):
 
 
 def probe_cube(args):
-    """The 64^3 Hex8 Neo-Hooke configuration's kernels (colour-pass assembly, 3-DOF SpMV), for
+    """The 64^3 Hex8 Neo-Hooke configuration's kernels (row-owner assembly, 3-DOF SpMV), for
     kernel-trace and counter runs: one Newton iteration of 20 Jacobi-PCG iterations from u = 0
     with the first load step's Dirichlet values (imposed by apx_newton before its first
     residual), FP64, then the mixed method (FP32 element arithmetic, FP64 Krylov vectors).

@@ -83,9 +83,9 @@ int apx_plan_set_params(apx_plan* plan, int set, const double* params, int n_par
 int apx_plan_bind_nodal_field(apx_plan* plan, int set, int which, const double* field_dev);
 
 /* Build the reduced CSR pattern (bit-identical to scipy's canonical CSR of the
- * reduced system, P4), element colours and slot maps; upload to the device. */
+ * reduced system, P4), element colours and row lists; upload to the device.  */
 int apx_plan_finalize(apx_plan* plan);
-/* Host-only part of apx_plan_finalize (pattern, colours, slot maps; no device
+/* Host-only part of apx_plan_finalize (pattern, colours, row lists; no device
  * calls), so the pattern can be built and inspected without a GPU.         */
 int apx_plan_build_pattern(apx_plan* plan);
 int apx_plan_destroy(apx_plan* plan);
