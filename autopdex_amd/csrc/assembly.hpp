@@ -68,11 +68,12 @@ void jacobi_inverse_f32_to_f64(Plan& P, const float* vals, double* inv_diag, hip
 // The iterations of a PCG run from x = 0, r, z = D^-1 r, p_old and the scalars S to a stop flag in one
 // launch, waited for (resident.hip).  x and p_new receive the solution and the last direction,
 // host_state (pinned, sizeof(ResidentOut)) and the ResidentOut in part the scalars; S stays as it was (a
-// re-anchored run goes on from the latter).  zt: 2 n_free words of scratch of the vectors' type.  false:
-// the system does not fit, or the run was given up; x is 0, r, z and p_old are as they were.
+// re-anchored run goes on from the latter).  zt: 2 n_free words of scratch of the vectors' type.  idle:
+// the stream has nothing to do but the run's start.  false: the system does not fit, or the run was given
+// up; x is 0, r, z and p_old are as they were.
 template <class M, class V>
 bool pcg_resident(Plan& P, const M* vals, const V* inv, V* x, const V* r, const V* z, const V* p_old, V* p_new,
-                  unsigned long long* zt, KState* S, double* part, KState* host_state, hipStream_t st);
+                  unsigned long long* zt, KState* S, double* part, KState* host_state, bool idle, hipStream_t st);
 
 // How a resident run deals out a system of n rows of at most `row` entries, bandwidth bw: T threads a
 // workgroup, K rows a thread, rows of up to RW entries in registers (0: read in every iteration), xl:
@@ -124,6 +125,7 @@ struct PcgRun {
   bool upper_known = false;
   int k0 = 0;  // iterations before the present streaming run
   int start_k = 0;         // iterations before the present resident run
+  bool idle = false;       // the stream had nothing to do before the run's start
   bool resident_last = false;  // the last run was resident: S still holds the scalars from before it
   int maxiter = 0, iterations = 0;
   int64_t launched = 0;

@@ -669,6 +669,12 @@ __global__ __launch_bounds__(kFinBS) void k_pcg_reanchor_fin(KState* S, double* 
 }
 
 // ---- PCG driver ----------------------------------------------------------------------
+static bool is_idle(hipStream_t st) {
+  if (hipStreamQuery(st) == hipSuccess) return true;
+  (void)hipGetLastError();  // not ready
+  return false;
+}
+
 template <class M, class T>
 PcgRun<M, T>::PcgRun(Plan& P_, const M* vals_, const T* inv_, hipStream_t st_)
     : P(P_), vals(vals_), inv(inv_), st(st_) {
@@ -713,6 +719,7 @@ void PcgRun<M, T>::init(const T* b, const double* r_full, T* x_, double tol, dou
   upper = nullptr;  // the matrix may be another one
   upper_known = false;
   maxiter = maxiter_ <= 0 ? (int)std::min<int64_t>(10 * n, INT32_MAX / 2) : maxiter_;
+  idle = is_idle(st);
   const PcgStart A{tol, atol, delta, maxiter};
   const int g = grid_for(n);
   auto start = [&](auto full, auto one) {
@@ -859,7 +866,7 @@ KState PcgRun<M, T>::run() {
     const EventPair e = timed ? timing_pair(P) : EventPair{};
     t_launch_events = timed ? &e : nullptr;
     const bool ran = !streaming && pcg_resident<M, T>(P, vals, inv, x, r, z, odd ? pb : pa, odd ? pa : pb,
-                                                      (unsigned long long*)q, S, part, pinned_state, st);
+                                                      (unsigned long long*)q, S, part, pinned_state, idle, st);
     if (timed && !t_launch_events)
       (ran ? ev_res : ev_given_up).push_back(e);
     else if (timed)
@@ -943,6 +950,7 @@ KState PcgRun<M, T>::run() {
 
 template <class M, class T>
 void PcgRun<M, T>::reanchor(const double* r_full) {
+  idle = is_idle(st);
   const int g = grid_for(n);
   hipLaunchKernelGGL(k_pcg_reanchor<T>, dim3(g), dim3(kBS), 0, st, n, P.red2full.p, r_full, inv, x, r, z, S, part);
   if (resident_last)

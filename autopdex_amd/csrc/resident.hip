@@ -589,7 +589,7 @@ bool launch_if(const ResidentShape& s, const ResidentArgs& A, const M* vals, con
 
 template <class M, class V>
 bool pcg_resident(Plan& P, const M* vals, const V* inv, V* x, const V* r, const V* z, const V* p_old, V* p_new, u64* zt,
-                  KState* S, double* part, KState* host_state, hipStream_t st) {
+                  KState* S, double* part, KState* host_state, bool idle, hipStream_t st) {
   int dev = 0;
   APX_HIP(hipGetDevice(&dev));
   if (dev < 0 || dev >= kMaxDevices || P.resident_wait < 0.0) return false;
@@ -629,12 +629,13 @@ bool pcg_resident(Plan& P, const M* vals, const V* inv, V* x, const V* r, const 
   A.host = host;
   std::memset(host, 0, sizeof(ResidentOut));
   {
-    // The compute units are held only while the run is on the device: what the stream has to do before it is
-    // waited for first, or a solve on another thread would wait for all of that (10 us a solve).  A
-    // single workgroup meets nobody and holds none; others at most wait for it to end.
+    // The compute units are held only while the run is on the device: what else the stream has to do before
+    // it is waited for first, or a solve on another thread would wait for all of that (10 us a solve, none
+    // where only the run's own start is queued, as in Newton).  A single workgroup meets nobody and holds none;
+    // others at most wait for it to end.
     std::optional<ResidentLease> lease;
     if (s.G > 1) {
-      APX_HIP(hipStreamSynchronize(st));
+      if (!idle) APX_HIP(hipStreamSynchronize(st));
       lease.emplace(dev, s.G, P.cus);
     }
     const bool launched = APX_SHAPE(1024, 1, 9, false) || APX_SHAPE(1024, 2, 9, false) || APX_SHAPE(512, 6, 9, true) || APX_SHAPE(512, 8, 9, true) ||
@@ -662,10 +663,10 @@ bool pcg_resident(Plan& P, const M* vals, const V* inv, V* x, const V* r, const 
 }
 
 template bool pcg_resident<double, double>(Plan&, const double*, const double*, double*, const double*, const double*,
-                                           const double*, double*, u64*, KState*, double*, KState*, hipStream_t);
+                                           const double*, double*, u64*, KState*, double*, KState*, bool, hipStream_t);
 template bool pcg_resident<float, float>(Plan&, const float*, const float*, float*, const float*, const float*,
-                                         const float*, float*, u64*, KState*, double*, KState*, hipStream_t);
+                                         const float*, float*, u64*, KState*, double*, KState*, bool, hipStream_t);
 template bool pcg_resident<float, double>(Plan&, const float*, const double*, double*, const double*, const double*,
-                                          const double*, double*, u64*, KState*, double*, KState*, hipStream_t);
+                                          const double*, double*, u64*, KState*, double*, KState*, bool, hipStream_t);
 
 }  // namespace apx
