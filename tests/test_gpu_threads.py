@@ -99,18 +99,16 @@ def test_a_solve_does_not_wait_for_another_threads_stream(torch_gpu):
     first, second = System("quad", (885, 886, 1), 0), System("quad", (300, 301, 1), 0)
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     assert first.layout(0, cus).workgroups + second.layout(0, cus).workgroups > cus  # not both at once
-    vals, b = torch.from_numpy(second.A.data).cuda(), torch.from_numpy(second.b).cuda()
-    x = torch.empty_like(b)
+    data = [tuple(torch.from_numpy(v).cuda() for v in (s.A.data, s.b, np.zeros(s.n))) for s in (first, second)]
 
-    def solve_second():
+    def solve(i):  # no copies from or to the host, which would wait for the stream
+        s, entry = ((first, "apx_pcg"), (second, "apx_pcg_noalloc"))[i]
         ks = N.KrylovStats()
-        N.call("apx_pcg_noalloc", second.plan, C.c_void_p(vals.data_ptr()), C.c_void_p(b.data_ptr()),
-               C.c_void_p(x.data_ptr()), N.APX_FP64, N.APX_PRECOND_JACOBI, 1e-12, 0.0, 0, C.byref(ks),
-               C.c_void_p(torch.cuda.current_stream().cuda_stream))
+        N.call(entry, s.plan, *(C.c_void_p(t.data_ptr()) for t in data[i]), N.APX_FP64, N.APX_PRECOND_JACOBI, 1e-12,
+               0.0, 0, C.byref(ks), C.c_void_p(torch.cuda.current_stream().cuda_stream))
         return ks.converged
 
-    _solve(torch, first)
-    assert solve_second() == 1
+    assert solve(0) == 1 and solve(1) == 1
     start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
     start.record()
     torch.cuda._sleep(10_000_000)
@@ -118,6 +116,7 @@ def test_a_solve_does_not_wait_for_another_threads_stream(torch_gpu):
     end.synchronize()
     cycles = int(10_000_000 * 500 / start.elapsed_time(end))
     print(f"[case] two threads, one with a busy stream: {cycles} cycles", flush=True)
+    torch.cuda.synchronize()
     queued, busy, seen = threading.Event(), torch.cuda.Event(), []
 
     def work(i):
@@ -125,12 +124,13 @@ def test_a_solve_does_not_wait_for_another_threads_stream(torch_gpu):
             torch.cuda._sleep(cycles)
             busy.record()
             queued.set()
-            _solve(torch, first)
+            assert solve(0) == 1
         else:
             assert queued.wait(10)
             threading.Event().wait(0.1)  # the first solve has come to its run
-            seen.append((solve_second(), busy.query()))
+            seen.append((solve(1), busy.query()))
 
     _in_threads(torch, 2, work)
     assert seen == [(1, False)]
-    assert np.linalg.norm(second.A @ x.cpu().numpy() - second.b) <= 1.1e-12 * np.linalg.norm(second.b)
+    for s, (_, _, x) in zip((first, second), data):
+        assert np.linalg.norm(s.A @ x.cpu().numpy() - s.b) <= 1.1e-12 * np.linalg.norm(s.b)
